@@ -14,6 +14,7 @@
 #include <cstring>
 #include <new>
 
+#include "bc_ghosts.h"
 #include "fft_lds.h"
 #include "symtri_eigen.h"
 
@@ -984,11 +985,17 @@ int dfp_substep(dfp_plan* p, int stage, double* U, double* V, double* W, const d
     // scalars: the update :256-258 (:394-396, :526-531), apply_boundary_conditions
     // :297 (:428, :564), the projection :300 (:431, :567) and the boundary
     // conditions after it :304 (:435, :571), boundary_conditions.f90:186-260
-    HIPCHK(p, launch_rk_update(p, stage, U, V, W, Fo, R, coef, dt));
-    HIPCHK(p, launch_apply_bc(p, U, V, W, alpha_x, alpha_y, alpha_z));
+    // Where every ghost has an interior source (all but one cell between
+    // walls), the update writes all of its ghosts and the correction its x
+    // ghosts, the y and z ghost rows following in one launch.
+    const BcArgs bc = make_bc(p, alpha_x, alpha_y, alpha_z);
+    const bool fused = bc_fusable(p->geo);
+    HIPCHK(p, launch_rk_update(p, stage, U, V, W, Fo, R, coef, dt, fused ? &bc : nullptr));
+    if (!fused) HIPCHK(p, launch_apply_bc(p, U, V, W, alpha_x, alpha_y, alpha_z));
     if ((rc = spectral_solve(p, U, V, W, rhs_p, P, dt * c, save_p, 1))) return rc;
-    HIPCHK(p, launch_correct(p, U, V, W, rhs_p, nullptr));
-    HIPCHK(p, launch_apply_bc(p, U, V, W, alpha_x, alpha_y, alpha_z));
+    HIPCHK(p, launch_correct(p, U, V, W, rhs_p, nullptr, fused ? &bc : nullptr));
+    if (fused) HIPCHK(p, launch_ghost_yz(p, U, V, W, bc));
+    else HIPCHK(p, launch_apply_bc(p, U, V, W, alpha_x, alpha_y, alpha_z));
     return finish(p, flags);
 }
 

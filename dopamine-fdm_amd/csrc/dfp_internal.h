@@ -271,6 +271,8 @@ struct dfp_plan {
 
 namespace dfp {
 
+struct BcArgs;  // bc_ghosts.h
+
 // launchers (defined next to their kernels)
 // inflow/outflow x: DCT-IV kernels; phib (mode 0 only) adds the outlet backflow term
 hipError_t launch_div_rfft_x(dfp_plan* p, const double* U, const double* V, const double* W,
@@ -311,8 +313,9 @@ hipError_t launch_mode00(dfp_plan* p, hipStream_t s);  // rowpart -> pbar of the
 int correct_blocks_z(const Geo& g);
 hipError_t launch_divergence(dfp_plan* p, const double* U, const double* V, const double* W, double* rhs);
 // phib: outlet face values of the inflow/outflow x with the backflow term, or null
+// bc: also write the x ghosts apply_boundary_conditions leaves (bc_ghosts.h), or null
 hipError_t launch_correct(dfp_plan* p, double* U, double* V, double* W, const double* rhs,
-                          const double* phib = nullptr);
+                          const double* phib = nullptr, const BcArgs* bc = nullptr);
 // set_outflow_backflow_pressure (projection.f90:65-96): phib from u* at the
 // outlet and Pb, with dtc = dt*rk_coef(rk_step,rk_step); rhs, if given, takes
 // -2 phib/dx^2 in its last x cell (the fused x kernel applies it itself)
@@ -320,9 +323,12 @@ hipError_t launch_outflow_phib(dfp_plan* p, const double* U, const double* V, co
                                double* phib, double* rhs, double dtc);
 hipError_t launch_max_div(dfp_plan* p, const double* U, const double* V, const double* W, double* out_dev);
 // RK3 stage update of the interiors (Fo: Uo, Vo, Wo; R[field][s]: right-hand sides, s < stage;
-// c = rk_coef(stage, 1:stage)) and the channel's apply_boundary_conditions (k_step.hip)
+// c = rk_coef(stage, 1:stage)) and the channel's apply_boundary_conditions (k_step.hip); with bc the
+// update writes the ghosts apply_boundary_conditions leaves as well
 hipError_t launch_rk_update(dfp_plan* p, int stage, double* U, double* V, double* W, const double* const Fo[3],
-                            const double* const* R[3], const double* c, double dt);
+                            const double* const* R[3], const double* c, double dt, const BcArgs* bc = nullptr);
+// the y and z ghost rows alone, after launch_correct with bc
+hipError_t launch_ghost_yz(dfp_plan* p, double* U, double* V, double* W, const BcArgs& bc);
 hipError_t launch_apply_bc(dfp_plan* p, double* U, double* V, double* W, const double* ax, const double* ay,
                            const double* az);
 // out_dev = 1 if a velocity value in the monitor's ranges is NaN or above 1e8 in magnitude, else 0

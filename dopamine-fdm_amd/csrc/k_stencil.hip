@@ -14,7 +14,7 @@
 #include <mutex>
 #include <string>
 
-#include "dfp_internal.h"
+#include "bc_ghosts.h"
 
 namespace dfp {
 
@@ -62,7 +62,22 @@ hipError_t launch_divergence(dfp_plan* p, const double* U, const double* V, cons
 // phi(k) of the next: phi is read from memory once.
 constexpr int kCorrectK = 4;
 
-__device__ __forceinline__ void correct_body(const CPar& c, int bx, int bz) {
+// Stores a pair of corrected values of field fi at (i, j, k), (i+1, j, k).
+// BC: with their x images, the duplicate cells left to their sources (image:
+// the row is one).
+template <bool BC>
+__device__ __forceinline__ void correct_store(Glob<double>* F, long at, int n1, int fi, int i, double a, double b,
+                                              bool ok0, bool ok1, bool image) {
+    if constexpr (BC) {
+        ok0 = ok0 && !image && !bc_image_x(fi, i, n1);
+        ok1 = ok1 && !image && !bc_image_x(fi, i + 1, n1);
+    }
+    st2(F + at, a, b, ok0, ok1);
+    if constexpr (BC) bc_images_x(F + at - i, n1, fi, i, a, b, ok0, ok1);
+}
+
+template <bool BC>
+__device__ __forceinline__ void correct_body(const CPar& c, int bx, int bz, const BcArgs& bc) {
 #pragma clang fp contract(off)
     const Geo& g = c.g;
     // U, V, W and phi are distinct arrays: the loads of later planes may be
@@ -140,23 +155,28 @@ __device__ __forceinline__ void correct_body(const CPar& c, int bx, int bz) {
             ub = phib ? uo[q].y + 2.0 * (pc[q].y - phib[(j - 2) + (long)(k - 2) * g.nym]) * g.inv_dx
                       : uo[q].y + 2.0 * pc[q].y * g.inv_dx;
         }
-        st2(U + iu + q * pu_k, ua, ub, u0 || f0, u1 || f1);
+        correct_store<BC>(U, iu + q * pu_k, g.nx, 0, i, ua, ub, u0 || f0, u1 || f1,
+                          BC && bc_image_yz(bc, 0, j, k, g.nyg, g.nzg));
         if (do_v)
-            st2(V + iv + q * pv_k, vo[q].x - (py[q].x - pc[q].x) * idyg, vo[q].y - (py[q].y - pc[q].y) * idyg, true,
-                in1);
+            correct_store<BC>(V, iv + q * pv_k, g.nxg, 1, i, vo[q].x - (py[q].x - pc[q].x) * idyg,
+                              vo[q].y - (py[q].y - pc[q].y) * idyg, true, in1,
+                              BC && bc_image_yz(bc, 1, j, k, g.ny, g.nzg));
         // phi(k+1) is used for W only, for k <= nz-1
         if (k <= g.nz - 1) {
             const double dz = inv_dzg[k - 2];
-            st2(W + iw + q * pw_k, wo[q].x - (pc[q + 1].x - pc[q].x) * dz, wo[q].y - (pc[q + 1].y - pc[q].y) * dz,
-                true, in1);
+            correct_store<BC>(W, iw + q * pw_k, g.nxg, 2, i, wo[q].x - (pc[q + 1].x - pc[q].x) * dz,
+                              wo[q].y - (pc[q + 1].y - pc[q].y) * dz, true, in1,
+                              BC && bc_image_yz(bc, 2, j, k, g.nyg, g.nz));
         }
     }
 }
 
-__global__ void __launch_bounds__(256) k_correct(CPar c) {
+// BC: a substage's correction, which writes its x images (the y and z ghost rows follow, k_ghost_rows)
+template <bool BC>
+__global__ void __launch_bounds__(256) k_correct(CPar c, BcArgs bc) {
     const int L = xcd_remap(blockIdx.x + gridDim.x * blockIdx.y, gridDim.x * gridDim.y);
     const int bz = L / gridDim.x;
-    correct_body(c, L - bz * gridDim.x, bz);
+    correct_body<BC>(c, L - bz * gridDim.x, bz, bc);
 }
 
 __global__ void __launch_bounds__(256) kb_correct(const CPar* __restrict__ cs, const int* __restrict__ off,
@@ -176,7 +196,7 @@ __global__ void __launch_bounds__(256) kb_correct(const CPar* __restrict__ cs, c
         const CPar& c = cs[idx[lo]];
         const int li = w - off[lo];
         const int bz = li / c.nbx;
-        correct_body(c, li - bz * c.nbx, bz);
+        correct_body<false>(c, li - bz * c.nbx, bz, BcArgs{});
     }
 }
 
@@ -192,12 +212,14 @@ CPar make_cpar(const dfp_plan* p, double* U, double* V, double* W, const double*
 
 int correct_blocks_z(const Geo& g) { return ceil_div(g.nzg - 2, kCorrectK); }
 
-hipError_t launch_correct(dfp_plan* p, double* U, double* V, double* W, const double* rhs, const double* phib) {
+hipError_t launch_correct(dfp_plan* p, double* U, double* V, double* W, const double* rhs, const double* phib,
+                          const BcArgs* bc) {
     CPar c = make_cpar(p, U, V, W, rhs);
     c.phib = phib;
     dim3 grid(c.nbx, correct_blocks_z(p->geo));
     const int slot = prof_begin(p, "correct");
-    hipLaunchKernelGGL(k_correct, grid, dim3(256), 0, p->stream, c);
+    if (bc) hipLaunchKernelGGL(k_correct<true>, grid, dim3(256), 0, p->stream, c, *bc);
+    else hipLaunchKernelGGL(k_correct<false>, grid, dim3(256), 0, p->stream, c, BcArgs{});
     prof_end(p, slot);
     return hipGetLastError();
 }
