@@ -495,8 +495,9 @@ int dfp_plan_tuning(const dfp_plan* p, dfp_tuning* t) {
     if (!p || !t) return DFP_E_ARG;
     t->z_split = p->zr;
     t->x_columns = p->tk_x;
-    t->z_rows = p->g_zs;
-    t->z_fused = p->zfused ? 2 : 1;
+    // the register-plane kernel is what 0, 0 choose
+    t->z_rows = p->zp_nb ? 0 : p->g_zs;
+    t->z_fused = p->zp_nb ? 0 : (p->zfused ? 2 : 1);
     return DFP_OK;
 }
 
@@ -562,6 +563,11 @@ int dfp_plan_create_tuned(const dfp_grid* g, int precision, int device, const df
     p->fy = sh.fy;
     p->gy = sh.gy;
     if (!sh.fused) z_two_pass(sh.fz.n, p->zn1, p->zn2);
+    // whole sub-planes in registers where they fit, unless the streaming kernel was asked for
+    if (!sh.fused && g->z_bc_type == 0 && !(tune && (tune->z_rows || tune->z_fused)) &&
+        !zplane_shape(sh.fz.n, g->nym, precision == DFP_FP32_REFINE, p->lds_limit, p->zp_nb, p->zp_nch, p->zp_n1,
+                      p->zp_n2, p->zp_br))
+        p->zp_nb = 0;
     if (hipSetDevice(device) != hipSuccess) return bail(DFP_E_HIP);
     Geo& G = p->geo;
     const bool dct = g->x_bc_type == 1;

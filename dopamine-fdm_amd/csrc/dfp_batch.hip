@@ -354,7 +354,7 @@ int dfp_batch_project(dfp_batch* b, int n, dfp_plan* const* plans, double* const
         x64[a] = q;
         xpar_columns(q, p, 1);
         x64i[a] = q;
-        z64[a] = make_zpar<double2>(p, 0);
+        z64[a] = make_zpar<double2>(p, 0, 1);
         w64x[a] = (size_t)x64[a].nbx * p->geo.nym;
         w64xi[a] = (size_t)x64i[a].nbx * p->geo.nym;
         w64z[a] = z64[a].nblocks;
@@ -390,7 +390,7 @@ int dfp_batch_project(dfp_batch* b, int n, dfp_plan* const* plans, double* const
         x32s[a] = r;
         x32si[a] = r;
         xpar_columns(x32si[a], p, 1);
-        z32[a] = make_zpar<float2>(p, 1);
+        z32[a] = make_zpar<float2>(p, 1, 1);
         m32[a] = make_mpar(p);
         w32x[a] = (size_t)q.nbx * p->geo.nym;
         w32xi[a] = (size_t)x32i[a].nbx * p->geo.nym;
@@ -470,7 +470,7 @@ int dfp_batch_project(dfp_batch* b, int n, dfp_plan* const* plans, double* const
             while (k < sz.size() && sz[k].first != v) ++k;
             if (k == sz.size()) { sz.push_back({v, {}}); lsz.push_back(0); }
             sz[k].second.push_back(a);
-            lsz[k] = std::max(lsz[k], z_lds_bytes(p, f32));
+            lsz[k] = std::max(lsz[k], z_lds_bytes(p, f32, 1));
         }
         // one phase: the fused kernel and the split pairs (each workgroup
         // eliminates a sub-plane and substitutes back through it)

@@ -134,6 +134,7 @@ struct ZPar {
     int nplanes;         // (kx, u) sub-planes: nxh * R
     int n1, n2;          // two-pass factorization n = n1*n2 (0: staged transform)
     FastDiv div_n;
+    int nch, pp;         // register planes (k_zplane): chunks of rows per plane, planes per workgroup
 };
 
 // Per-case parameters of the periodic-y z/y kernel (k_zfused.hip): the fused
@@ -266,6 +267,9 @@ struct dfp_plan {
     int g_zs = 4;   // rows per group of the split z kernels, or rows per FFT call of the fused one
     int zfused = 0; // 1: one fused z kernel (whole sub-plane in LDS); 0: the split pair
     int zn1 = 0, zn2 = 0;  // two-pass z transforms of the split pair (0: staged transform)
+    // sub-planes in registers (k_zplane): passes per thread (0: the kernels above), chunks of rows, and the
+    // factors and rows per pass of the transform
+    int zp_nb = 0, zp_nch = 0, zp_n1 = 0, zp_n2 = 0, zp_br = 0;
     size_t lds_limit = 65536;  // LDS bytes per block on this device
 };
 
@@ -283,8 +287,32 @@ hipError_t launch_lu_table(dfp_plan* p);  // pins the (0,0) mode of the periodic
 hipError_t launch_zsolve(dfp_plan* p);
 int zsolve_rows_per_group(const FftDesc& fz, int nym, size_t lds_limit);
 bool z_two_pass(int n, int& n1, int& n2);
-// z kernel variant of a plan: -1 fused, else n1*32 + n2 of the split pair (0: staged transform)
+// z kernel variant of a plan: -1 fused, n1*32 + n2 of the split pair (0: staged transform), or
+// kZvPlane + passes * 1024 + n1*32 + n2 of the register-plane kernel
+constexpr int kZvPlane = 1 << 16;
 int z_variant(const dfp_plan* p);
+
+// (N1, N2, rows per pass): n = N1*N2 modes per row; the rows per pass are a
+// multiple of N2, so that a thread's items fill its registers
+#define DFP_ZP_SHORT(X) X(2, 4, 8) X(3, 4, 8) X(2, 8, 8) X(9, 2, 8) X(3, 8, 8) X(9, 3, 9) X(4, 8, 8)
+#define DFP_ZP_LONG(X)                                                                                    \
+    X(9, 4, 8) X(6, 8, 8) X(6, 9, 9) X(8, 8, 8) X(9, 8, 8) X(9, 9, 9) X(12, 8, 8) X(12, 9, 9) X(16, 8, 8)
+
+// Threads of the largest workgroup of the register-plane kernel with nb passes over rows of n modes.
+// Two passes hold 16 or 18 complex values and as many pivots per thread: 168 registers, which 768
+// threads (12 waves) have each, or more in the transforms of the longer first steps, held to 512
+// threads (256 registers) so that nothing spills.
+constexpr int zplane_threads(int n, int nb) {
+    if (nb == 1) return 384;
+    return n == 18 || n == 27 || n == 36 || n == 54 || n == 81 || n == 96 || n == 108 || n == 128 ? 512 : 768;
+}
+// passes, chunks and factors of the register-plane kernel for rows of n modes; false if a plane does not fit
+bool zplane_shape(int n, int nym, bool f32, size_t lds_limit, int& nb, int& nch, int& n1, int& n2, int& br);
+template <typename C>
+hipError_t launch_zplane(dfp_plan* p, const ZPar<C>& zp);
+template <typename C>
+hipError_t launch_zplane_batch(hipStream_t s, int variant, const ZPar<C>* cs, const int* off, const int* idx,
+                               const int* nc, int grid, size_t lds);
 hipError_t launch_irfft_x(dfp_plan* p, double* rhs, double* P, double dtc, int save_p);
 // fused z transform + y solve (whole sub-plane in LDS)
 template <typename C> hipError_t launch_zfused(dfp_plan* p, const ZPar<C>& zp);
@@ -341,12 +369,13 @@ hipError_t launch_synth(dfp_plan* p, double* U, double* V, double* W, uint64_t s
 template <typename C> XPar<C> make_xpar(const dfp_plan* p, int inv = 0);
 // set the column fields (T, nbx, strip, div_t) of q for the forward (inv = 0) or inverse x kernel
 template <typename C> void xpar_columns(XPar<C>& q, const dfp_plan* p, int inv);
-template <typename C> ZPar<C> make_zpar(const dfp_plan* p, int zero00);
+// batch: the record of a batched launch (planes per workgroup of the register-plane kernel)
+template <typename C> ZPar<C> make_zpar(const dfp_plan* p, int zero00, int batch = 0);
 CPar make_cpar(const dfp_plan* p, double* U, double* V, double* W, const double* rhs);
 MPar make_mpar(const dfp_plan* p);
 SPar make_spar(const dfp_plan* p, const double* rhs, double* P, double dtc);
 size_t x_lds_bytes(const dfp_plan* p, int inv, int f32);
-size_t z_lds_bytes(const dfp_plan* p, int f32);
+size_t z_lds_bytes(const dfp_plan* p, int f32, int batch = 0);
 template <typename C>
 hipError_t launch_xfwd_batch(hipStream_t s, int R, int mode, const XPar<C>* cs, const int* off, const int* idx,
                              const int* nc, int grid, size_t lds);

@@ -188,6 +188,19 @@ __device__ __forceinline__ void dft_rt(C (&a)[RMAX], int R) {
     }
 }
 
+// Two-step row transforms (n = N1*N2) of the z kernels: LDS position of element (i1, k2) of row r in the two-pass layouts (i1*N2 + k2
+// unswizzled): the N2 elements of each i1 are rotated by i1 and, for N2 = 8
+// and rows of a multiple of 16 points, odd rows swap 8-element halves, so the
+// 16 lanes of an LDS pass (FP64) hit distinct banks in both passes and the
+// sweep; the same map serves the Y and X layouts, so both passes stay in place
+template <int N1, int N2>
+__device__ __forceinline__ int zsw(int r, int i1, int k2) {
+    constexpr int N = N1 * N2;
+    int p = i1 * N2 + (k2 + i1) % N2;
+    if constexpr (N2 == 8 && N % 16 == 0) p ^= (r & 1) << 3;
+    return r * N + p;
+}
+
 // Sum over the block of one value per thread in a fixed order (butterflies
 // within each 64-lane wave, then the waves in order); every thread of the
 // block must call it and receives the total.  wsum holds NT/64 doubles.

@@ -1,0 +1,7 @@
+// k_zplane for the longer rows, FP64
+#include "k_zplane_impl.h"
+
+namespace dfp {
+#define DFP_ZP_ONE(a, b, r) DFP_ZP_INSTANTIATE(double2, a, b, r)
+DFP_ZP_LONG(DFP_ZP_ONE)
+}  // namespace dfp

@@ -1,0 +1,465 @@
+// z transforms and y solve of one (kx, u) sub-plane held in registers: the
+// rows are read once and written once (32 H bytes in FP64, 16 H in the FP32
+// form, and the pivots), where the streaming kernel (k_zsolve.hip) writes the
+// eliminated rows back and reads them again.
+//
+// A plane of nym rows of n = N1*N2 modes is cut into nch chunks of L = BR*NB
+// consecutive rows.  A workgroup has n*nch threads per plane (and PP planes,
+// where one plane would leave a wavefront empty); thread (chunk c, mode m)
+// owns rows cL .. cL+L-1 of mode m.
+//
+//   forward z transform, BR rows of every chunk at a time (NB passes): each
+//   thread loads BR/N2 items (row, i1) of N2 points straight from HBM,
+//   transforms them in registers, exchanges through LDS for the length-N1
+//   step (the two-step transform and LDS layout of k_zsolve.hip), and takes
+//   its BR rows of its mode back into registers: through LDS again, or, for
+//   16, 32 and 64 modes, across the lanes of its wave;
+//   y solve, with the plan's inverse pivots 1/D'(j) in registers: every chunk
+//   runs the elimination b'(j) = b(j) - DL(j-1)/D'(j-1) b'(j-1) from a zero
+//   carry for its last row and for the product of its multipliers, the chunks'
+//   ends are chained through LDS (each thread folds the ends before its own),
+//   and the elimination proper runs from the chained carry: the same
+//   recurrence as one long sweep, with only the carries associated
+//   differently.  The back substitution likewise from the top;
+//   inverse z transform: the same steps backwards, stored from registers.
+//
+// All of a plane's loads are in flight at once and no wave waits for another's
+// sweep: the serial part is 4 L + 2 nch steps instead of 2 nym.  The working
+// set (L complex values and L pivots per thread) is what limits it: planes
+// that need more threads than zplane_threads stay with the streaming kernel.
+#pragma once
+
+#include "fft_lds.h"
+
+namespace dfp {
+
+// Keeps the compiler from carrying the FP64 images of FP32 values from the
+// first sweep over them into the second (twice the registers of the values).
+template <int NB, int BR>
+__device__ __forceinline__ void keep(float2 (&x)[NB][BR]) {
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int q = 0; q < BR; ++q) asm volatile("" : "+v"(x[b][q].x), "+v"(x[b][q].y));
+}
+template <int NB, int BR>
+__device__ __forceinline__ void keep(double2 (&)[NB][BR]) {}
+
+// Exchanges the register index r = 0..7 of v with bits 3..5 of the lane:
+// v[r] of lane (h, k) becomes v[h] of lane (r, k), k = lane % 8.  One register
+// bit and one lane bit at a time: within 16 lanes by DPP (rotate by 8, half of
+// each row written), across them by the permlane swaps.
+__device__ __forceinline__ void swap_bit(uint32_t& a, uint32_t& b, int bit) {
+    if (bit == 0) {
+        const uint32_t na = (uint32_t)__builtin_amdgcn_update_dpp((int)a, (int)b, 0x128, 0xf, 0xc, false);
+        b = (uint32_t)__builtin_amdgcn_update_dpp((int)b, (int)a, 0x128, 0xf, 0x3, false);
+        a = na;
+    } else if (bit == 1) {
+        const auto s = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+        a = s[0];
+        b = s[1];
+    } else {
+        const auto s = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+        a = s[0];
+        b = s[1];
+    }
+}
+__device__ __forceinline__ void swap_bit(float& a, float& b, int bit) {
+    uint32_t x = __float_as_uint(a), y = __float_as_uint(b);
+    swap_bit(x, y, bit);
+    a = __uint_as_float(x);
+    b = __uint_as_float(y);
+}
+__device__ __forceinline__ void swap_bit(double& a, double& b, int bit) {
+    uint32_t xl = (uint32_t)__double2loint(a), yl = (uint32_t)__double2loint(b);
+    uint32_t xh = (uint32_t)__double2hiint(a), yh = (uint32_t)__double2hiint(b);
+    swap_bit(xl, yl, bit);
+    swap_bit(xh, yh, bit);
+    a = __hiloint2double((int)xh, (int)xl);
+    b = __hiloint2double((int)yh, (int)yl);
+}
+template <typename C>
+__device__ __forceinline__ void lane_transpose(C (&v)[8]) {
+#pragma unroll
+    for (int bit = 0; bit < 3; ++bit)
+#pragma unroll
+        for (int r = 0; r < 8; ++r) {
+            if (r >> bit & 1) continue;
+            swap_bit(v[r].x, v[r | 1 << bit].x, bit);
+            swap_bit(v[r].y, v[r | 1 << bit].y, bit);
+        }
+}
+
+// Runs the workgroup's items: rec(w, blk) gives the case record of item w and
+// its block there, same(w) whether the next item w has the record of the last
+// one.  An item's rows load into the registers that the item before frees,
+// behind that item's inverse transform and stores.
+template <typename C, int N1, int N2, int BR, int NB, typename Rec, typename Same>
+__device__ __forceinline__ void zplane_run(int w0, int total, Rec rec, Same same, unsigned char* smem_raw) {
+    using Rl = typename CplxT<C>::real;
+    constexpr int N = N1 * N2;
+    constexpr int L = BR * NB;
+    constexpr int SI = BR / N2;  // first-step items per thread and pass
+    static_assert(BR % N2 == 0, "items of a thread fill its rows");
+    // rows of 16, 32 or 64 modes, eight per second-step item: a wave holds the
+    // eight rows of NC whole chunks in both layouts (lane (row, k2), register
+    // (chunk, k1); lane (chunk, mode), register row), so the second exchange
+    // stays within the wave and out of LDS
+    constexpr bool kLane = BR == 8 && N2 == 8 && 64 % N == 0;
+    constexpr int NC = kLane ? 64 / N : 1;
+    C x[NB][BR];
+    bool loaded = false;
+    for (int w = w0; w < total; w += gridDim.x) {
+    int blk;
+    const ZPar<C>& zp = rec(w, blk);
+    const int nym = zp.nym, R = zp.R, nch = zp.nch;
+    const int nzs = zp.nzp / 2 + 1;
+    const int S1 = N * nch, S = S1 * zp.pp;  // threads per plane, per workgroup
+    // opaque, so that no address derived from it is held in a register over the loop
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    const bool act = tid < S;
+    const int t = min(tid, S - 1);
+    C* A = reinterpret_cast<C*>(smem_raw);  // S * BR values: BR rows of every chunk and plane
+    double* dls = reinterpret_cast<double*>(A + (size_t)S * BR);  // DL(j-1), nch*L
+    double* dus = dls + nch * L;                                  // DU(j), nch*L
+    C* twl = reinterpret_cast<C*>(dus + nch * L);                 // w_n^e, N
+    double2* ce = reinterpret_cast<double2*>(smem_raw);           // chunk ends (in A between the transforms)
+    double2* ge = ce + S;
+    double* cp = reinterpret_cast<double*>(ge + S);
+    double* gp = cp + S;  // 48 S bytes in all, within A's 64 S or more
+    // HBM accesses are a uniform base and a 32-bit byte offset per thread (one register per address): the
+    // workgroup's planes and pivot rows span well under 4 GiB
+    const int b0 = blk * zp.pp;
+    const long plane = (long)nym * N;
+
+    // this thread's rows of its mode
+    const int tp = t / S1;
+    const int tr = t - tp * S1;
+    const int c = tr / N, m = tr - c * N;
+    const int j0 = c * L;
+    const int vrow = (tp * nch + c) * BR;
+    // second-step items of the lane exchange: rows v0 + 8 cb, cb < NC
+    const int v0 = (tid >> 6) * (NC * 8) + ((tid >> 3) & 7), vend = S / N * BR;
+
+    // its transform items: item s covers local row v (plane p, row j of pass 0), elements i1 + N1 i2;
+    // formed anew at each use (opaque to the compiler) rather than held over the solve
+    struct Item {
+        int v, i1, p, j;
+    };
+    auto item = [&](int s) {
+        int tt = t;
+        asm volatile("" : "+v"(tt));
+        const int it = tt + s * S;
+        const int v = it / N1;
+        const int vc = v / BR, p = vc / nch;
+        return Item{v, it - v * N1, p, (vc - p * nch) * L + v - vc * BR};
+    };
+    // rows of pass b of block k (a partial last workgroup repeats its last plane, unstored)
+    auto load_rows = [&](int k, int b) {
+        const auto base = reinterpret_cast<const Glob<char>*>(gptr(zp.spec) + (long)k * zp.pp * plane);
+#pragma unroll
+        for (int s = 0; s < SI; ++s) {
+            const Item q = item(s);
+            const int pk = min(q.p, zp.nplanes - 1 - k * zp.pp);
+            const uint32_t o = (uint32_t)((pk * nym + min(q.j + b * BR, nym - 1)) * N + q.i1) * (uint32_t)sizeof(C);
+#pragma unroll
+            for (int i2 = 0; i2 < N2; ++i2)
+                x[b][s * N2 + i2] = gld<C>(reinterpret_cast<const Glob<C>*>(base + o) + N1 * i2);
+        }
+    };
+    double pl[L], plm;
+    auto load_pivots = [&](int k) {
+        const int kx0 = k * zp.pp / R;
+        const auto base = reinterpret_cast<const Glob<char>*>(gptr(zp.lu) + (long)kx0 * nym * nzs);
+        const int pk = min(k * zp.pp + tp, zp.nplanes - 1), kx = pk / R, u = pk - kx * R;
+        const uint32_t o = (uint32_t)((kx - kx0) * nym * nzs + lu_pos_mu(m, u, R, N));
+        auto at = [&](int j) {
+            return *reinterpret_cast<const Glob<double>*>(base + (o + (uint32_t)(j * nzs)) * (uint32_t)sizeof(double));
+        };
+        plm = at(max(j0 - 1, 0));
+#pragma unroll
+        for (int r = 0; r < L; ++r) pl[r] = at(min(j0 + r, nym - 1));
+    };
+    __syncthreads();  // the last item has read its tables and rows
+    if (!loaded) {
+#pragma unroll
+        for (int b = 0; b < NB; ++b) load_rows(blk, b);
+        for (int e = threadIdx.x; e < N; e += blockDim.x) twl[e] = gld<C>(gptr(zp.tw2) + e);
+        for (int e = threadIdx.x; e < nch * L; e += blockDim.x) {
+            dls[e] = e > 0 && e < nym ? gptr(zp.dl)[e - 1] : 0.0;
+            dus[e] = e < nym - 1 ? gptr(zp.du)[e] : 0.0;
+        }
+        __syncthreads();
+    }
+
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        if (act) {
+#pragma unroll
+            for (int s = 0; s < SI; ++s) {
+                const Item q = item(s);
+                const int v = q.v, i1 = q.i1;
+                C w[N2];
+#pragma unroll
+                for (int i2 = 0; i2 < N2; ++i2) w[i2] = x[b][s * N2 + i2];
+                if constexpr (N2 > 1) dft_reg<-1, N2>(w);
+                if (q.j + b * BR >= nym) {  // rows past the plane
+#pragma unroll
+                    for (int i2 = 0; i2 < N2; ++i2) w[i2] = CplxT<C>::make((Rl)0, (Rl)0);
+                }
+                A[zsw<N1, N2>(v, i1, 0)] = w[0];
+#pragma unroll
+                for (int k2 = 1; k2 < N2; ++k2) A[zsw<N1, N2>(v, i1, k2)] = twiddle<-1>(w[k2], twl[i1 * k2]);
+            }
+        }
+        if (b == NB - 1) load_pivots(blk);  // in flight over the last second step
+        __syncthreads();
+        if constexpr (kLane) {
+#pragma unroll
+            for (int cb = 0; cb < NC; ++cb) {
+                const int v = min(v0 + 8 * cb, vend - 1), k2 = tid & 7;
+                C w[N1];
+#pragma unroll
+                for (int i1 = 0; i1 < N1; ++i1) w[i1] = A[zsw<N1, N2>(v, i1, k2)];
+                dft_reg<-1, N1>(w);
+#pragma unroll
+                for (int k1 = 0; k1 < N1; ++k1) x[b][cb * N1 + k1] = w[k1];
+            }
+            lane_transpose(x[b]);
+        } else {
+            if (act) {
+                const int items = S * BR / N1;
+#pragma unroll 1
+                for (int it = t; it < items; it += S) {
+                    const int v = it / N2, k2 = it - v * N2;
+                    C w[N1];
+#pragma unroll
+                    for (int i1 = 0; i1 < N1; ++i1) w[i1] = A[zsw<N1, N2>(v, i1, k2)];
+                    dft_reg<-1, N1>(w);
+#pragma unroll
+                    for (int k1 = 0; k1 < N1; ++k1) A[zsw<N1, N2>(v, k1, k2)] = w[k1];
+                }
+            }
+            __syncthreads();
+#pragma unroll
+            for (int q = 0; q < BR; ++q) x[b][q] = A[zsw<N1, N2>(vrow + q, m / N2, m % N2)];
+        }
+        __syncthreads();
+    }
+
+    // elimination.  Rows past the plane hold zero, take no multiplier and a
+    // zero inverse pivot, so they carry nothing into the back substitution.
+    if (j0 == 0) plm = 0.0;
+    {
+        double ex = 0.0, ey = 0.0, pi = 1.0, ip = plm;
+#pragma unroll
+        for (int r = 0; r < L; ++r) {
+            if (j0 + r >= nym) pl[r] = 0.0;
+            const double mu = dls[j0 + r] * ip;
+            const C v = x[r / BR][r % BR];
+            ex = (double)v.x - mu * ex;
+            ey = (double)v.y - mu * ey;
+            pi *= -mu;
+            ip = pl[r];
+        }
+        if (act) {
+            ce[t] = make_double2(ex, ey);
+            cp[t] = pi;
+        }
+    }
+    __syncthreads();
+    {
+        double bx = 0.0, by = 0.0, ip = plm;
+        keep(x);
+#pragma unroll 2
+        for (int q = 0; q < c; ++q) {
+            const double2 e = ce[t - (c - q) * N];
+            const double f = cp[t - (c - q) * N];
+            bx = e.x + f * bx;
+            by = e.y + f * by;
+        }
+#pragma unroll
+        for (int r = 0; r < L; ++r) {
+            const double mu = dls[j0 + r] * ip;
+            C& v = x[r / BR][r % BR];
+            bx = (double)v.x - mu * bx;
+            by = (double)v.y - mu * by;
+            v = CplxT<C>::make((Rl)bx, (Rl)by);
+            ip = pl[r];
+        }
+    }
+    // back substitution, from the top
+    {
+        double gx = 0.0, gy = 0.0, pi = 1.0;
+#pragma unroll
+        for (int r = L - 1; r >= 0; --r) {
+            const double d = dus[j0 + r];
+            const C v = x[r / BR][r % BR];
+            gx = ((double)v.x - d * gx) * pl[r];
+            gy = ((double)v.y - d * gy) * pl[r];
+            pi *= -d * pl[r];
+        }
+        if (act) {
+            ge[t] = make_double2(gx, gy);
+            gp[t] = pi;
+        }
+    }
+    __syncthreads();
+    {
+        keep(x);
+        const bool is00 = zp.zero00 && b0 + tp == 0 && m == 0;  // the FP32 form solves the (0,0) mode on its own
+        double xx = 0.0, xy = 0.0;
+#pragma unroll 2
+        for (int q = nch - 1; q > c; --q) {
+            const double2 e = ge[t + (q - c) * N];
+            const double f = gp[t + (q - c) * N];
+            xx = e.x + f * xx;
+            xy = e.y + f * xy;
+        }
+#pragma unroll
+        for (int r = L - 1; r >= 0; --r) {
+            const double d = dus[j0 + r];
+            C& v = x[r / BR][r % BR];
+            xx = ((double)v.x - d * xx) * pl[r];
+            xy = ((double)v.y - d * xy) * pl[r];
+            v = is00 ? CplxT<C>::make((Rl)0, (Rl)0) : CplxT<C>::make((Rl)xx, (Rl)xy);
+        }
+    }
+    const int wn = w + gridDim.x;
+    loaded = wn < total && same(wn);
+    const int kn = blk + gridDim.x;  // an item of the same record
+    __syncthreads();
+
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        if constexpr (kLane) {
+            lane_transpose(x[b]);
+#pragma unroll
+            for (int cb = 0; cb < NC; ++cb) {
+                const int v = v0 + 8 * cb, k2 = tid & 7;
+                C w[N1];
+#pragma unroll
+                for (int k1 = 0; k1 < N1; ++k1) w[k1] = x[b][cb * N1 + k1];
+                dft_reg<1, N1>(w);
+                if (v < vend) {
+                    A[zsw<N1, N2>(v, 0, k2)] = w[0];
+#pragma unroll
+                    for (int i1 = 1; i1 < N1; ++i1) A[zsw<N1, N2>(v, i1, k2)] = twiddle<1>(w[i1], twl[i1 * k2]);
+                }
+            }
+            if (loaded) load_rows(kn, b);
+        } else {
+            if (act) {
+#pragma unroll
+                for (int q = 0; q < BR; ++q) A[zsw<N1, N2>(vrow + q, m / N2, m % N2)] = x[b][q];
+            }
+            if (loaded) load_rows(kn, b);
+            __syncthreads();
+            if (act) {
+                const int items = S * BR / N1;
+#pragma unroll 1
+                for (int it = t; it < items; it += S) {
+                    const int v = it / N2, k2 = it - v * N2;
+                    C w[N1];
+#pragma unroll
+                    for (int k1 = 0; k1 < N1; ++k1) w[k1] = A[zsw<N1, N2>(v, k1, k2)];
+                    dft_reg<1, N1>(w);
+                    A[zsw<N1, N2>(v, 0, k2)] = w[0];
+#pragma unroll
+                    for (int i1 = 1; i1 < N1; ++i1) A[zsw<N1, N2>(v, i1, k2)] = twiddle<1>(w[i1], twl[i1 * k2]);
+                }
+            }
+        }
+        __syncthreads();
+        if (act) {
+#pragma unroll
+            for (int s = 0; s < SI; ++s) {
+                const Item q = item(s);
+                const int v = q.v, i1 = q.i1;
+                C w[N2];
+#pragma unroll
+                for (int k2 = 0; k2 < N2; ++k2) w[k2] = A[zsw<N1, N2>(v, i1, k2)];
+                if constexpr (N2 > 1) dft_reg<1, N2>(w);
+                if (q.j + b * BR < nym && b0 + q.p < zp.nplanes) {
+                    const auto base = reinterpret_cast<Glob<char>*>(gptr(zp.spec) + b0 * plane);
+                    const uint32_t o = (uint32_t)((q.p * nym + q.j + b * BR) * N + i1) * (uint32_t)sizeof(C);
+                    const auto dst = reinterpret_cast<Glob<C>*>(base + o);
+#pragma unroll
+                    for (int i2 = 0; i2 < N2; ++i2) gst<C>(dst + N1 * i2, w[i2]);
+                }
+            }
+        }
+        if (b + 1 < NB) __syncthreads();
+    }
+    }
+}
+
+template <typename C, int N1, int N2, int BR, int NB>
+__global__ void __launch_bounds__(zplane_threads(N1 * N2, NB)) k_zplane(ZPar<C> zp) {
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    zplane_run<C, N1, N2, BR, NB>(
+        xcd_remap(blockIdx.x, gridDim.x), zp.nblocks,
+        [&](int w, int& blk) -> const ZPar<C>& {
+            blk = w;
+            return zp;
+        },
+        [](int) { return true; }, smem_raw);
+}
+
+template <typename C, int N1, int N2, int BR, int NB>
+__global__ void __launch_bounds__(zplane_threads(N1 * N2, NB))
+kb_zplane(const ZPar<C>* __restrict__ cs, const int* __restrict__ off, const int* __restrict__ idx,
+          const int* __restrict__ pnc) {
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    const int nc = *pnc;
+    int at = -1;  // case of the item in hand
+    zplane_run<C, N1, N2, BR, NB>(
+        xcd_remap(blockIdx.x, gridDim.x), off[nc],
+        [&](int w, int& blk) -> const ZPar<C>& {
+            int lo = 0, hi = nc;
+            while (hi - lo > 1) {
+                const int mid = (lo + hi) >> 1;
+                if (off[mid] <= w) lo = mid;
+                else hi = mid;
+            }
+            at = lo;
+            blk = w - off[lo];
+            return cs[idx[lo]];
+        },
+        [&](int w) { return w < off[at + 1]; }, smem_raw);
+}
+
+template <typename C, int N1, int N2, int BR>
+hipError_t launch_zplane_n(hipStream_t s, int nb, const ZPar<C>& zp, int threads, size_t lds) {
+    const dim3 blk(threads);
+    auto go = [&](auto k) {
+        hipLaunchKernelGGL(k, dim3(resident_grid(k, zp.nblocks, threads, lds)), blk, lds, s, zp);
+    };
+    if (nb == 1) go(k_zplane<C, N1, N2, BR, 1>);
+    else go(k_zplane<C, N1, N2, BR, 2>);
+    return hipGetLastError();
+}
+
+template <typename C, int N1, int N2, int BR>
+hipError_t launch_zplane_batch_n(hipStream_t s, int nb, const ZPar<C>* cs, const int* off, const int* idx,
+                                 const int* nc, int grid, int threads, size_t lds) {
+    auto go = [&](auto k) {
+        hipLaunchKernelGGL(k, dim3(resident_grid(k, grid, threads, lds)), dim3(threads), lds, s, cs, off, idx, nc);
+    };
+    if (nb == 1) go(kb_zplane<C, N1, N2, BR, 1>);
+    else go(kb_zplane<C, N1, N2, BR, 2>);
+    return hipGetLastError();
+}
+
+// one translation unit per half of the list and precision
+#define DFP_ZP_EXTERN(C, a, b, r)                                                                               \
+    extern template hipError_t launch_zplane_n<C, a, b, r>(hipStream_t, int, const ZPar<C>&, int, size_t);      \
+    extern template hipError_t launch_zplane_batch_n<C, a, b, r>(hipStream_t, int, const ZPar<C>*, const int*,  \
+                                                                 const int*, const int*, int, int, size_t);
+#define DFP_ZP_INSTANTIATE(C, a, b, r)                                                                          \
+    template hipError_t launch_zplane_n<C, a, b, r>(hipStream_t, int, const ZPar<C>&, int, size_t);             \
+    template hipError_t launch_zplane_batch_n<C, a, b, r>(hipStream_t, int, const ZPar<C>*, const int*,         \
+                                                          const int*, const int*, int, int, size_t);
+
+}  // namespace dfp

@@ -295,19 +295,6 @@ __device__ __forceinline__ void zbwd_body(const ZPar<C>& zp, int b, unsigned cha
 // same two steps in the other order, the second one storing x[i1 + N1*i2]
 // from registers to HBM.  Both replace the log(n) LDS passes of the staged
 // transform by one exchange through LDS.
-// LDS position of element (i1, k2) of row r in the two-pass layouts (i1*N2 + k2
-// unswizzled): the N2 elements of each i1 are rotated by i1 and, for N2 = 8
-// and rows of a multiple of 16 points, odd rows swap 8-element halves, so the
-// 16 lanes of an LDS pass (FP64) hit distinct banks in both passes and the
-// sweep; the same map serves the Y and X layouts, so both passes stay in place
-template <int N1, int N2>
-__device__ __forceinline__ int zsw(int r, int i1, int k2) {
-    constexpr int N = N1 * N2;
-    int p = i1 * N2 + (k2 + i1) % N2;
-    if constexpr (N2 == 8 && N % 16 == 0) p ^= (r & 1) << 3;
-    return r * N + p;
-}
-
 // Rows of 24 or 32 points: a block takes P = 2 consecutive sub-planes, so the
 // sweeping wave has a mode in (nearly) every lane and a launch needs half the
 // blocks.  Group row r of plane p is the virtual row v = r*P + p (n points,
@@ -613,8 +600,40 @@ __global__ void __launch_bounds__(kZsThreads) kb_zsolve(const ZPar<C>* __restric
     }
 }
 
+// planes per workgroup of the register-plane kernel: enough to fill a
+// wavefront, or a batched launch's fixed workgroup
+static int zplane_planes(const dfp_plan* p, int batch) {
+    return std::max(1, (batch ? zplane_threads(p->fz.n, p->zp_nb) : 64) / (p->fz.n * p->zp_nch));
+}
+
+static size_t zplane_lds(int threads, int n, int nch, int br, int nb, bool f32) {
+    const size_t cs = f32 ? sizeof(float2) : sizeof(double2);
+    return cs * ((size_t)threads * br + n) + 2 * sizeof(double) * (size_t)nch * br * nb;
+}
+
+// One pass where the plane fits its narrow workgroup (the most threads, the
+// shortest chains), else two.
+bool zplane_shape(int n, int nym, bool f32, size_t lds_limit, int& nb, int& nch, int& n1, int& n2, int& br) {
+    n1 = n2 = br = 0;
+#define DFP_ZP_TRY(a, c, r) \
+    if (a * c == n) { n1 = a; n2 = c; br = r; }
+    DFP_ZP_SHORT(DFP_ZP_TRY)
+    DFP_ZP_LONG(DFP_ZP_TRY)
+#undef DFP_ZP_TRY
+    if (!n1) return false;
+    for (int q : {1, 2}) {
+        const long threads = (long)n * ceil_div(nym, q * br);
+        if (threads > zplane_threads(n, q)) continue;
+        nb = q;
+        nch = (int)(threads / n);
+        // a batched workgroup holds up to zplane_threads threads of planes
+        return zplane_lds(zplane_threads(n, q), n, nch, br, nb, f32) <= lds_limit;
+    }
+    return false;
+}
+
 template <typename C>
-ZPar<C> make_zpar(const dfp_plan* p, int f32_zero00) {
+ZPar<C> make_zpar(const dfp_plan* p, int f32_zero00, int batch) {
     ZPar<C> z{};
     const Geo& g = p->geo;
     z.spec = reinterpret_cast<C*>(p->d_spec);
@@ -637,18 +656,28 @@ ZPar<C> make_zpar(const dfp_plan* p, int f32_zero00) {
     z.nplanes = g.nxh * p->zr;
     z.nblocks = ceil_div(z.nplanes, z.n1 ? zplanes(p->fz.n) : 1);
     z.div_n = FastDiv(p->fz.n);
+    if (p->zp_nb) {
+        z.nch = p->zp_nch;
+        z.pp = zplane_planes(p, batch);
+        z.nblocks = ceil_div(z.nplanes, z.pp);
+    }
     return z;
 }
-template ZPar<double2> make_zpar<double2>(const dfp_plan*, int);
-template ZPar<float2> make_zpar<float2>(const dfp_plan*, int);
+template ZPar<double2> make_zpar<double2>(const dfp_plan*, int, int);
+template ZPar<float2> make_zpar<float2>(const dfp_plan*, int, int);
 
-size_t z_lds_bytes(const dfp_plan* p, int f32) {
+size_t z_lds_bytes(const dfp_plan* p, int f32, int batch) {
+    if (p->zp_nb)
+        return zplane_lds(p->fz.n * p->zp_nch * zplane_planes(p, batch), p->fz.n, p->zp_nch, p->zp_br, p->zp_nb, f32);
     const int G = p->g_zs, n = p->fz.n, ntw = p->zn1 ? n : twiddle_count(p->fz);
     const size_t pts = (size_t)G * n * (p->zn1 ? zplanes(n) : 1);
     return (f32 ? sizeof(float2) : sizeof(double2)) * (pts + ntw) + sizeof(double) * (pts + G);
 }
 
-int z_variant(const dfp_plan* p) { return p->zfused ? -1 : p->zn1 * 32 + p->zn2; }
+int z_variant(const dfp_plan* p) {
+    if (p->zp_nb) return kZvPlane + p->zp_nb * 1024 + p->zp_n1 * 32 + p->zp_n2;
+    return p->zfused ? -1 : p->zn1 * 32 + p->zn2;
+}
 
 template <typename C>
 static hipError_t launch_zsolve_t(dfp_plan* p, const ZPar<C>& zp) {
@@ -670,14 +699,23 @@ static hipError_t launch_zsolve_t(dfp_plan* p, const ZPar<C>& zp) {
     return hipGetLastError();
 }
 
-hipError_t launch_zsolve(dfp_plan* p) { return launch_zsolve_t<double2>(p, make_zpar<double2>(p, 0)); }
+// The register-plane kernel where the plan's planes fit one (zplane_shape) and
+// no row grouping was asked for, else the streaming kernel.
+hipError_t launch_zsolve(dfp_plan* p) {
+    const ZPar<double2> zp = make_zpar<double2>(p, 0);
+    return p->zp_nb ? launch_zplane(p, zp) : launch_zsolve_t<double2>(p, zp);
+}
 
-hipError_t launch_zsolve32(dfp_plan* p) { return launch_zsolve_t<float2>(p, make_zpar<float2>(p, 1)); }
+hipError_t launch_zsolve32(dfp_plan* p) {
+    const ZPar<float2> zp = make_zpar<float2>(p, 1);
+    return p->zp_nb ? launch_zplane(p, zp) : launch_zsolve_t<float2>(p, zp);
+}
 
 // variant: z_variant of the cases of the list (all alike)
 template <typename C>
 hipError_t launch_zsolve_batch(hipStream_t s, int variant, const ZPar<C>* cs, const int* off, const int* idx,
                                const int* nc, int grid, size_t lds) {
+    if (variant >= kZvPlane) return launch_zplane_batch<C>(s, variant, cs, off, idx, nc, grid, lds);
     const dim3 blk(kZsThreads);
     auto go = [&](auto k) {
         hipLaunchKernelGGL(k, dim3(resident_grid(k, grid, kZsThreads, lds)), blk, lds, s, cs, off, idx, nc);

@@ -105,10 +105,13 @@ int dfp_plan_destroy(dfp_plan *plan);
  *   z_fused    1: split pair of z kernels (FFT + elimination, back
  *              substitution + inverse FFT, spectrum read and written twice);
  *              2: one fused kernel holding a whole (kx, z-split) sub-plane
- *              of nym x nzp/R modes in LDS (read and written once)
- * Results do not depend on x_columns or z_rows; z_split changes the FFT's
- * factorisation and z_fused = 2 the association of the y solve (chunked
- * across lanes), both at round-off level.  DFP_E_ARG for values out of
+ *              of nym x nzp/R modes in LDS (read and written once);
+ *              0 with z_rows = 0: a sub-plane held in registers where it
+ *              fits (read and written once; dfp_plan_tuning then reports
+ *              z_rows = z_fused = 0), else 1
+ * Results do not depend on x_columns or, at z_fused = 1, on z_rows; z_split
+ * changes the FFT's factorisation and z_fused the association of the y solve
+ * (chunked across lanes at 0 and 2), both at round-off level.  DFP_E_ARG for values out of
  * range, DFP_E_UNSUPPORTED for shapes that do not fit the device's LDS. */
 typedef struct dfp_tuning {
     int32_t z_split, x_columns, z_rows, z_fused;
