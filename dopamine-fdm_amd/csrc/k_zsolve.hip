@@ -738,7 +738,8 @@ template hipError_t launch_zsolve_batch<float2>(hipStream_t, int, const ZPar<flo
                                                 const int*, int, size_t);
 
 // rows per group: the group (its rows in each of the block's planes) fits
-// the prefetch registers (kZsPf points per thread), the in-place FFT capacity
+// the block's threads (one row coefficient each), the prefetch registers
+// (kZsPf points per thread), the in-place FFT capacity
 // (2 butterflies per thread; not a limit of the two-pass transforms) and,
 // with the twiddles and pivots, the device's LDS per block; 0 if one row does
 // not fit
@@ -750,7 +751,8 @@ int zsolve_rows_per_group(const FftDesc& fz, int nym, size_t lds_limit) {
     const size_t ntw = two ? (size_t)n : (size_t)twiddle_count(fz);
     const int pn = n * (two ? zplanes(n) : 1);  // points of one group row
     int G = (two ? kZsPf * kZsThreads : std::min(kZsPf * kZsThreads, inplace_capacity(fz, kZsThreads, 2))) / pn;
-    G = std::max(0, std::min(G, nym));
+    // one thread stages each row's coefficient
+    G = std::max(0, std::min({G, nym, kZsThreads}));
     auto bytes = [&](int g) {
         return sizeof(double2) * ((size_t)g * pn + ntw) + sizeof(double) * ((size_t)g * pn + g);
     };
