@@ -13,16 +13,53 @@
 
 namespace dfp {
 
+// y <- e + f y, the recurrence of a run of rows
+struct Affine {
+    double e, f;
+};
+
+// Runs y(t) = row(t, y(t-1)) over t = 0 .. len-1 (len <= kM00Chunk) in the
+// first wave: lane l takes the l-th run of rows, composes its rows' affine
+// maps (map(t): y(t) = e + f y(t-1)), the lanes' maps are scanned across the
+// wave, and each lane runs its rows from the carry that reaches it.  The
+// recurrence is a contraction or nearly so (the elimination's multipliers and
+// the substitution's ratios are below one in size up to rounding), and the
+// rows themselves are evaluated as the serial sweep would: only the carries
+// are associated differently.  carry: y(-1) in, y(len-1) out (all lanes).
+template <typename Map, typename Row>
+__device__ __forceinline__ void wave_recurrence(int len, double& carry, Map map, Row row) {
+    const int lane = threadIdx.x;  // 0..63
+    const int per = (len + 63) / 64, t0 = lane * per, t1 = min(t0 + per, len);
+    Affine a{0.0, 1.0};
+    for (int t = t0; t < t1; ++t) {
+        const Affine r = map(t);
+        a.e = r.e + r.f * a.e;
+        a.f = r.f * a.f;
+    }
+    for (int d = 1; d < 64; d *= 2) {
+        const double pe = __shfl_up(a.e, d, 64), pf = __shfl_up(a.f, d, 64);
+        if (lane >= d) {
+            a.e = a.e + a.f * pe;
+            a.f = a.f * pf;
+        }
+    }
+    const double le = __shfl_up(a.e, 1, 64), lf = __shfl_up(a.f, 1, 64);
+    double y = lane == 0 ? carry : le + lf * carry;
+    for (int t = t0; t < t1; ++t) y = row(t, y);
+    carry = __shfl(y, (len - 1) / per, 64);
+}
+
 // Row means of the field from the x kernel's per-block partial sums, then the
 // (0,0)-mode solve Dyy_pin x = mean with the inverse pivots the plan holds for
 // kx = kz = 0 (lu[j*nzs], pin of projection.f90:292 included) and the
-// elimination order of the spectral kernels.  Rows are staged through LDS in
-// chunks by the whole block; one thread runs each recurrence over a chunk
-// from LDS (distinct arrays, so its loads run ahead of its stores).
+// elimination order of the spectral kernels.  One workgroup, all of its
+// operands staged through LDS at once (in chunks beyond kM00Chunk rows): bound
+// by the latency of the loads and of the two scans, 21 -> 7 us at 192 rows and
+// 39 -> 8.5 us at 384 against one lane running the rows in turn.
 constexpr int kM00Chunk = 1024;
 
 __device__ __forceinline__ void mode00_body(const MPar& m) {
-    __shared__ double s_in[kM00Chunk], s_mul[kM00Chunk], s_cu[kM00Chunk], s_out[kM00Chunk];
+    __shared__ double s_in[kM00Chunk], s_mul[kM00Chunk], s_ip[kM00Chunk], s_cu[kM00Chunk], s_out[kM00Chunk];
     const auto rowpart = gptr(m.rowpart);
     const auto lu = gptr(m.lu);
     const auto dl = gptr(m.o.dl);
@@ -30,12 +67,18 @@ __device__ __forceinline__ void mode00_body(const MPar& m) {
     const auto x = gptr(m.x);
     const int nym = m.nym, nparts = m.nparts;
     const long nzs = m.nzs;
+    const bool once = nym <= kM00Chunk;  // one chunk: nothing passes through memory
     // forward: y(0) = mean(0); y(j) = mean(j) - DL(j-1)/D'(j-1) * y(j-1)
     double yp = 0.0;
     for (int c0 = 0; c0 < nym; c0 += kM00Chunk) {
         const int len = min(kM00Chunk, nym - c0);
         for (int t = threadIdx.x; t < len; t += blockDim.x) {
             const int j = c0 + t;
+            const double mul = j > 0 ? dl[j - 1] * lu[(j - 1) * nzs] : 0.0;
+            if (once) {
+                s_ip[t] = lu[j * nzs];
+                s_cu[t] = j < nym - 1 ? du[j] : 0.0;
+            }
             // the parts in order, eight loads in flight at a time
             const auto rp = rowpart + (long)j * nparts;
             double s = 0.0;
@@ -49,66 +92,45 @@ __device__ __forceinline__ void mode00_body(const MPar& m) {
             }
             for (; q < nparts; ++q) s += rp[q];
             s_in[t] = s / m.count;
-            s_mul[t] = j > 0 ? dl[j - 1] * lu[(j - 1) * nzs] : 0.0;
+            s_mul[t] = mul;
         }
         __syncthreads();
-        if (threadIdx.x == 0) {
-            // eight rows' operands are read together, so one LDS round trip
-            // serves eight steps of the recurrence
-            for (int t0 = 0; t0 < len; t0 += 8) {
-                double a[8], mu[8];
-#pragma unroll
-                for (int q = 0; q < 8; ++q) {
-                    const int t = min(t0 + q, len - 1);
-                    a[q] = s_in[t];
-                    mu[q] = s_mul[t];
-                }
-#pragma unroll
-                for (int q = 0; q < 8; ++q) {
-                    if (t0 + q < len) {
-                        yp = a[q] - mu[q] * yp;
-                        s_out[t0 + q] = yp;
-                    }
-                }
-            }
+        if (threadIdx.x < 64)
+            wave_recurrence(
+                len, yp, [&](int t) { return Affine{s_in[t], -s_mul[t]}; },
+                [&](int t, double y) { return s_out[t] = s_in[t] - s_mul[t] * y; });
+        __syncthreads();
+        if (!once) {
+            for (int t = threadIdx.x; t < len; t += blockDim.x) x[c0 + t] = s_out[t];
+            __syncthreads();
         }
-        __syncthreads();
-        for (int t = threadIdx.x; t < len; t += blockDim.x) x[c0 + t] = s_out[t];
-        __syncthreads();
     }
-    // backward: x(nym-1) = y/D'; x(j) = (y(j) - DU(j) x(j+1)) / D'(j)
+    // backward: x(nym-1) = y/D'; x(j) = (y(j) - DU(j) x(j+1)) / D'(j), rows from the top
     double xn = 0.0;
     for (int c1 = nym; c1 > 0; c1 -= kM00Chunk) {
         const int c0 = max(0, c1 - kM00Chunk), len = c1 - c0;
-        for (int t = threadIdx.x; t < len; t += blockDim.x) {
-            const int j = c0 + t;
-            s_in[t] = x[j];
-            s_mul[t] = lu[j * nzs];
-            s_cu[t] = j < nym - 1 ? du[j] : 0.0;
-        }
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            for (int t1 = len - 1; t1 >= 0; t1 -= 8) {
-                double a[8], ip[8], cu[8];
-#pragma unroll
-                for (int q = 0; q < 8; ++q) {
-                    const int t = max(t1 - q, 0);
-                    a[q] = s_in[t];
-                    ip[q] = s_mul[t];
-                    cu[q] = s_cu[t];
-                }
-#pragma unroll
-                for (int q = 0; q < 8; ++q) {
-                    const int t = t1 - q;
-                    if (t >= 0) {
-                        xn = c0 + t == nym - 1 ? a[q] * ip[q] : (a[q] - cu[q] * xn) * ip[q];
-                        s_out[t] = xn;
-                    }
-                }
+        if (!once) {
+            for (int t = threadIdx.x; t < len; t += blockDim.x) {
+                const int j = c0 + t;
+                s_out[t] = x[j];
+                s_ip[t] = lu[j * nzs];
+                s_cu[t] = j < nym - 1 ? du[j] : 0.0;
             }
+            __syncthreads();
         }
+        if (threadIdx.x < 64)
+            wave_recurrence(
+                len, xn,
+                [&](int t) {
+                    const int r = len - 1 - t;
+                    return Affine{s_out[r] * s_ip[r], -s_cu[r] * s_ip[r]};
+                },
+                [&](int t, double y) {
+                    const int r = len - 1 - t;
+                    return s_in[r] = (s_out[r] - s_cu[r] * y) * s_ip[r];
+                });
         __syncthreads();
-        for (int t = threadIdx.x; t < len; t += blockDim.x) x[c0 + t] = s_out[t];
+        for (int t = threadIdx.x; t < len; t += blockDim.x) x[c0 + t] = s_in[t];
         __syncthreads();
     }
 }
