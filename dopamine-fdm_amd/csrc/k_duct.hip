@@ -23,7 +23,7 @@
 // line's additive constant; k_zwall00 solves exactly that pinned system
 // (Thomas along z) and hands its eigenbasis image to k_yfft_solve, so phi
 // carries the reference's constant.
-#include "fft_lds.h"
+#include "ychunk.h"
 
 namespace dfp {
 
@@ -224,6 +224,60 @@ __global__ void __launch_bounds__(256) k_duct_ysolve(double2* __restrict__ S, co
                 gst<double2>(col + (long)j * nzp, make_double2(xx, xy));
             }
         }
+    }
+}
+
+// The same solve with the columns in registers (ychunk.h): a workgroup takes G
+// neighbouring eigenmodes of one kx, thread (chunk, mode) kDuctRows rows, so
+// the plane is read and written once and its loads are all in flight (32 + 8
+// bytes a mode and row; the lane-per-column sweep above moves 64 + 16 and
+// waits for four rows at a time): 147 -> 46 us at 256x192x256, 5.5 TB/s, bound
+// by HBM; 160 registers, held to three waves per SIMD (80 us at four, with
+// spills).  G is
+// the most of 16, 8, 4 modes (256 to 64 contiguous bytes a row) whose chunks
+// fit kDuctThreads threads; columns beyond kDuctThreads/4 chunks (1024 rows)
+// keep the sweep.
+constexpr int kDuctRows = 16;
+constexpr int kDuctThreads = 256;
+__global__ void __launch_bounds__(kDuctThreads) __attribute__((amdgpu_waves_per_eu(3)))
+k_duct_ychunk(double2* __restrict__ S, const double* __restrict__ lu, Ops o, int nym, int nzp, int G, int nch) {
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    constexpr int L = kDuctRows;
+    const int T = G * nch;
+    double2* ends = reinterpret_cast<double2*>(smem_raw);      // 48 T bytes
+    double* dls = reinterpret_cast<double*>(ends + 3 * T);     // DL(j-1), nch*L
+    double* dus = dls + nch * L;                               // DU(j), nch*L
+    const int ngrp = (nzp + G - 1) / G;
+    const int w = xcd_remap(blockIdx.x, gridDim.x);
+    const int kx = w / ngrp, m0 = (w - kx * ngrp) * G;
+    const int t = min((int)threadIdx.x, T - 1);
+    const int c = t / G, m = m0 + t - c * G;
+    const bool act = (int)threadIdx.x < T;
+    const int mm = min(m, nzp - 1);
+    const int j0 = c * L;
+    const auto col = gptr(S) + (long)kx * nym * nzp;
+    const auto piv = gptr(lu) + (long)kx * nym * nzp;
+    double2 x[L];
+    double pl[L], plm;
+#pragma unroll
+    for (int r = 0; r < L; ++r) {
+        const double2 v = gld<double2>(col + (uint32_t)(min(j0 + r, nym - 1) * nzp + mm));
+        x[r] = j0 + r < nym ? v : make_double2(0.0, 0.0);
+    }
+    plm = piv[(uint32_t)(max(j0 - 1, 0) * nzp + mm)];
+#pragma unroll
+    for (int r = 0; r < L; ++r) pl[r] = piv[(uint32_t)(min(j0 + r, nym - 1) * nzp + mm)];
+    for (int e = threadIdx.x; e < nch * L; e += blockDim.x) {
+        dls[e] = e > 0 && e < nym ? gptr(o.dl)[e - 1] : 0.0;
+        dus[e] = e < nym - 1 ? gptr(o.du)[e] : 0.0;
+    }
+    __syncthreads();
+    chunk_ysolve<L, double2>([&](int r) -> double2& { return x[r]; }, pl, plm, dls, dus, nym, j0, c, nch, G, t, T, act,
+                             false, ends);
+    if (act && m < nzp) {
+#pragma unroll
+        for (int r = 0; r < L; ++r)
+            if (j0 + r < nym) gst<double2>(col + (uint32_t)((j0 + r) * nzp + m), x[r]);
     }
 }
 
@@ -458,10 +512,19 @@ hipError_t launch_duct_solve(dfp_plan* p) {
     }
     e = launch_zeig(p, p->d_spec, p->duct_qf, p->d_spec2, "zeig_fwd");
     if (e != hipSuccess) return e;
-    const long n = (long)g.nxh * g.nzp;
     const int slot = prof_begin(p, "duct_ysolve");
-    hipLaunchKernelGGL(k_duct_ysolve, dim3(ceil_div(n, 256)), dim3(256), 0, p->stream, p->d_spec2, p->d_lu, p->ops,
-                       g.nxh, g.nym, g.nzp);
+    const int nch = ceil_div(g.nym, kDuctRows);
+    int G = 16;
+    while (G > 4 && G * nch > kDuctThreads) G /= 2;
+    if (G * nch <= kDuctThreads) {
+        const size_t lds = 48 * (size_t)(G * nch) + 2 * sizeof(double) * (size_t)nch * kDuctRows;
+        hipLaunchKernelGGL(k_duct_ychunk, dim3(g.nxh * ceil_div(g.nzp, G)), dim3(ceil_div(G * nch, 64) * 64), lds,
+                           p->stream, p->d_spec2, p->d_lu, p->ops, g.nym, g.nzp, G, nch);
+    } else {
+        const long n = (long)g.nxh * g.nzp;
+        hipLaunchKernelGGL(k_duct_ysolve, dim3(ceil_div(n, 256)), dim3(256), 0, p->stream, p->d_spec2, p->d_lu, p->ops,
+                           g.nxh, g.nym, g.nzp);
+    }
     prof_end(p, slot);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     return launch_zeig(p, p->d_spec2, p->duct_qi, p->d_spec, "zeig_inv");

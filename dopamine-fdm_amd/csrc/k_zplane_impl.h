@@ -14,13 +14,7 @@
 //   step (the two-step transform and LDS layout of k_zsolve.hip), and takes
 //   its BR rows of its mode back into registers: through LDS again, or, for
 //   16, 32 and 64 modes, across the lanes of its wave;
-//   y solve, with the plan's inverse pivots 1/D'(j) in registers: every chunk
-//   runs the elimination b'(j) = b(j) - DL(j-1)/D'(j-1) b'(j-1) from a zero
-//   carry for its last row and for the product of its multipliers, the chunks'
-//   ends are chained through LDS (each thread folds the ends before its own),
-//   and the elimination proper runs from the chained carry: the same
-//   recurrence as one long sweep, with only the carries associated
-//   differently.  The back substitution likewise from the top;
+//   y solve in chunks (ychunk.h), with the plan's inverse pivots in registers;
 //   inverse z transform: the same steps backwards, stored from registers.
 //
 // All of a plane's loads are in flight at once and no wave waits for another's
@@ -29,21 +23,9 @@
 // that need more threads than zplane_threads stay with the streaming kernel.
 #pragma once
 
-#include "fft_lds.h"
+#include "ychunk.h"
 
 namespace dfp {
-
-// Keeps the compiler from carrying the FP64 images of FP32 values from the
-// first sweep over them into the second (twice the registers of the values).
-template <int NB, int BR>
-__device__ __forceinline__ void keep(float2 (&x)[NB][BR]) {
-#pragma unroll
-    for (int b = 0; b < NB; ++b)
-#pragma unroll
-        for (int q = 0; q < BR; ++q) asm volatile("" : "+v"(x[b][q].x), "+v"(x[b][q].y));
-}
-template <int NB, int BR>
-__device__ __forceinline__ void keep(double2 (&)[NB][BR]) {}
 
 // Exchanges the register index r = 0..7 of v with bits 3..5 of the lane:
 // v[r] of lane (h, k) becomes v[h] of lane (r, k), k = lane % 8.  One register
@@ -124,10 +106,6 @@ __device__ __forceinline__ void zplane_run(int w0, int total, Rec rec, Same same
     double* dls = reinterpret_cast<double*>(A + (size_t)S * BR);  // DL(j-1), nch*L
     double* dus = dls + nch * L;                                  // DU(j), nch*L
     C* twl = reinterpret_cast<C*>(dus + nch * L);                 // w_n^e, N
-    double2* ce = reinterpret_cast<double2*>(smem_raw);           // chunk ends (in A between the transforms)
-    double2* ge = ce + S;
-    double* cp = reinterpret_cast<double*>(ge + S);
-    double* gp = cp + S;  // 48 S bytes in all, within A's 64 S or more
     // HBM accesses are a uniform base and a 32-bit byte offset per thread (one register per address): the
     // workgroup's planes and pivot rows span well under 4 GiB
     const int b0 = blk * zp.pp;
@@ -248,88 +226,12 @@ __device__ __forceinline__ void zplane_run(int w0, int total, Rec rec, Same same
         __syncthreads();
     }
 
-    // elimination.  Rows past the plane hold zero, take no multiplier and a
-    // zero inverse pivot, so they carry nothing into the back substitution.
-    if (j0 == 0) plm = 0.0;
-    {
-        double ex = 0.0, ey = 0.0, pi = 1.0, ip = plm;
-#pragma unroll
-        for (int r = 0; r < L; ++r) {
-            if (j0 + r >= nym) pl[r] = 0.0;
-            const double mu = dls[j0 + r] * ip;
-            const C v = x[r / BR][r % BR];
-            ex = (double)v.x - mu * ex;
-            ey = (double)v.y - mu * ey;
-            pi *= -mu;
-            ip = pl[r];
-        }
-        if (act) {
-            ce[t] = make_double2(ex, ey);
-            cp[t] = pi;
-        }
-    }
-    __syncthreads();
-    {
-        double bx = 0.0, by = 0.0, ip = plm;
-        keep(x);
-#pragma unroll 2
-        for (int q = 0; q < c; ++q) {
-            const double2 e = ce[t - (c - q) * N];
-            const double f = cp[t - (c - q) * N];
-            bx = e.x + f * bx;
-            by = e.y + f * by;
-        }
-#pragma unroll
-        for (int r = 0; r < L; ++r) {
-            const double mu = dls[j0 + r] * ip;
-            C& v = x[r / BR][r % BR];
-            bx = (double)v.x - mu * bx;
-            by = (double)v.y - mu * by;
-            v = CplxT<C>::make((Rl)bx, (Rl)by);
-            ip = pl[r];
-        }
-    }
-    // back substitution, from the top
-    {
-        double gx = 0.0, gy = 0.0, pi = 1.0;
-#pragma unroll
-        for (int r = L - 1; r >= 0; --r) {
-            const double d = dus[j0 + r];
-            const C v = x[r / BR][r % BR];
-            gx = ((double)v.x - d * gx) * pl[r];
-            gy = ((double)v.y - d * gy) * pl[r];
-            pi *= -d * pl[r];
-        }
-        if (act) {
-            ge[t] = make_double2(gx, gy);
-            gp[t] = pi;
-        }
-    }
-    __syncthreads();
-    {
-        keep(x);
-        const bool is00 = zp.zero00 && b0 + tp == 0 && m == 0;  // the FP32 form solves the (0,0) mode on its own
-        double xx = 0.0, xy = 0.0;
-#pragma unroll 2
-        for (int q = nch - 1; q > c; --q) {
-            const double2 e = ge[t + (q - c) * N];
-            const double f = gp[t + (q - c) * N];
-            xx = e.x + f * xx;
-            xy = e.y + f * xy;
-        }
-#pragma unroll
-        for (int r = L - 1; r >= 0; --r) {
-            const double d = dus[j0 + r];
-            C& v = x[r / BR][r % BR];
-            xx = ((double)v.x - d * xx) * pl[r];
-            xy = ((double)v.y - d * xy) * pl[r];
-            v = is00 ? CplxT<C>::make((Rl)0, (Rl)0) : CplxT<C>::make((Rl)xx, (Rl)xy);
-        }
-    }
+    chunk_ysolve<L, C>([&](int r) -> C& { return x[r / BR][r % BR]; }, pl, plm, dls, dus, nym, j0, c, nch, N, t, S, act,
+                       zp.zero00 && b0 + tp == 0 && m == 0, reinterpret_cast<double2*>(smem_raw));
+
     const int wn = w + gridDim.x;
     loaded = wn < total && same(wn);
     const int kn = blk + gridDim.x;  // an item of the same record
-    __syncthreads();
 
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
