@@ -612,6 +612,7 @@ int dfp_plan_create_tuned(const dfp_grid* g, int precision, int device, const df
     // to the eigenbasis, Qi = Qz^T W^(-1/2) back; the eigenmode of the zero
     // eigenvalue (by magnitude, :207) is pinned at kx = 0
     std::vector<double> duct_tab;
+    size_t duct_half = 0;  // offset of the even and odd halves in duct_tab (0: none)
     if (G.zbc == 1) {
         const int n = G.nzp;
         auto Z = [&](int k) { return p->hz[k - 1]; };
@@ -626,8 +627,38 @@ int dfp_plan_create_tuned(const dfp_grid* g, int precision, int device, const df
             if (kk + 1 < n) so[kk] = 1.0 / ((ZG(k + 1) - ZG(k)) * std::sqrt((Z(k) - Z(k - 1)) * (Z(k + 1) - Z(k))));
         }
         for (int k = 0; k < n; ++k) sw[k] = std::sqrt(Z(k + 2) - Z(k + 1));
-        if (!std::isfinite(std::accumulate(sd.begin(), sd.end(), 0.0)) || !symtri_eigen(n, sd, so, Q))
-            return bail(DFP_E_NONFINITE);
+        if (!std::isfinite(std::accumulate(sd.begin(), sd.end(), 0.0))) return bail(DFP_E_NONFINITE);
+        // a grid symmetric about its middle up to the rounding of its coordinates
+        // (a few units in the last place of the largest one, in every cell width
+        // and centre spacing): even and odd eigenvectors
+        bool sym = n > 1;
+        {
+            double zmax = 0.0;
+            for (double v : p->hz) zmax = std::max(zmax, std::fabs(v));
+            const double tol = 16.0 * std::numeric_limits<double>::epsilon() * zmax;
+            for (int k = 0; k < n && sym; ++k) {
+                sym = std::fabs((Z(k + 2) - Z(k + 1)) - (Z(n + 1 - k) - Z(n - k))) <= tol;
+                if (k + 1 < n)
+                    sym = sym && std::fabs((ZG(k + 3) - ZG(k + 2)) - (ZG(n + 1 - k) - ZG(n - k))) <= tol;
+            }
+        }
+        bool ok;
+        if (sym) {
+            // the same S in long double, its rows built from the coordinates (the
+            // diagonal's rounding would show in the smallest eigenvalues)
+            std::vector<long double> ld(n, 0.0L), le(n > 1 ? n - 1 : 1, 0.0L);
+            for (int k = 0; k + 1 < n; ++k) {
+                const long double w0 = (long double)Z(k + 2) - Z(k + 1), w1 = (long double)Z(k + 3) - Z(k + 2);
+                const long double gap = (long double)ZG(k + 3) - ZG(k + 2);
+                le[k] = 1.0L / (gap * std::sqrt(w0 * w1));
+                ld[k] -= 1.0L / (gap * w0);
+                ld[k + 1] -= 1.0L / (gap * w1);
+            }
+            ok = symtri_eigen_sym(n, ld, le, sd, Q);
+        } else {
+            ok = symtri_eigen(n, sd, so, Q);
+        }
+        if (!ok) return bail(DFP_E_NONFINITE);
         double lmax = 0.0;
         for (double l : sd) lmax = std::max(lmax, std::fabs(l));
         for (int m = 0; m < n && p->pin_m < 0; ++m)
@@ -640,6 +671,22 @@ int dfp_plan_create_tuned(const dfp_grid* g, int precision, int device, const df
                 duct_tab[(size_t)n * n + (size_t)m * n + k] = q / sw[k];    // Qi(m, k)
             }
         std::copy(sd.begin(), sd.end(), duct_tab.begin() + (size_t)2 * n * n);
+        if (sym) {
+            // Qf = (Be, Bo) on the sums and differences, Qi = their transposes on the halves; W is
+            // symmetric too, so each half row stands for its mirror image
+            const int h = (n + 1) / 2;
+            duct_half = duct_tab.size();
+            duct_tab.resize(duct_half + (size_t)4 * h * h, 0.0);
+            double* sf = duct_tab.data() + duct_half;
+            double* si = sf + (size_t)2 * h * h;
+            for (int par = 0; par < 2; ++par)
+                for (int m = 0; m < (par ? n - h : h); ++m)
+                    for (int k = 0; k < h; ++k) {
+                        const size_t qf = (size_t)k * n + (par ? h + m : m), qi = (size_t)n * n + (size_t)(par ? h + m : m) * n + k;
+                        sf[(size_t)par * h * h + (size_t)k * h + m] = duct_tab[qf];
+                        si[(size_t)par * h * h + (size_t)m * h + k] = duct_tab[qi];
+                    }
+        }
     }
 
     std::vector<double> tab;
@@ -762,6 +809,11 @@ int dfp_plan_create_tuned(const dfp_grid* g, int precision, int device, const df
         p->duct_qf = p->d_duct;
         p->duct_qi = p->d_duct + nn;
         p->duct_lam = p->d_duct + 2 * nn;
+        if (duct_half) {
+            const size_t h = (G.nzp + 1) / 2;
+            p->duct_sf = p->d_duct + duct_half;
+            p->duct_si = p->duct_sf + 2 * h * h;
+        }
         if (G.ybc == 1 && (launch_duct_lu(p) != hipSuccess || hipStreamSynchronize(p->stream) != hipSuccess))
             return bail(DFP_E_HIP);
     } else if (G.ybc == 1) {  // pivots of the wall solve

@@ -208,10 +208,14 @@ struct dfp_plan {
     // the duct (z walls): second spectrum (the eigenmode planes), the z
     // eigenbasis tables and the pinned eigenmode (the zero eigenvalue)
     double2* d_spec2 = nullptr;
-    double* d_duct = nullptr;    // Qf (nzp x nzp, row k) | Qi (nzp x nzp, row m) | lambda_z (nzp)
+    double* d_duct = nullptr;    // Qf (nzp x nzp, row k) | Qi (nzp x nzp, row m) | lambda_z (nzp) | halves
     const double* duct_qf = nullptr;
     const double* duct_qi = nullptr;
     const double* duct_lam = nullptr;
+    // z grid symmetric about its middle: the even and odd halves of Qf and Qi (h x h each, h = ceil(nzp/2)),
+    // the eigenmodes ordered even, odd (null otherwise: ascending order)
+    const double* duct_sf = nullptr;
+    const double* duct_si = nullptr;
     int pin_m = -1;
     // z walls with a periodic y: Dzz's three diagonals, the multipliers DL/D'
     // and inverse pivots of the pinned kx = ky = 0 z system (in d_tables),

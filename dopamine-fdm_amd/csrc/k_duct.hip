@@ -8,6 +8,8 @@
 //                  complex plane, B real: Qf = W^(1/2) Qz forward,
 //                  Qi = Qz^T W^(-1/2) back (a batched complex-by-real GEMM
 //                  on the FP64 matrix cores)
+//   k_zeig_sym     the same for a z grid symmetric about its middle: even and
+//                  odd eigenmodes apart, half the work
 //   k_duct_lu      inverse pivots of each (kx, m) system Dyy + kxx + lambda_z(m)
 //                  (the pin where kx = 0 on the zero eigenvalue)
 //   k_duct_ysolve  elimination and back substitution along y, one lane per
@@ -133,6 +135,148 @@ __global__ void __launch_bounds__(kGemmThreads) k_zeig_mfma(const double2* __res
             if (j + 4 < nrow) gst<double2>(cp + (long)(j + 4) * N + n, make_double2(acc[r][c][2], acc[r][c][3]));
         }
     }
+}
+
+// The same transforms for a z grid that is symmetric about its middle (uniform
+// or symmetric tanh; Plan set-up), whose eigenvectors are even or odd: the
+// even modes see only the sums s(k) = p(k) + p(K-1-k) of the plane, the odd
+// ones the differences d(k), k < h = ceil(K/2), so each is a GEMM of half the
+// depth and the work halves (Q: the eigenmodes in the order even, odd).
+//   forward  z(m) = sum_k s(k) Be(k, m) (m < h), z(h+m) = sum_k d(k) Bo(k, m)
+//   inverse  e(k) = sum_m z(m) Be(m, k), o(k) = sum_m z(h+m) Bo(m, k),
+//            p(k) = e + o, p(K-1-k) = e - o
+// Be, Bo are h x h (B then B + h*h; an odd K pads the odd modes with zeros).
+// A block's tile is 64 complex rows x 32 columns of both parities, the rows'
+// two images staged side by side in LDS (double rows of kSymKC + 1 for A and
+// 48 for B: fragment reads and staging writes fall in distinct banks), so
+// every plane value is loaded once per tile; the inverse holds e and o of the
+// same output in the same lane.  Workgroups are renumbered so that the column
+// tiles of one row tile share an XCD's L2.  160 registers (three workgroups a
+// CU; 107 us at two).  162 -> 98 us forward and 87 us back at 256x192x256
+// (3.25 GFLOP, 203 MB): without the products it runs in 65 and 49 us, without
+// the plane loads in 75, so loads and matrix pipes overlap but in part.
+// Fragments loaded straight from memory, without LDS for A, took 107 and 99.
+constexpr int kSymKC = 16;  // k per LDS stage
+constexpr int kSymTN = 32;  // columns of each parity per tile
+template <bool INV>
+__global__ void __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(3)))
+k_zeig_sym(const double2* __restrict__ A, const double* __restrict__ B, double2* __restrict__ C, int nym, int nrow,
+           int K, int nbx, int nby) {
+    __shared__ double As[2][2 * kGemmTJ][kSymKC + 1];
+    __shared__ double Bs[2][kSymKC][48];
+    const int t = threadIdx.x;
+    const int lane = t & 63, w = t >> 6;
+    const int li = lane & 15, lk = lane >> 4;
+    const int h = (K + 1) / 2;
+    const int W = xcd_remap(blockIdx.x, gridDim.x);
+    const int bxy = W / nbx, kx = bxy / nby;
+    const int n0 = (W - bxy * nbx) * kSymTN, j0 = (bxy - kx * nby) * kGemmTJ;
+    const auto a = gptr(A) + (long)kx * nym * K;
+    const auto b = gptr(B);
+    constexpr int QA = kGemmTJ * kSymKC / kGemmThreads, QB = kSymKC * kSymTN / kGemmThreads;
+    // the next stage's values, in flight while the current stage multiplies: rows past the plane repeat its
+    // last one and are not stored; k past h repeats the row's last value against zero rows of B
+    double2 p1[QA], p2[QA];
+    double pb[2][QB];
+    const int tj = t / kSymKC, tk = t % kSymKC;
+    auto fetch = [&](int k0) {
+        const int k = min(k0 + tk, h - 1);
+        const int k2 = INV ? min(h + k, K - 1) : K - 1 - k;  // the odd mode, or the mirrored cell
+#pragma unroll
+        for (int q = 0; q < QA; ++q) {
+            const uint32_t row = (uint32_t)(min(j0 + tj + q * (kGemmThreads / kSymKC), nrow - 1) * K);
+            p1[q] = gld<double2>(a + (row + k));
+            p2[q] = gld<double2>(a + (row + k2));
+        }
+#pragma unroll
+        for (int q = 0; q < QB; ++q) {
+            const int e = t + q * kGemmThreads;
+            const int kb = k0 + e / kSymTN, n = n0 + e % kSymTN;
+            const uint32_t at = (uint32_t)(min(kb, h - 1) * h + min(n, h - 1));
+            pb[0][q] = b[at];
+            pb[1][q] = b[(uint32_t)(h * h) + at];
+            if (kb >= h || n >= h) pb[0][q] = pb[1][q] = 0.0;
+        }
+    };
+    auto stage = [&](int k0) {
+        const bool mid = !INV && 2 * (k0 + tk) == K - 1;  // the middle cell of an odd K: its own image
+#pragma unroll
+        for (int q = 0; q < QA; ++q) {
+            const int jj = tj + q * (kGemmThreads / kSymKC);
+            const int cr = jj & 7;                                     // complex row within its tile
+            const int i0 = 16 * (jj >> 3) + (cr & 3) + 8 * (cr >> 2);  // its re row; im is 4 rows on
+            double2 u = p1[q], v = p2[q];
+            if (!INV) {
+                u = mid ? p1[q] : make_double2(p1[q].x + p2[q].x, p1[q].y + p2[q].y);
+                v = mid ? make_double2(0.0, 0.0) : make_double2(p1[q].x - p2[q].x, p1[q].y - p2[q].y);
+            }
+            As[0][i0][tk] = u.x;
+            As[0][i0 + 4][tk] = u.y;
+            As[1][i0][tk] = v.x;
+            As[1][i0 + 4][tk] = v.y;
+        }
+#pragma unroll
+        for (int q = 0; q < QB; ++q) {
+            const int e = t + q * kGemmThreads;
+            Bs[0][e / kSymTN][e % kSymTN] = pb[0][q];
+            Bs[1][e / kSymTN][e % kSymTN] = pb[1][q];
+        }
+    };
+    v4d acc[2][2][2];  // parity, tile row, tile column
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+        for (int r = 0; r < 2; ++r)
+#pragma unroll
+            for (int c = 0; c < 2; ++c) acc[s][r][c] = v4d{0.0, 0.0, 0.0, 0.0};
+    fetch(0);
+    for (int k0 = 0; k0 < h; k0 += kSymKC) {
+        stage(k0);
+        __syncthreads();
+        if (k0 + kSymKC < h) fetch(k0 + kSymKC);
+#pragma unroll
+        for (int ks = 0; ks < kSymKC / 4; ++ks) {
+            const int kk = 4 * ks + lk;
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                double av[2], bv[2];
+#pragma unroll
+                for (int r = 0; r < 2; ++r) av[r] = As[s][32 * w + 16 * r + li][kk];
+#pragma unroll
+                for (int c = 0; c < 2; ++c) bv[c] = Bs[s][kk][16 * c + li];
+#pragma unroll
+                for (int r = 0; r < 2; ++r)
+#pragma unroll
+                    for (int c = 0; c < 2; ++c)
+                        acc[s][r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[r], bv[c], acc[s][r][c], 0, 0, 0);
+            }
+        }
+        __syncthreads();
+    }
+    const auto cp = gptr(C) + (long)kx * nym * K;
+#pragma unroll
+    for (int r = 0; r < 2; ++r)
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            const int n = n0 + 16 * c + li;
+            if (n >= h) continue;
+            const int n2 = INV ? K - 1 - n : h + n;
+            const bool two = INV ? n2 != n : n2 < K;
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {  // complex rows j and j + 4
+                const int j = j0 + 16 * w + 8 * r + lk + 4 * q;
+                if (j >= nrow) continue;
+                double2 u = make_double2(acc[0][r][c][2 * q], acc[0][r][c][2 * q + 1]);
+                double2 v = make_double2(acc[1][r][c][2 * q], acc[1][r][c][2 * q + 1]);
+                if (INV) {
+                    const double2 e = u, o = v;
+                    u = make_double2(e.x + o.x, e.y + o.y);
+                    v = make_double2(e.x - o.x, e.y - o.y);
+                }
+                gst<double2>(cp + (long)j * K + n, u);
+                if (two) gst<double2>(cp + (long)j * K + n2, v);
+            }
+        }
 }
 
 // inverse pivots lu[(kx*nym + j)*nzp + m] = 1/D'(j) of the elimination
@@ -465,12 +609,28 @@ hipError_t launch_duct_lu(dfp_plan* p) {
     return hipGetLastError();
 }
 
-static hipError_t launch_zeig(dfp_plan* p, const double2* A, const double* B, double2* C, const char* name) {
+// z eigenbasis transform of the spectrum, forward (d_spec -> d_spec2) or back
+static hipError_t launch_zeig(dfp_plan* p, bool inv) {
     const Geo& g = p->geo;
     const int nrow = g.ybc == 0 ? g.nym - 1 : g.nym;  // the duplicate row of a periodic y is not transformed
-    const dim3 grid(ceil_div(g.nzp, kGemmTN), ceil_div(nrow, kGemmTJ), g.nxh);
-    const int slot = prof_begin(p, name);
-    hipLaunchKernelGGL(k_zeig_mfma, grid, dim3(kGemmThreads), 0, p->stream, A, B, C, g.nym, nrow, g.nzp, g.nzp);
+    const double2* A = inv ? p->d_spec2 : p->d_spec;
+    double2* C = inv ? p->d_spec : p->d_spec2;
+    const int slot = prof_begin(p, inv ? "zeig_inv" : "zeig_fwd");
+    const int nby = ceil_div(nrow, kGemmTJ);
+    if (p->duct_sf) {
+        const int nbx = ceil_div((g.nzp + 1) / 2, kSymTN);
+        const dim3 grid(nbx * nby * g.nxh);
+        if (inv)
+            hipLaunchKernelGGL(k_zeig_sym<true>, grid, dim3(kGemmThreads), 0, p->stream, A, p->duct_si, C, g.nym, nrow,
+                               g.nzp, nbx, nby);
+        else
+            hipLaunchKernelGGL(k_zeig_sym<false>, grid, dim3(kGemmThreads), 0, p->stream, A, p->duct_sf, C, g.nym,
+                               nrow, g.nzp, nbx, nby);
+    } else {
+        const dim3 grid(ceil_div(g.nzp, kGemmTN), nby, g.nxh);
+        hipLaunchKernelGGL(k_zeig_mfma, grid, dim3(kGemmThreads), 0, p->stream, A, inv ? p->duct_qi : p->duct_qf, C,
+                           g.nym, nrow, g.nzp, g.nzp);
+    }
     prof_end(p, slot);
     return hipGetLastError();
 }
@@ -499,7 +659,7 @@ hipError_t launch_duct_solve(dfp_plan* p) {
         prof_end(p, slot);
         if ((e = hipGetLastError()) != hipSuccess) return e;
         if (fork && (e = hipEventRecord(p->join_ev, p->aux)) != hipSuccess) return e;
-        if ((e = launch_zeig(p, p->d_spec, p->duct_qf, p->d_spec2, "zeig_fwd")) != hipSuccess) return e;
+        if ((e = launch_zeig(p, false)) != hipSuccess) return e;
         if (fork && (e = hipStreamWaitEvent(p->stream, p->join_ev, 0)) != hipSuccess) return e;
         const int G = p->gy, ngrp = ceil_div(g.nzp, G), ntwy = twiddle_count(p->fy);
         slot = prof_begin(p, "yfft_solve");
@@ -508,9 +668,9 @@ hipError_t launch_duct_solve(dfp_plan* p) {
                            g.nym, g.nzp, G, FastDiv((uint32_t)G));
         prof_end(p, slot);
         if ((e = hipGetLastError()) != hipSuccess) return e;
-        return launch_zeig(p, p->d_spec2, p->duct_qi, p->d_spec, "zeig_inv");
+        return launch_zeig(p, true);
     }
-    e = launch_zeig(p, p->d_spec, p->duct_qf, p->d_spec2, "zeig_fwd");
+    e = launch_zeig(p, false);
     if (e != hipSuccess) return e;
     const int slot = prof_begin(p, "duct_ysolve");
     const int nch = ceil_div(g.nym, kDuctRows);
@@ -527,7 +687,7 @@ hipError_t launch_duct_solve(dfp_plan* p) {
     }
     prof_end(p, slot);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    return launch_zeig(p, p->d_spec2, p->duct_qi, p->d_spec, "zeig_inv");
+    return launch_zeig(p, true);
 }
 
 }  // namespace dfp
