@@ -137,6 +137,7 @@ void dyy(const std::vector<double>& y, const std::vector<double>& yg, std::vecto
 struct Shape {
     int R = 1, T = 1, Ti = 1, G = 1, fused = 0;  // T, Ti: columns of the forward, inverse x kernels
     int gy = 1;                                  // periodic y: columns per y-transform call
+    int py_nb = 0, py_nch = 0;                   // periodic y with the planes in registers: passes, chunks
     FftDesc fx{}, fz{}, fy{};
 };
 
@@ -214,7 +215,7 @@ int choose_shape(const dfp_grid* g, int f32, size_t lds_limit, const dfp_tuning*
     if (py && !factor(g->nym - 1, fy)) return DFP_E_UNSUPPORTED;
     const bool allow_fused = want_f == 2 || (want_f == 0 && want_G == 0);
     const bool allow_split = want_f != 2 && !py;
-    std::vector<Shape> fused, split;
+    std::vector<Shape> fused, split, planes;
     for (int R : kRadices) {
         if (g->nzp % R != 0 || (want_R > 0 && R != want_R)) continue;
         Shape sh;
@@ -224,6 +225,15 @@ int choose_shape(const dfp_grid* g, int f32, size_t lds_limit, const dfp_tuning*
         sh.T = x_columns(sh, g->nxp, g->nzp, lds_limit, cs, want_T, 0, dct);
         sh.Ti = x_columns(sh, g->nxp, g->nzp, lds_limit, cs, want_T, 1, dct);
         if (sh.T == 0 || sh.Ti == 0 || sh.fz.n > 256) continue;
+        if (py && want_f == 0) {
+            Shape f = sh;
+            if (zplane_py_shape(sh.fz.n, g->nym - 1, lds_limit, f.py_nb, f.py_nch)) {
+                f.fused = 1;
+                f.G = zf_rows_per_call(f.fz);
+                f.fy = fy;
+                planes.push_back(f);
+            }
+        }
         if (py) {
             const int gy = zf_py_columns(fy, sh.fz.n);
             if (gy > 0 && zf_py_lds_bytes(g->nym, sh.fz.n, twiddle_count(sh.fz), twiddle_count(fy)) <= lds_limit) {
@@ -246,6 +256,16 @@ int choose_shape(const dfp_grid* g, int f32, size_t lds_limit, const dfp_tuning*
             if (want_G > 0) q.G = want_G <= q.G ? want_G : 0;
             if (q.G >= 1) split.push_back(q);
         }
+    }
+    // periodic y, planes in registers: the smallest split from 4 on (the x
+    // kernels' spectrum segments shorten with R), else the largest below.
+    // 256x257x256: 682 us in LDS (R = 16), 558-567 in registers (R = 8);
+    // 64x65x64: 56 -> 43 us (R = 4), 128x129x96: 94 -> 76 (R = 4; 73 at 8).
+    if (!planes.empty()) {
+        for (const Shape& q : planes)
+            if (q.R >= 4) { out = q; return DFP_OK; }
+        out = planes.back();
+        return DFP_OK;
     }
     // default: the split pair with the classic split (R = 4 when it leaves at
     // least 8 points per row, else 2, else 3, else none); the fused form when
@@ -562,6 +582,8 @@ int dfp_plan_create_tuned(const dfp_grid* g, int precision, int device, const df
     p->zfused = sh.fused;
     p->fy = sh.fy;
     p->gy = sh.gy;
+    p->zp_nb = sh.py_nb;
+    p->zp_nch = sh.py_nch;
     if (!sh.fused) z_two_pass(sh.fz.n, p->zn1, p->zn2);
     // whole sub-planes in registers where they fit, unless the streaming kernel was asked for
     if (!sh.fused && g->z_bc_type == 0 && !(tune && (tune->z_rows || tune->z_fused)) &&
@@ -773,6 +795,9 @@ int dfp_plan_create_tuned(const dfp_grid* g, int precision, int device, const df
         stage_twiddles(p->fy, tw);
         for (int st = 0; st < p->fy.nst; ++st) p->fy.twoff[st] -= (int)o_ty;
     }
+    const size_t o_ty2 = tw.size();
+    if (G.ybc == 0)
+        for (int e = 0; e < G.nym - 1; ++e) tw.push_back(expi(e, G.nym - 1));
     if (hipMalloc(&p->d_tw, sizeof(double2) * tw.size()) != hipSuccess) return bail(DFP_E_NOMEM);
     if (hipMemcpy(p->d_tw, tw.data(), sizeof(double2) * tw.size(), hipMemcpyHostToDevice) != hipSuccess)
         return bail(DFP_E_HIP);
@@ -782,6 +807,7 @@ int dfp_plan_create_tuned(const dfp_grid* g, int precision, int device, const df
     p->tw_zs = p->d_tw + o_zs;
     p->tw_z2 = p->d_tw + o_t2;
     p->tw_y = p->d_tw + o_ty;
+    p->tw_y2 = p->d_tw + o_ty2;
     if (precision == DFP_FP32_REFINE) {
         std::vector<float2> tw32(tw.size());
         for (size_t e = 0; e < tw.size(); ++e) tw32[e] = make_float2((float)tw[e].x, (float)tw[e].y);

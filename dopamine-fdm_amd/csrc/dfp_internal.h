@@ -145,6 +145,7 @@ struct ZyPar {
     ZPar<C> z;
     FftDesc fy;          // y FFT of length nym-1
     const C* twy;        // its stage twiddles
+    const C* twy2;       // exp(-2 pi i e / (nym-1)), e < nym-1 (planes in registers)
     const double* kxx;   // nxh
     const double* kyy;   // nym-1
     const double* kzz;   // nzp
@@ -204,6 +205,7 @@ struct dfp_plan {
     dfp::FftDesc fx{}, fz{};     // x: length nxp/2 (half-length complex), z: length nzp/zr
     dfp::FftDesc fy{};           // periodic y: length nym-1
     const double2* tw_y = nullptr;  // periodic y: stage twiddles of fy
+    const double2* tw_y2 = nullptr; // periodic y: exp(-2 pi i e / (nym-1)), e < nym-1
     int gy = 1;                  // periodic y: columns per y-transform call
     // the duct (z walls): second spectrum (the eigenmode planes), the z
     // eigenbasis tables and the pinned eigenmode (the zero eigenvalue)
@@ -336,6 +338,10 @@ size_t zf_py_lds_bytes(int nym, int n, int ntwz, int ntwy);
 int zf_py_columns(const FftDesc& fy, int n);
 size_t zf_lds_bytes(const dfp_plan* p, int f32);
 int zf_rows_per_call(const FftDesc& fz);
+// the same with the planes in registers: nym-1 = 16, 32, 64, 128 or 256 rows (k_zplane_py.hip)
+bool zplane_py_shape(int n, int nyp, size_t lds_limit, int& nb, int& nch);
+size_t zplane_py_lds(int threads, int n, int nyp);
+hipError_t launch_zplane_py(dfp_plan* p, ZyPar<double2> zy);
 // FP32 form
 hipError_t launch_rfft_x32(dfp_plan* p, int mode, const XArgs& a);
 hipError_t launch_zsolve32(dfp_plan* p);

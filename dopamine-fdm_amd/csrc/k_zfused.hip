@@ -298,6 +298,13 @@ hipError_t launch_zfused_py(dfp_plan* p) {
     q.gy = p->gy;
     q.div_gy = FastDiv((uint32_t)p->gy);
     q.inv_ny = 1.0 / (double)(p->geo.nym - 1);
+    q.twy2 = p->tw_y2;
+    if (p->zp_nb) {  // the planes fit registers (zplane_py_shape)
+        const int slot = prof_begin(p, "zfused_py");
+        const hipError_t e = launch_zplane_py(p, q);
+        prof_end(p, slot);
+        return e;
+    }
     const size_t lds = zf_py_lds_bytes(p->geo.nym, p->fz.n, q.z.ntw, q.ntwy);
     const int slot = prof_begin(p, "zfused_py");
     hipLaunchKernelGGL(k_zfused_py, dim3(q.z.nblocks), dim3(kZfPyThreads), lds, p->stream, q);

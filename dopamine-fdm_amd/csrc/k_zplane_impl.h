@@ -72,12 +72,97 @@ __device__ __forceinline__ void lane_transpose(C (&v)[8]) {
         }
 }
 
+// The y solve of a periodic y for columns in registers: nyp = NCH*L independent
+// rows, thread (chunk c, mode m) holding rows c + NCH r, r < L, of its mode.
+//   X(ky) = sum_c w_NCH^{c k1} w_nyp^{c k2} [sum_r w_L^{r k2} x(c + NCH r)],  ky = k2 + L k1
+// so the length-L transform runs in registers, the real and then the imaginary
+// parts are exchanged through LDS (all chunks of one k2 to one thread, S*L
+// doubles), and the length-NCH transforms run in registers again; the modes
+// are divided by lx + kyy(ky) + lz (1/nyp folded in, the zero mode set to
+// zero) and taken back the same way.  A thread takes the IT = L/NCH values
+// k2 = c + NCH s.  twy[e] = exp(-2 pi i e/nyp).
+template <int NCH, int L, int N>
+__device__ __forceinline__ void periodic_ysolve(double2 (&x)[L], double* ex, const double2* twy, const double* kyy,
+                                                double lxz, double inv_ny, bool zero_plane, int c, int m, int base,
+                                                bool act) {
+    constexpr int IT = L / NCH;
+    static_assert(L % NCH == 0, "whole second-step items");
+    dft_reg<-1, L>(x);
+#pragma unroll
+    for (int k2 = 1; k2 < L; ++k2) x[k2] = twiddle<-1>(x[k2], twy[c * k2]);
+    // slot of (k2, chunk) for this thread's plane and mode
+    auto slot = [&](int k2, int cc) { return base + (k2 * NCH + cc) * N + m; };
+    auto to_chunks = [&]() {  // x[k2] of chunk c -> x[s*NCH + cc] = chunk cc of k2 = c + NCH s
+#pragma unroll
+        for (int part = 0; part < 2; ++part) {
+            if (act) {
+#pragma unroll
+                for (int k2 = 0; k2 < L; ++k2) ex[slot(k2, c)] = part ? x[k2].y : x[k2].x;
+            }
+            __syncthreads();
+#pragma unroll
+            for (int s = 0; s < IT; ++s)
+#pragma unroll
+                for (int cc = 0; cc < NCH; ++cc) {
+                    const double v = ex[slot(c + NCH * s, cc)];
+                    if (part) x[s * NCH + cc].y = v;
+                    else x[s * NCH + cc].x = v;
+                }
+            __syncthreads();
+        }
+    };
+    auto to_rows = [&]() {  // and back
+#pragma unroll
+        for (int part = 0; part < 2; ++part) {
+            if (act) {
+#pragma unroll
+                for (int s = 0; s < IT; ++s)
+#pragma unroll
+                    for (int cc = 0; cc < NCH; ++cc)
+                        ex[slot(c + NCH * s, cc)] = part ? x[s * NCH + cc].y : x[s * NCH + cc].x;
+            }
+            __syncthreads();
+#pragma unroll
+            for (int k2 = 0; k2 < L; ++k2) {
+                const double v = ex[slot(k2, c)];
+                if (part) x[k2].y = v;
+                else x[k2].x = v;
+            }
+            __syncthreads();
+        }
+    };
+    to_chunks();
+#pragma unroll
+    for (int s = 0; s < IT; ++s) {
+        double2 v[NCH];
+#pragma unroll
+        for (int cc = 0; cc < NCH; ++cc) v[cc] = x[s * NCH + cc];
+        dft_reg<-1, NCH>(v);
+#pragma unroll
+        for (int k1 = 0; k1 < NCH; ++k1) {
+            const int ky = c + NCH * s + L * k1;
+            const double f = inv_ny / (lxz + kyy[ky]);
+            v[k1] = zero_plane && ky == 0 ? make_double2(0.0, 0.0) : make_double2(v[k1].x * f, v[k1].y * f);
+        }
+        dft_reg<1, NCH>(v);
+#pragma unroll
+        for (int cc = 0; cc < NCH; ++cc) x[s * NCH + cc] = v[cc];
+    }
+    to_rows();
+#pragma unroll
+    for (int k2 = 1; k2 < L; ++k2) x[k2] = twiddle<1>(x[k2], twy[c * k2]);
+    dft_reg<1, L>(x);
+}
+
 // Runs the workgroup's items: rec(w, blk) gives the case record of item w and
 // its block there, same(w) whether the next item w has the record of the last
 // one.  An item's rows load into the registers that the item before frees,
-// behind that item's inverse transform and stores.
-template <typename C, int N1, int N2, int BR, int NB, typename Rec, typename Same>
-__device__ __forceinline__ void zplane_run(int w0, int total, Rec rec, Same same, unsigned char* smem_raw) {
+// behind that item's inverse transform and stores.  NCHY: the chunks of a
+// periodic y (rows interleaved over them, periodic_ysolve, zy its tables; row
+// nym-1 receives row 0's values), or 0 for the wall solve.
+template <typename C, int N1, int N2, int BR, int NB, int NCHY, typename Rec, typename Same>
+__device__ __forceinline__ void zplane_run(int w0, int total, Rec rec, Same same, const ZyPar<C>* zy,
+                                           unsigned char* smem_raw) {
     using Rl = typename CplxT<C>::real;
     constexpr int N = N1 * N2;
     constexpr int L = BR * NB;
@@ -94,7 +179,9 @@ __device__ __forceinline__ void zplane_run(int w0, int total, Rec rec, Same same
     for (int w = w0; w < total; w += gridDim.x) {
     int blk;
     const ZPar<C>& zp = rec(w, blk);
-    const int nym = zp.nym, R = zp.R, nch = zp.nch;
+    const int nym = zp.nym, R = zp.R, nch = NCHY ? NCHY : zp.nch;
+    const int nrow = NCHY ? nym - 1 : nym;           // rows transformed
+    constexpr int kStep = NCHY ? NCHY * BR : BR;     // rows from one pass to the next
     const int nzs = zp.nzp / 2 + 1;
     const int S1 = N * nch, S = S1 * zp.pp;  // threads per plane, per workgroup
     // opaque, so that no address derived from it is held in a register over the loop
@@ -106,6 +193,7 @@ __device__ __forceinline__ void zplane_run(int w0, int total, Rec rec, Same same
     double* dls = reinterpret_cast<double*>(A + (size_t)S * BR);  // DL(j-1), nch*L
     double* dus = dls + nch * L;                                  // DU(j), nch*L
     C* twl = reinterpret_cast<C*>(dus + nch * L);                 // w_n^e, N
+    C* twy = twl + N;                                             // periodic y: w_nyp^e (and kyy in dls)
     // HBM accesses are a uniform base and a 32-bit byte offset per thread (one register per address): the
     // workgroup's planes and pivot rows span well under 4 GiB
     const int b0 = blk * zp.pp;
@@ -131,7 +219,8 @@ __device__ __forceinline__ void zplane_run(int w0, int total, Rec rec, Same same
         const int it = tt + s * S;
         const int v = it / N1;
         const int vc = v / BR, p = vc / nch;
-        return Item{v, it - v * N1, p, (vc - p * nch) * L + v - vc * BR};
+        const int cc = vc - p * nch, q = v - vc * BR;
+        return Item{v, it - v * N1, p, NCHY ? cc + NCHY * q : cc * L + q};
     };
     // rows of pass b of block k (a partial last workgroup repeats its last plane, unstored)
     auto load_rows = [&](int k, int b) {
@@ -140,7 +229,7 @@ __device__ __forceinline__ void zplane_run(int w0, int total, Rec rec, Same same
         for (int s = 0; s < SI; ++s) {
             const Item q = item(s);
             const int pk = min(q.p, zp.nplanes - 1 - k * zp.pp);
-            const uint32_t o = (uint32_t)((pk * nym + min(q.j + b * BR, nym - 1)) * N + q.i1) * (uint32_t)sizeof(C);
+            const uint32_t o = (uint32_t)((pk * nym + min(q.j + b * kStep, nrow - 1)) * N + q.i1) * (uint32_t)sizeof(C);
 #pragma unroll
             for (int i2 = 0; i2 < N2; ++i2)
                 x[b][s * N2 + i2] = gld<C>(reinterpret_cast<const Glob<C>*>(base + o) + N1 * i2);
@@ -164,7 +253,13 @@ __device__ __forceinline__ void zplane_run(int w0, int total, Rec rec, Same same
 #pragma unroll
         for (int b = 0; b < NB; ++b) load_rows(blk, b);
         for (int e = threadIdx.x; e < N; e += blockDim.x) twl[e] = gld<C>(gptr(zp.tw2) + e);
-        for (int e = threadIdx.x; e < nch * L; e += blockDim.x) {
+        if constexpr (NCHY != 0) {
+            for (int e = threadIdx.x; e < NCHY * L; e += blockDim.x) {
+                dls[e] = gptr(zy->kyy)[e];
+                twy[e] = gld<C>(gptr(zy->twy2) + e);
+            }
+        }
+        for (int e = threadIdx.x; e < (NCHY ? 0 : nch * L); e += blockDim.x) {
             dls[e] = e > 0 && e < nym ? gptr(zp.dl)[e - 1] : 0.0;
             dus[e] = e < nym - 1 ? gptr(zp.du)[e] : 0.0;
         }
@@ -182,7 +277,7 @@ __device__ __forceinline__ void zplane_run(int w0, int total, Rec rec, Same same
 #pragma unroll
                 for (int i2 = 0; i2 < N2; ++i2) w[i2] = x[b][s * N2 + i2];
                 if constexpr (N2 > 1) dft_reg<-1, N2>(w);
-                if (q.j + b * BR >= nym) {  // rows past the plane
+                if (!NCHY && q.j + b * BR >= nym) {  // rows past the plane
 #pragma unroll
                     for (int i2 = 0; i2 < N2; ++i2) w[i2] = CplxT<C>::make((Rl)0, (Rl)0);
                 }
@@ -191,7 +286,7 @@ __device__ __forceinline__ void zplane_run(int w0, int total, Rec rec, Same same
                 for (int k2 = 1; k2 < N2; ++k2) A[zsw<N1, N2>(v, i1, k2)] = twiddle<-1>(w[k2], twl[i1 * k2]);
             }
         }
-        if (b == NB - 1) load_pivots(blk);  // in flight over the last second step
+        if (!NCHY && b == NB - 1) load_pivots(blk);  // in flight over the last second step
         __syncthreads();
         if constexpr (kLane) {
 #pragma unroll
@@ -226,8 +321,19 @@ __device__ __forceinline__ void zplane_run(int w0, int total, Rec rec, Same same
         __syncthreads();
     }
 
+    if constexpr (NCHY != 0) {
+        const int pk = min(b0 + tp, zp.nplanes - 1), kx = pk / R, kz = R * m + pk - kx * R;
+        C f[L];
+#pragma unroll
+        for (int r = 0; r < L; ++r) f[r] = x[r / BR][r % BR];
+        periodic_ysolve<NCHY, L, N>(f, reinterpret_cast<double*>(smem_raw), twy, dls, gptr(zy->kxx)[kx] + gptr(zy->kzz)[kz],
+                                    zy->inv_ny, kx == 0 && kz == 0, c, m, tp * NCHY * L * N, act);
+#pragma unroll
+        for (int r = 0; r < L; ++r) x[r / BR][r % BR] = f[r];
+    } else {
     chunk_ysolve<L, C>([&](int r) -> C& { return x[r / BR][r % BR]; }, pl, plm, dls, dus, nym, j0, c, nch, N, t, S, act,
                        zp.zero00 && b0 + tp == 0 && m == 0, reinterpret_cast<double2*>(smem_raw));
+    }
 
     const int wn = w + gridDim.x;
     loaded = wn < total && same(wn);
@@ -283,9 +389,9 @@ __device__ __forceinline__ void zplane_run(int w0, int total, Rec rec, Same same
 #pragma unroll
                 for (int k2 = 0; k2 < N2; ++k2) w[k2] = A[zsw<N1, N2>(v, i1, k2)];
                 if constexpr (N2 > 1) dft_reg<1, N2>(w);
-                if (q.j + b * BR < nym && b0 + q.p < zp.nplanes) {
+                if (q.j + b * kStep < nrow && b0 + q.p < zp.nplanes) {
                     const auto base = reinterpret_cast<Glob<char>*>(gptr(zp.spec) + b0 * plane);
-                    const uint32_t o = (uint32_t)((q.p * nym + q.j + b * BR) * N + i1) * (uint32_t)sizeof(C);
+                    const uint32_t o = (uint32_t)((q.p * nym + q.j + b * kStep) * N + i1) * (uint32_t)sizeof(C);
                     const auto dst = reinterpret_cast<Glob<C>*>(base + o);
 #pragma unroll
                     for (int i2 = 0; i2 < N2; ++i2) gst<C>(dst + N1 * i2, w[i2]);
@@ -300,13 +406,13 @@ __device__ __forceinline__ void zplane_run(int w0, int total, Rec rec, Same same
 template <typename C, int N1, int N2, int BR, int NB>
 __global__ void __launch_bounds__(zplane_threads(N1 * N2, NB)) k_zplane(ZPar<C> zp) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    zplane_run<C, N1, N2, BR, NB>(
+    zplane_run<C, N1, N2, BR, NB, 0>(
         xcd_remap(blockIdx.x, gridDim.x), zp.nblocks,
         [&](int w, int& blk) -> const ZPar<C>& {
             blk = w;
             return zp;
         },
-        [](int) { return true; }, smem_raw);
+        [](int) { return true; }, nullptr, smem_raw);
 }
 
 template <typename C, int N1, int N2, int BR, int NB>
@@ -316,7 +422,7 @@ kb_zplane(const ZPar<C>* __restrict__ cs, const int* __restrict__ off, const int
     extern __shared__ __align__(16) unsigned char smem_raw[];
     const int nc = *pnc;
     int at = -1;  // case of the item in hand
-    zplane_run<C, N1, N2, BR, NB>(
+    zplane_run<C, N1, N2, BR, NB, 0>(
         xcd_remap(blockIdx.x, gridDim.x), off[nc],
         [&](int w, int& blk) -> const ZPar<C>& {
             int lo = 0, hi = nc;
@@ -329,7 +435,23 @@ kb_zplane(const ZPar<C>* __restrict__ cs, const int* __restrict__ off, const int
             blk = w - off[lo];
             return cs[idx[lo]];
         },
-        [&](int w) { return w < off[at + 1]; }, smem_raw);
+        [&](int w) { return w < off[at + 1]; }, nullptr, smem_raw);
+}
+
+// periodic y: rows of N1*N2 modes, nyp = NCHY * 8 NB rows.  Up to 512 threads:
+// the transforms of 16 values and their twiddles take about 200 registers
+// (held to 128, for 1024 threads, they spill 350 bytes a lane).
+constexpr int kZpyThreads = 512;
+template <int N1, int N2, int NB, int NCHY>
+__global__ void __launch_bounds__(kZpyThreads) k_zplane_py(ZyPar<double2> zy) {
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    zplane_run<double2, N1, N2, 8, NB, NCHY>(
+        xcd_remap(blockIdx.x, gridDim.x), zy.z.nblocks,
+        [&](int w, int& blk) -> const ZPar<double2>& {
+            blk = w;
+            return zy.z;
+        },
+        [](int) { return true; }, &zy, smem_raw);
 }
 
 template <typename C, int N1, int N2, int BR>
