@@ -312,6 +312,13 @@ constexpr int zplane_threads(int n, int nb) {
     if (nb == 1) return 384;
     return n == 18 || n == 27 || n == 36 || n == 54 || n == 81 || n == 96 || n == 108 || n == 128 ? 512 : 768;
 }
+// rows whose second exchange stays within a wave (16, 32, 64 modes), and the LDS slots per N2 elements of a row
+__host__ __device__ constexpr bool zplane_lane(int n1, int n2, int br) { return br == 8 && n2 == 8 && 64 % (n1 * n2) == 0; }
+__host__ __device__ constexpr int zplane_pad(int n1, int n2, int br) { return zplane_lane(n1, n2, br) ? n2 + 1 : n2; }
+// LDS slots of br rows per chunk for t threads; with the lane exchange those of whole waves
+__host__ __device__ constexpr size_t zplane_slots(int n1, int n2, int br, int t) {
+    return (size_t)(zplane_lane(n1, n2, br) ? (t + 63) / 64 * 64 : t) * br / n2 * zplane_pad(n1, n2, br);
+}
 // passes, chunks and factors of the register-plane kernel for rows of n modes; false if a plane does not fit
 bool zplane_shape(int n, int nym, bool f32, size_t lds_limit, int& nb, int& nch, int& n1, int& n2, int& br);
 template <typename C>
@@ -479,6 +486,16 @@ __host__ __device__ __forceinline__ int lu_pos(int kz, int R, int nz2) {
 // same halo rows, pivot rows or cache lines) then share an L2.  A bijection
 // on [0, n) for every n; only locality, never correctness, depends on the
 // dispatch order.
+// case of work item w: the last c with off[c] <= w (off[0] = 0, off[nc] =
+// total, w < total).  Every lane of the wave must call it: 64 offsets are
+// read at once, where a bisection waits for log2(nc) loads in turn.
+__device__ __forceinline__ int find_case(const int* __restrict__ off, int nc, int w) {
+    const int lane = threadIdx.x & 63;
+    int c = -1;
+    for (int b = 0; b < nc; b += 64) c += __popcll(__ballot(off[min(b + lane, nc)] <= w && b + lane < nc));
+    return __builtin_amdgcn_readfirstlane(c);
+}
+
 constexpr int kXcds = 8;
 __device__ __forceinline__ int xcd_remap(int w, int n) {
     const int q = n / kXcds, r = n - q * kXcds;

@@ -416,8 +416,8 @@ k_duct_ychunk(double2* __restrict__ S, const double* __restrict__ lu, Ops o, int
         dus[e] = e < nym - 1 ? gptr(o.du)[e] : 0.0;
     }
     __syncthreads();
-    chunk_ysolve<L, double2>([&](int r) -> double2& { return x[r]; }, pl, plm, dls, dus, nym, j0, c, nch, G, t, T, act,
-                             false, ends);
+    chunk_ysolve<L, double2>([&](int r) -> double2& { return x[r]; }, pl, plm, dls, dus, nym, j0, c, nch, G, t, act,
+                             false, FlatEnds{ends, T});
     if (act && m < nzp) {
 #pragma unroll
         for (int r = 0; r < L; ++r)

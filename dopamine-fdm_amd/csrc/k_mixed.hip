@@ -197,12 +197,7 @@ __global__ void __launch_bounds__(256) kb_save_p(const SPar* __restrict__ cs, co
     const int nc = *pnc;
     const int total = off[nc];
     for (int w = blockIdx.x; w < total; w += gridDim.x) {
-        int lo = 0, hi = nc;
-        while (hi - lo > 1) {
-            const int mid = (lo + hi) >> 1;
-            if (off[mid] <= w) lo = mid;
-            else hi = mid;
-        }
+        const int lo = find_case(off, nc, w);
         save_p_body(cs[idx[lo]], w - off[lo]);
     }
 }

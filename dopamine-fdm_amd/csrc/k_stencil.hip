@@ -187,12 +187,7 @@ __global__ void __launch_bounds__(256) kb_correct(const CPar* __restrict__ cs, c
     for (int base = 0; base < total; base += gridDim.x) {
         const int w = base + me;
         if (w >= total) break;
-        int lo = 0, hi = nc;
-        while (hi - lo > 1) {
-            const int mid = (lo + hi) >> 1;
-            if (off[mid] <= w) lo = mid;
-            else hi = mid;
-        }
+        const int lo = find_case(off, nc, w);
         const CPar& c = cs[idx[lo]];
         const int li = w - off[lo];
         const int bz = li / c.nbx;

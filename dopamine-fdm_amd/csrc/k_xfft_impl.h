@@ -234,17 +234,6 @@ __global__ void __launch_bounds__(kXThreads) k_div_rfft_x(XPar<C> q) {
     xfwd_body<MODE, C, R, KX>(q, bx, j, smem_raw);
 }
 
-// case of work item w: the last c with off[c] <= w (off[0] = 0, off[nc] = total)
-__device__ __forceinline__ int xfind_case(const int* __restrict__ off, int nc, int w) {
-    int lo = 0, hi = nc;
-    while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (off[mid] <= w) lo = mid;
-        else hi = mid;
-    }
-    return lo;
-}
-
 // KX butterfly slots per thread (4: FP32 tiles too large for two);
 // with two, at most four waves per SIMD (128 VGPRs): two workgroups per CU
 template <int MODE, typename C, int R, int KX>
@@ -258,7 +247,7 @@ kb_div_rfft_x(const XPar<C>* __restrict__ cs, const int* __restrict__ off, const
     for (int base = 0; base < total; base += gridDim.x) {
         const int w = base + me;
         if (w >= total) break;
-        const int c = xfind_case(off, nc, w);
+        const int c = find_case(off, nc, w);
         const XPar<C>& q = cs[idx[c]];
         int bx, j;
         xtile(w - off[c], q.nbx, q.g.nym, q.strip, bx, j);
@@ -452,7 +441,7 @@ __global__ void __launch_bounds__(kXThreads) kb_irfft_x(const XPar<C>* __restric
     for (int base = 0; base < total; base += gridDim.x) {
         const int w = base + me;
         if (w >= total) break;
-        const int c = xfind_case(off, nc, w);
+        const int c = find_case(off, nc, w);
         const XPar<C>& q = cs[idx[c]];
         int bx, j;
         xtile(w - off[c], q.nbx, q.g.nym, q.strip, bx, j);

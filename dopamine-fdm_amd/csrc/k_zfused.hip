@@ -203,12 +203,7 @@ __global__ void __launch_bounds__(kZfThreads) kb_zfused(const ZPar<C>* __restric
     for (int base = 0; base < total; base += gridDim.x) {
         const int w = base + me;
         if (w >= total) break;
-        int lo = 0, hi = nc;
-        while (hi - lo > 1) {
-            const int mid = (lo + hi) >> 1;
-            if (off[mid] <= w) lo = mid;
-            else hi = mid;
-        }
+        const int lo = find_case(off, nc, w);
         zfused_body<C>(cs[idx[lo]], w - off[lo], smem_raw);
         __syncthreads();
     }

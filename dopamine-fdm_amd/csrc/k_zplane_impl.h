@@ -17,6 +17,13 @@
 //   y solve in chunks (ychunk.h), with the plan's inverse pivots in registers;
 //   inverse z transform: the same steps backwards, stored from registers.
 //
+// Bound by HBM for the rows' loads and stores, in which all workgroups are at
+// first in step, with the transforms and the solve between (9 us a plane of
+// 192 x 64 modes, 12 with its stores; 129 x 4 such planes on 256 CUs leave a
+// third round of four).  With the exchanges free of barriers and of address
+// arithmetic (kLane below): 256x192x256 73 -> 64 us, inflow (1024 planes)
+// 100 -> 88 us = 4.6 TB/s, periodic y 256x257x256 105 -> 96 us.
+//
 // All of a plane's loads are in flight at once and no wave waits for another's
 // sweep: the serial part is 4 L + 2 nch steps instead of 2 nym.  The working
 // set (L complex values and L pivots per thread) is what limits it: planes
@@ -154,6 +161,37 @@ __device__ __forceinline__ void periodic_ysolve(double2 (&x)[L], double* ex, con
     dft_reg<1, L>(x);
 }
 
+// What the z kernel reads of a case record, uniform over the workgroup.
+template <typename C>
+struct ZRec {
+    C* spec;
+    const double* lu;
+    const double* dl;
+    const double* du;
+    const C* tw2;
+    int nym, nzp, R, zero00, nplanes, nch, pp;
+};
+template <typename C>
+__device__ __forceinline__ ZRec<C> zrec_of(const ZPar<C>& z) {
+    return ZRec<C>{z.spec, z.lu, z.dl, z.du, z.tw2, z.nym, z.nzp, z.R, z.zero00, z.nplanes, z.nch, z.pp};
+}
+// the same from a record in memory, held in scalar registers
+template <typename T>
+__device__ __forceinline__ T* first_lane(T* p) {
+    const uint64_t v = reinterpret_cast<uint64_t>(p);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
+    return reinterpret_cast<T*>((uint64_t)hi << 32 | lo);
+}
+__device__ __forceinline__ int first_lane(int v) { return __builtin_amdgcn_readfirstlane(v); }
+template <typename C>
+__device__ __forceinline__ ZRec<C> zrec_uniform(const ZPar<C>& z) {
+    const ZRec<C> r = zrec_of(z);
+    return ZRec<C>{first_lane(r.spec), first_lane(r.lu),      first_lane(r.dl),  first_lane(r.du),
+                   first_lane(r.tw2),  first_lane(r.nym),     first_lane(r.nzp), first_lane(r.R),
+                   first_lane(r.zero00), first_lane(r.nplanes), first_lane(r.nch), first_lane(r.pp)};
+}
+
 // Runs the workgroup's items: rec(w, blk) gives the case record of item w and
 // its block there, same(w) whether the next item w has the record of the last
 // one.  An item's rows load into the registers that the item before frees,
@@ -172,13 +210,32 @@ __device__ __forceinline__ void zplane_run(int w0, int total, Rec rec, Same same
     // eight rows of NC whole chunks in both layouts (lane (row, k2), register
     // (chunk, k1); lane (chunk, mode), register row), so the second exchange
     // stays within the wave and out of LDS
-    constexpr bool kLane = BR == 8 && N2 == 8 && 64 % N == 0;
+    constexpr bool kLane = zplane_lane(N1, N2, BR);
     constexpr int NC = kLane ? 64 / N : 1;
+    // LDS position of element (i1, k2) of local row v: with the lane exchange
+    // the eight k2 of an i1 take nine slots, which puts the 8 (FP64) lanes of
+    // an LDS cycle in distinct banks in both steps and leaves every access of a
+    // thread at a constant distance from its first (instruction offsets, no
+    // address arithmetic); else the rotated layout, which needs no room
+    constexpr int kPad = zplane_pad(N1, N2, BR);
+    // and a wave's first-step items are those same rows (BR/N2 = 1 item a thread): both exchanges are the wave's own,
+    // in its own slots, and take no workgroup barrier, so the waves run apart and one's arithmetic covers another's
+    // LDS and HBM accesses
+    auto exchange = [] {
+        if constexpr (kLane) {
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        } else {
+            __syncthreads();
+        }
+    };
+    auto pos = [](int v, int i1, int k2) { return kLane ? (v * N1 + i1) * kPad + k2 : zsw<N1, N2>(v, i1, k2); };
     C x[NB][BR];
     bool loaded = false;
     for (int w = w0; w < total; w += gridDim.x) {
     int blk;
-    const ZPar<C>& zp = rec(w, blk);
+    const ZRec<C> zp = rec(w, blk);
     const int nym = zp.nym, R = zp.R, nch = NCHY ? NCHY : zp.nch;
     const int nrow = NCHY ? nym - 1 : nym;           // rows transformed
     constexpr int kStep = NCHY ? NCHY * BR : BR;     // rows from one pass to the next
@@ -190,10 +247,11 @@ __device__ __forceinline__ void zplane_run(int w0, int total, Rec rec, Same same
     const bool act = tid < S;
     const int t = min(tid, S - 1);
     C* A = reinterpret_cast<C*>(smem_raw);  // S * BR values: BR rows of every chunk and plane
-    double* dls = reinterpret_cast<double*>(A + (size_t)S * BR);  // DL(j-1), nch*L
-    double* dus = dls + nch * L;                                  // DU(j), nch*L
-    C* twl = reinterpret_cast<C*>(dus + nch * L);                 // w_n^e, N
-    C* twy = twl + N;                                             // periodic y: w_nyp^e (and kyy in dls)
+    double* dls = reinterpret_cast<double*>(A + zplane_slots(N1, N2, BR, S));  // DL(j-1), nch*L
+    double* dus = dls + nch * L;                                               // DU(j), nch*L
+    C* twl = reinterpret_cast<C*>(dus + nch * L);  // w_n^(i1 k2) at i1*kPad + k2 (lane exchange), or w_n^e, N
+    C* twy = twl + N1 * kPad;                      // periodic y: w_nyp^e (and kyy in dls)
+    auto twz = [&](int i1, int k2) { return kLane ? twl[i1 * kPad + k2] : twl[i1 * k2]; };
     // HBM accesses are a uniform base and a 32-bit byte offset per thread (one register per address): the
     // workgroup's planes and pivot rows span well under 4 GiB
     const int b0 = blk * zp.pp;
@@ -208,28 +266,32 @@ __device__ __forceinline__ void zplane_run(int w0, int total, Rec rec, Same same
     // second-step items of the lane exchange: rows v0 + 8 cb, cb < NC
     const int v0 = (tid >> 6) * (NC * 8) + ((tid >> 3) & 7), vend = S / N * BR;
 
-    // its transform items: item s covers local row v (plane p, row j of pass 0), elements i1 + N1 i2;
-    // formed anew at each use (opaque to the compiler) rather than held over the solve
+    // its transform items: item s covers elements i1 + N1 i2 of local row v, which is row `row` of pass 0, counted over
+    // the workgroup's planes (`end`: its plane's last); formed anew at each use (opaque to the
+    // compiler) rather than held over the solve
     struct Item {
-        int v, i1, p, j;
+        int v, i1, row, end;
     };
     auto item = [&](int s) {
         int tt = t;
         asm volatile("" : "+v"(tt));
         const int it = tt + s * S;
         const int v = it / N1;
-        const int vc = v / BR, p = vc / nch;
+        const int vc = v / BR;
+        int p = 0;
+        if (zp.pp > 1) p = vc / nch;
         const int cc = vc - p * nch, q = v - vc * BR;
-        return Item{v, it - v * N1, p, NCHY ? cc + NCHY * q : cc * L + q};
+        return Item{v, it - v * N1, p * nym + (NCHY ? cc + NCHY * q : cc * L + q), p * nym + nrow - 1};
     };
-    // rows of pass b of block k (a partial last workgroup repeats its last plane, unstored)
+    // rows of pass b of block k (a partial last workgroup loads rows of its last plane again, unstored)
     auto load_rows = [&](int k, int b) {
         const auto base = reinterpret_cast<const Glob<char>*>(gptr(zp.spec) + (long)k * zp.pp * plane);
+        const int last = (zp.nplanes - k * zp.pp) * nym - 1;
 #pragma unroll
         for (int s = 0; s < SI; ++s) {
             const Item q = item(s);
-            const int pk = min(q.p, zp.nplanes - 1 - k * zp.pp);
-            const uint32_t o = (uint32_t)((pk * nym + min(q.j + b * kStep, nrow - 1)) * N + q.i1) * (uint32_t)sizeof(C);
+            const int row = min(min(q.row + b * kStep, q.end), last);
+            const uint32_t o = (uint32_t)(row * N + q.i1) * (uint32_t)sizeof(C);
 #pragma unroll
             for (int i2 = 0; i2 < N2; ++i2)
                 x[b][s * N2 + i2] = gld<C>(reinterpret_cast<const Glob<C>*>(base + o) + N1 * i2);
@@ -239,20 +301,30 @@ __device__ __forceinline__ void zplane_run(int w0, int total, Rec rec, Same same
     auto load_pivots = [&](int k) {
         const int kx0 = k * zp.pp / R;
         const auto base = reinterpret_cast<const Glob<char>*>(gptr(zp.lu) + (long)kx0 * nym * nzs);
-        const int pk = min(k * zp.pp + tp, zp.nplanes - 1), kx = pk / R, u = pk - kx * R;
-        const uint32_t o = (uint32_t)((kx - kx0) * nym * nzs + lu_pos_mu(m, u, R, N));
-        auto at = [&](int j) {
-            return *reinterpret_cast<const Glob<double>*>(base + (o + (uint32_t)(j * nzs)) * (uint32_t)sizeof(double));
-        };
-        plm = at(max(j0 - 1, 0));
+        int dk = 0, u = k * zp.pp - kx0 * R;
+        if (zp.pp > 1) {
+            const int pk = min(k * zp.pp + tp, zp.nplanes - 1), kx = pk / R;
+            dk = kx - kx0;
+            u = pk - kx * R;
+        }
+        const uint32_t step = (uint32_t)nzs * (uint32_t)sizeof(double);
+        uint32_t o = (uint32_t)((dk * nym + j0) * nzs + lu_pos_mu(m, u, R, N)) * (uint32_t)sizeof(double);
+        const uint32_t end = o + (uint32_t)(nym - 1 - j0) * step;  // the plane's last row
+        auto at = [&](uint32_t e) { return *reinterpret_cast<const Glob<double>*>(base + e); };
+        plm = at(j0 > 0 ? o - step : o);
 #pragma unroll
-        for (int r = 0; r < L; ++r) pl[r] = at(min(j0 + r, nym - 1));
+        for (int r = 0; r < L; ++r) {
+            pl[r] = at(min(o, end));
+            o += step;
+        }
     };
-    __syncthreads();  // the last item has read its tables and rows
+    if (!kLane || !loaded) __syncthreads();  // the last item has read its tables and rows
     if (!loaded) {
-#pragma unroll
-        for (int b = 0; b < NB; ++b) load_rows(blk, b);
-        for (int e = threadIdx.x; e < N; e += blockDim.x) twl[e] = gld<C>(gptr(zp.tw2) + e);
+        // tables first: their waits leave the rows' loads in flight
+        for (int e = threadIdx.x; e < N; e += blockDim.x) {
+            const int i1 = e / N2, k2 = e - i1 * N2;
+            twl[kLane ? i1 * kPad + k2 : e] = gld<C>(gptr(zp.tw2) + (kLane ? i1 * k2 : e));
+        }
         if constexpr (NCHY != 0) {
             for (int e = threadIdx.x; e < NCHY * L; e += blockDim.x) {
                 dls[e] = gptr(zy->kyy)[e];
@@ -263,6 +335,8 @@ __device__ __forceinline__ void zplane_run(int w0, int total, Rec rec, Same same
             dls[e] = e > 0 && e < nym ? gptr(zp.dl)[e - 1] : 0.0;
             dus[e] = e < nym - 1 ? gptr(zp.du)[e] : 0.0;
         }
+#pragma unroll
+        for (int b = 0; b < NB; ++b) load_rows(blk, b);
         __syncthreads();
     }
 
@@ -277,24 +351,24 @@ __device__ __forceinline__ void zplane_run(int w0, int total, Rec rec, Same same
 #pragma unroll
                 for (int i2 = 0; i2 < N2; ++i2) w[i2] = x[b][s * N2 + i2];
                 if constexpr (N2 > 1) dft_reg<-1, N2>(w);
-                if (!NCHY && q.j + b * BR >= nym) {  // rows past the plane
+                if (!NCHY && q.row + b * BR > q.end) {  // rows past the plane
 #pragma unroll
                     for (int i2 = 0; i2 < N2; ++i2) w[i2] = CplxT<C>::make((Rl)0, (Rl)0);
                 }
-                A[zsw<N1, N2>(v, i1, 0)] = w[0];
+                A[pos(v, i1, 0)] = w[0];
 #pragma unroll
-                for (int k2 = 1; k2 < N2; ++k2) A[zsw<N1, N2>(v, i1, k2)] = twiddle<-1>(w[k2], twl[i1 * k2]);
+                for (int k2 = 1; k2 < N2; ++k2) A[pos(v, i1, k2)] = twiddle<-1>(w[k2], twz(i1, k2));
             }
         }
         if (!NCHY && b == NB - 1) load_pivots(blk);  // in flight over the last second step
-        __syncthreads();
+        exchange();
         if constexpr (kLane) {
 #pragma unroll
             for (int cb = 0; cb < NC; ++cb) {
                 const int v = min(v0 + 8 * cb, vend - 1), k2 = tid & 7;
                 C w[N1];
 #pragma unroll
-                for (int i1 = 0; i1 < N1; ++i1) w[i1] = A[zsw<N1, N2>(v, i1, k2)];
+                for (int i1 = 0; i1 < N1; ++i1) w[i1] = A[pos(v, i1, k2)];
                 dft_reg<-1, N1>(w);
 #pragma unroll
                 for (int k1 = 0; k1 < N1; ++k1) x[b][cb * N1 + k1] = w[k1];
@@ -308,20 +382,21 @@ __device__ __forceinline__ void zplane_run(int w0, int total, Rec rec, Same same
                     const int v = it / N2, k2 = it - v * N2;
                     C w[N1];
 #pragma unroll
-                    for (int i1 = 0; i1 < N1; ++i1) w[i1] = A[zsw<N1, N2>(v, i1, k2)];
+                    for (int i1 = 0; i1 < N1; ++i1) w[i1] = A[pos(v, i1, k2)];
                     dft_reg<-1, N1>(w);
 #pragma unroll
-                    for (int k1 = 0; k1 < N1; ++k1) A[zsw<N1, N2>(v, k1, k2)] = w[k1];
+                    for (int k1 = 0; k1 < N1; ++k1) A[pos(v, k1, k2)] = w[k1];
                 }
             }
-            __syncthreads();
+            exchange();
 #pragma unroll
-            for (int q = 0; q < BR; ++q) x[b][q] = A[zsw<N1, N2>(vrow + q, m / N2, m % N2)];
+            for (int q = 0; q < BR; ++q) x[b][q] = A[pos(vrow + q, m / N2, m % N2)];
         }
-        __syncthreads();
+        exchange();
     }
 
     if constexpr (NCHY != 0) {
+        if constexpr (kLane) __syncthreads();  // every wave's rows have left the slots that the columns exchange through
         const int pk = min(b0 + tp, zp.nplanes - 1), kx = pk / R, kz = R * m + pk - kx * R;
         C f[L];
 #pragma unroll
@@ -331,8 +406,12 @@ __device__ __forceinline__ void zplane_run(int w0, int total, Rec rec, Same same
 #pragma unroll
         for (int r = 0; r < L; ++r) x[r / BR][r % BR] = f[r];
     } else {
-    chunk_ysolve<L, C>([&](int r) -> C& { return x[r / BR][r % BR]; }, pl, plm, dls, dus, nym, j0, c, nch, N, t, S, act,
-                       zp.zero00 && b0 + tp == 0 && m == 0, reinterpret_cast<double2*>(smem_raw));
+    auto solve = [&](auto ends) {
+        chunk_ysolve<L, C>([&](int r) -> C& { return x[r / BR][r % BR]; }, pl, plm, dls, dus, nym, j0, c, nch, N, t,
+                           act, zp.zero00 && b0 + tp == 0 && m == 0, ends);
+    };
+    if constexpr (kLane) solve(WaveEnds<64 * kPad * (int)sizeof(C)>{smem_raw});
+    else solve(FlatEnds{reinterpret_cast<double2*>(smem_raw), S});
     }
 
     const int wn = w + gridDim.x;
@@ -351,19 +430,19 @@ __device__ __forceinline__ void zplane_run(int w0, int total, Rec rec, Same same
                 for (int k1 = 0; k1 < N1; ++k1) w[k1] = x[b][cb * N1 + k1];
                 dft_reg<1, N1>(w);
                 if (v < vend) {
-                    A[zsw<N1, N2>(v, 0, k2)] = w[0];
+                    A[pos(v, 0, k2)] = w[0];
 #pragma unroll
-                    for (int i1 = 1; i1 < N1; ++i1) A[zsw<N1, N2>(v, i1, k2)] = twiddle<1>(w[i1], twl[i1 * k2]);
+                    for (int i1 = 1; i1 < N1; ++i1) A[pos(v, i1, k2)] = twiddle<1>(w[i1], twz(i1, k2));
                 }
             }
             if (loaded) load_rows(kn, b);
         } else {
             if (act) {
 #pragma unroll
-                for (int q = 0; q < BR; ++q) A[zsw<N1, N2>(vrow + q, m / N2, m % N2)] = x[b][q];
+                for (int q = 0; q < BR; ++q) A[pos(vrow + q, m / N2, m % N2)] = x[b][q];
             }
             if (loaded) load_rows(kn, b);
-            __syncthreads();
+            exchange();
             if (act) {
                 const int items = S * BR / N1;
 #pragma unroll 1
@@ -371,15 +450,15 @@ __device__ __forceinline__ void zplane_run(int w0, int total, Rec rec, Same same
                     const int v = it / N2, k2 = it - v * N2;
                     C w[N1];
 #pragma unroll
-                    for (int k1 = 0; k1 < N1; ++k1) w[k1] = A[zsw<N1, N2>(v, k1, k2)];
+                    for (int k1 = 0; k1 < N1; ++k1) w[k1] = A[pos(v, k1, k2)];
                     dft_reg<1, N1>(w);
-                    A[zsw<N1, N2>(v, 0, k2)] = w[0];
+                    A[pos(v, 0, k2)] = w[0];
 #pragma unroll
-                    for (int i1 = 1; i1 < N1; ++i1) A[zsw<N1, N2>(v, i1, k2)] = twiddle<1>(w[i1], twl[i1 * k2]);
+                    for (int i1 = 1; i1 < N1; ++i1) A[pos(v, i1, k2)] = twiddle<1>(w[i1], twz(i1, k2));
                 }
             }
         }
-        __syncthreads();
+        exchange();
         if (act) {
 #pragma unroll
             for (int s = 0; s < SI; ++s) {
@@ -387,18 +466,19 @@ __device__ __forceinline__ void zplane_run(int w0, int total, Rec rec, Same same
                 const int v = q.v, i1 = q.i1;
                 C w[N2];
 #pragma unroll
-                for (int k2 = 0; k2 < N2; ++k2) w[k2] = A[zsw<N1, N2>(v, i1, k2)];
+                for (int k2 = 0; k2 < N2; ++k2) w[k2] = A[pos(v, i1, k2)];
                 if constexpr (N2 > 1) dft_reg<1, N2>(w);
-                if (q.j + b * kStep < nrow && b0 + q.p < zp.nplanes) {
+                const int row = q.row + b * kStep;
+                if (row <= q.end && row < (zp.nplanes - b0) * nym) {
                     const auto base = reinterpret_cast<Glob<char>*>(gptr(zp.spec) + b0 * plane);
-                    const uint32_t o = (uint32_t)((q.p * nym + q.j + b * kStep) * N + i1) * (uint32_t)sizeof(C);
+                    const uint32_t o = (uint32_t)(row * N + i1) * (uint32_t)sizeof(C);
                     const auto dst = reinterpret_cast<Glob<C>*>(base + o);
 #pragma unroll
                     for (int i2 = 0; i2 < N2; ++i2) gst<C>(dst + N1 * i2, w[i2]);
                 }
             }
         }
-        if (b + 1 < NB) __syncthreads();
+        if (b + 1 < NB) exchange();
     }
     }
 }
@@ -408,9 +488,9 @@ __global__ void __launch_bounds__(zplane_threads(N1 * N2, NB)) k_zplane(ZPar<C> 
     extern __shared__ __align__(16) unsigned char smem_raw[];
     zplane_run<C, N1, N2, BR, NB, 0>(
         xcd_remap(blockIdx.x, gridDim.x), zp.nblocks,
-        [&](int w, int& blk) -> const ZPar<C>& {
+        [&](int w, int& blk) {
             blk = w;
-            return zp;
+            return zrec_of(zp);
         },
         [](int) { return true; }, nullptr, smem_raw);
 }
@@ -422,18 +502,16 @@ kb_zplane(const ZPar<C>* __restrict__ cs, const int* __restrict__ off, const int
     extern __shared__ __align__(16) unsigned char smem_raw[];
     const int nc = *pnc;
     int at = -1;  // case of the item in hand
+    ZRec<C> r;
     zplane_run<C, N1, N2, BR, NB, 0>(
         xcd_remap(blockIdx.x, gridDim.x), off[nc],
-        [&](int w, int& blk) -> const ZPar<C>& {
-            int lo = 0, hi = nc;
-            while (hi - lo > 1) {
-                const int mid = (lo + hi) >> 1;
-                if (off[mid] <= w) lo = mid;
-                else hi = mid;
+        [&](int w, int& blk) {
+            if (at < 0 || w >= off[at + 1]) {
+                at = find_case(off, nc, w);
+                r = zrec_uniform(cs[idx[at]]);
             }
-            at = lo;
-            blk = w - off[lo];
-            return cs[idx[lo]];
+            blk = w - off[at];
+            return r;
         },
         [&](int w) { return w < off[at + 1]; }, nullptr, smem_raw);
 }
@@ -447,9 +525,9 @@ __global__ void __launch_bounds__(kZpyThreads) k_zplane_py(ZyPar<double2> zy) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     zplane_run<double2, N1, N2, 8, NB, NCHY>(
         xcd_remap(blockIdx.x, gridDim.x), zy.z.nblocks,
-        [&](int w, int& blk) -> const ZPar<double2>& {
+        [&](int w, int& blk) {
             blk = w;
-            return zy.z;
+            return zrec_of(zy.z);
         },
         [](int) { return true; }, &zy, smem_raw);
 }

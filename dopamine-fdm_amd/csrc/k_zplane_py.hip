@@ -34,7 +34,12 @@ bool zplane_py_shape(int n, int nyp, size_t lds_limit, int& nb, int& nch) {
 
 // rows of eight per chunk for every thread, kyy (twice, as the wall solve's two tables), w_n, w_nyp
 size_t zplane_py_lds(int threads, int n, int nyp) {
-    return sizeof(double2) * ((size_t)threads * 8 + n + nyp) + 2 * sizeof(double) * (size_t)nyp;
+    size_t slots = 0;
+#define DFP_ZPY_PAD(a, b, ...) \
+    if (a * b == n) slots = zplane_slots(a, b, 8, threads) + a * zplane_pad(a, b, 8);
+    DFP_ZPY_ROWS(DFP_ZPY_PAD, )
+#undef DFP_ZPY_PAD
+    return sizeof(double2) * (slots + nyp) + 2 * sizeof(double) * (size_t)nyp;
 }
 
 hipError_t launch_zplane_py(dfp_plan* p, ZyPar<double2> zy) {

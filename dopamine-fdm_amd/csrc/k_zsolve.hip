@@ -565,16 +565,6 @@ __global__ void __launch_bounds__(kZsThreads) k_zsolve(ZPar<C> zp) {
     }
 }
 
-__device__ __forceinline__ int zfind_case(const int* __restrict__ off, int nc, int w) {
-    int lo = 0, hi = nc;
-    while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (off[mid] <= w) lo = mid;
-        else hi = mid;
-    }
-    return lo;
-}
-
 template <typename C, int N1, int N2>
 __global__ void __launch_bounds__(kZsThreads) kb_zsolve(const ZPar<C>* __restrict__ cs, const int* __restrict__ off,
                                                         const int* __restrict__ idx, const int* __restrict__ pnc) {
@@ -585,7 +575,7 @@ __global__ void __launch_bounds__(kZsThreads) kb_zsolve(const ZPar<C>* __restric
     for (int base = 0; base < total; base += gridDim.x) {
         const int w = base + me;
         if (w >= total) break;
-        const int c = zfind_case(off, nc, w);
+        const int c = find_case(off, nc, w);
         // both halves of the sub-plane, as k_zsolve
         if constexpr (N1 == 0) {
             zfwd_body<C>(cs[idx[c]], w - off[c], smem_raw);
@@ -606,9 +596,10 @@ static int zplane_planes(const dfp_plan* p, int batch) {
     return std::max(1, (batch ? zplane_threads(p->fz.n, p->zp_nb) : 64) / (p->fz.n * p->zp_nch));
 }
 
-static size_t zplane_lds(int threads, int n, int nch, int br, int nb, bool f32) {
+static size_t zplane_lds(int threads, int n1, int n2, int nch, int br, int nb, bool f32) {
     const size_t cs = f32 ? sizeof(float2) : sizeof(double2);
-    return cs * ((size_t)threads * br + n) + 2 * sizeof(double) * (size_t)nch * br * nb;
+    const int pad = zplane_pad(n1, n2, br);
+    return cs * (zplane_slots(n1, n2, br, threads) + n1 * pad) + 2 * sizeof(double) * (size_t)nch * br * nb;
 }
 
 // One pass where the plane fits its narrow workgroup (the most threads, the
@@ -627,7 +618,7 @@ bool zplane_shape(int n, int nym, bool f32, size_t lds_limit, int& nb, int& nch,
         nb = q;
         nch = (int)(threads / n);
         // a batched workgroup holds up to zplane_threads threads of planes
-        return zplane_lds(zplane_threads(n, q), n, nch, br, nb, f32) <= lds_limit;
+        return zplane_lds(zplane_threads(n, q), n1, n2, nch, br, nb, f32) <= lds_limit;
     }
     return false;
 }
@@ -668,7 +659,8 @@ template ZPar<float2> make_zpar<float2>(const dfp_plan*, int, int);
 
 size_t z_lds_bytes(const dfp_plan* p, int f32, int batch) {
     if (p->zp_nb)
-        return zplane_lds(p->fz.n * p->zp_nch * zplane_planes(p, batch), p->fz.n, p->zp_nch, p->zp_br, p->zp_nb, f32);
+        return zplane_lds(p->fz.n * p->zp_nch * zplane_planes(p, batch), p->zp_n1, p->zp_n2, p->zp_nch, p->zp_br, p->zp_nb,
+                          f32);
     const int G = p->g_zs, n = p->fz.n, ntw = p->zn1 ? n : twiddle_count(p->fz);
     const size_t pts = (size_t)G * n * (p->zn1 ? zplanes(n) : 1);
     return (f32 ? sizeof(float2) : sizeof(double2)) * (pts + ntw) + sizeof(double) * (pts + G);

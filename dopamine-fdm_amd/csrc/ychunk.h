@@ -18,23 +18,39 @@ namespace dfp {
 __device__ __forceinline__ void keep_value(float2& v) { asm volatile("" : "+v"(v.x), "+v"(v.y)); }
 __device__ __forceinline__ void keep_value(double2&) {}
 
+// Where the chunks' ends lie in LDS: thread t's end value and multiplier
+// product of the elimination (ce, cp) and of the back substitution (ge, gp).
+struct FlatEnds {  // T threads, 48 T bytes
+    double2* p;
+    int T;
+    __device__ __forceinline__ double2& ce(int t) const { return p[t]; }
+    __device__ __forceinline__ double2& ge(int t) const { return p[T + t]; }
+    __device__ __forceinline__ double& cp(int t) const { return reinterpret_cast<double*>(p + 2 * T)[t]; }
+    __device__ __forceinline__ double& gp(int t) const { return reinterpret_cast<double*>(p + 2 * T)[T + t]; }
+};
+template <int W>
+struct WaveEnds {  // each wave's in its own W bytes (3072 used)
+    unsigned char* p;
+    __device__ __forceinline__ unsigned char* at(int t, int size) const { return p + (t >> 6) * W + (t & 63) * size; }
+    __device__ __forceinline__ double2& ce(int t) const { return *reinterpret_cast<double2*>(at(t, 16)); }
+    __device__ __forceinline__ double2& ge(int t) const { return *reinterpret_cast<double2*>(at(t, 16) + 1024); }
+    __device__ __forceinline__ double& cp(int t) const { return *reinterpret_cast<double*>(at(t, 8) + 2048); }
+    __device__ __forceinline__ double& gp(int t) const { return *reinterpret_cast<double*>(at(t, 8) + 2560); }
+};
+
 // at(r): row j0 + r of this thread's column, r < L (C: double2, or float2,
 // solved in FP64 and rounded where stored); rows past nym hold zero.
 // pl[r] = 1/D'(j0 + r), plm = 1/D'(j0 - 1); dls[j] = DL(j-1), dus[j] = DU(j)
-// for j < nch*L, zero outside the operator.  Thread t of T solving threads
-// (act) owns chunk c of its column; the same column's next chunk is thread
-// t + stride.  ends: LDS for 48 T bytes, free on entry (every thread has
-// passed a barrier since its last other use) and on return.  Every thread of
-// the block must call it.  zero: the column's solution is replaced by zero.
-template <int L, typename C, typename At>
+// for j < nch*L, zero outside the operator.  Thread t (act: one of the
+// solving threads) owns chunk c of its column; the same column's next chunk is
+// thread t + stride.  ends: LDS where thread t may write its own entries on
+// entry, free again on return.  Every thread of the block must call it.
+// zero: the column's solution is replaced by zero.
+template <int L, typename C, typename At, typename Ends>
 __device__ __forceinline__ void chunk_ysolve(At at, double (&pl)[L], double plm, const double* dls, const double* dus,
-                                             int nym, int j0, int c, int nch, int stride, int t, int T, bool act,
-                                             bool zero, double2* ends) {
+                                             int nym, int j0, int c, int nch, int stride, int t, bool act,
+                                             bool zero, const Ends& ends) {
     using Rl = typename CplxT<C>::real;
-    double2* ce = ends;
-    double2* ge = ce + T;
-    double* cp = reinterpret_cast<double*>(ge + T);
-    double* gp = cp + T;
     // elimination.  Rows past nym hold zero, take no multiplier and a zero
     // inverse pivot, so they carry nothing into the back substitution.
     if (j0 == 0) plm = 0.0;
@@ -51,8 +67,8 @@ __device__ __forceinline__ void chunk_ysolve(At at, double (&pl)[L], double plm,
             ip = pl[r];
         }
         if (act) {
-            ce[t] = make_double2(ex, ey);
-            cp[t] = pi;
+            ends.ce(t) = make_double2(ex, ey);
+            ends.cp(t) = pi;
         }
     }
     __syncthreads();
@@ -62,8 +78,8 @@ __device__ __forceinline__ void chunk_ysolve(At at, double (&pl)[L], double plm,
         for (int r = 0; r < L; ++r) keep_value(at(r));
 #pragma unroll 2
         for (int q = 0; q < c; ++q) {
-            const double2 e = ce[t - (c - q) * stride];
-            const double f = cp[t - (c - q) * stride];
+            const double2 e = ends.ce(t - (c - q) * stride);
+            const double f = ends.cp(t - (c - q) * stride);
             bx = e.x + f * bx;
             by = e.y + f * by;
         }
@@ -89,8 +105,8 @@ __device__ __forceinline__ void chunk_ysolve(At at, double (&pl)[L], double plm,
             pi *= -d * pl[r];
         }
         if (act) {
-            ge[t] = make_double2(gx, gy);
-            gp[t] = pi;
+            ends.ge(t) = make_double2(gx, gy);
+            ends.gp(t) = pi;
         }
     }
     __syncthreads();
@@ -100,8 +116,8 @@ __device__ __forceinline__ void chunk_ysolve(At at, double (&pl)[L], double plm,
         for (int r = 0; r < L; ++r) keep_value(at(r));
 #pragma unroll 2
         for (int q = nch - 1; q > c; --q) {
-            const double2 e = ge[t + (q - c) * stride];
-            const double f = gp[t + (q - c) * stride];
+            const double2 e = ends.ge(t + (q - c) * stride);
+            const double f = ends.gp(t + (q - c) * stride);
             xx = e.x + f * xx;
             xy = e.y + f * xy;
         }
@@ -111,7 +127,12 @@ __device__ __forceinline__ void chunk_ysolve(At at, double (&pl)[L], double plm,
             C& v = at(r);
             xx = ((double)v.x - d * xx) * pl[r];
             xy = ((double)v.y - d * xy) * pl[r];
-            v = zero ? CplxT<C>::make((Rl)0, (Rl)0) : CplxT<C>::make((Rl)xx, (Rl)xy);
+            v = CplxT<C>::make((Rl)xx, (Rl)xy);
+        }
+        if (zero) {
+            asm volatile("");  // a branch, not a selection of every value
+#pragma unroll
+            for (int r = 0; r < L; ++r) at(r) = CplxT<C>::make((Rl)0, (Rl)0);
         }
     }
     __syncthreads();
