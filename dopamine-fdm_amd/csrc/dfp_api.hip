@@ -578,6 +578,7 @@ int dfp_plan_create_tuned(const dfp_grid* g, int precision, int device, const df
     p->fz = sh.fz;
     p->tk_x = sh.T;
     p->tk_xi = sh.Ti;
+    p->tuned_columns = tune && tune->x_columns > 0;
     p->g_zs = sh.G;
     p->zfused = sh.fused;
     p->fy = sh.fy;

@@ -125,6 +125,7 @@ struct dfp_batch {
     // launches of one phase (independent case lists) run side by side on the
     // caller's stream and these, forked and joined with events
     std::vector<hipStream_t> aux;
+    bool fixed_grid = false;  // dfp_batch_set_occupancy: persistent launches of that many workgroups
     int n_par = 3;  // auxiliary streams in use (<= aux.size())
     hipEvent_t ev_fork = nullptr;
     std::vector<hipEvent_t> ev_join;
@@ -162,6 +163,7 @@ struct Launch {
     int R;        // z-split radix (x kernels)
     size_t tab;   // offset of the case records
     int list;     // case list
+    int items;    // its work items
     size_t lds;
     int phase;    // launches of one phase are independent and may run concurrently
 };
@@ -255,6 +257,7 @@ int dfp_batch_set_occupancy(dfp_batch* b, int x_per_cu, int z_per_cu, int s_per_
     if (!b) return DFP_E_ARG;
     if (x_per_cu < 1 || x_per_cu > 16 || z_per_cu < 1 || z_per_cu > 16 || s_per_cu < 1 || s_per_cu > 32)
         return bfail(b, DFP_E_ARG, "workgroups per CU out of range");
+    b->fixed_grid = true;
     b->occ_x = x_per_cu;
     b->occ_z = z_per_cu;
     b->occ_s = s_per_cu;
@@ -434,7 +437,9 @@ int dfp_batch_project(dfp_batch* b, int n, dfp_plan* const* plans, double* const
     std::vector<Launch> ls;
     int phase = 0;
     auto add = [&](Launch::Kind k, int f32, int mode, int R, size_t tab, int list, size_t lds) {
-        ls.push_back(Launch{k, f32, mode, R, tab, list, lds_bucket(lds, lds_limit), phase});
+        const int items = pool[(size_t)list * list_stride + counts[list]];
+        ls.push_back(Launch{k, f32, mode, R, tab, list, items, b->use_graphs ? lds_bucket(lds, lds_limit) : align_up(lds, 1024),
+                            phase});
     };
     // the x launches of a set of records, one per radix present; the z launches
     // for its fused and split members
@@ -465,7 +470,7 @@ int dfp_batch_project(dfp_batch* b, int n, dfp_plan* const* plans, double* const
         for (int a : recs) {
             dfp_plan* p = plans[f32 ? i32[a] : i64[a]];
             if (Fs[a]) { fz.push_back(a); lf = std::max(lf, zf_lds_bytes(p, f32)); continue; }
-            const int v = z_variant(p);
+            const int v = 2 * z_variant(p) + zplane_wide(p);
             size_t k = 0;
             while (k < sz.size() && sz[k].first != v) ++k;
             if (k == sz.size()) { sz.push_back({v, {}}); lsz.push_back(0); }
@@ -475,7 +480,7 @@ int dfp_batch_project(dfp_batch* b, int n, dfp_plan* const* plans, double* const
         // one phase: the fused kernel and the split pairs (each workgroup
         // eliminates a sub-plane and substitutes back through it)
         if (!fz.empty()) add(Launch::ZFUSED, f32, 0, 0, tab, make_list(fz, w), lf);
-        for (size_t k = 0; k < sz.size(); ++k) add(Launch::ZFB, f32, 0, sz[k].first, tab, make_list(sz[k].second, w), lsz[k]);
+        for (size_t k = 0; k < sz.size(); ++k) add(Launch::ZFB, f32, sz[k].first & 1, sz[k].first >> 1, tab, make_list(sz[k].second, w), lsz[k]);
         ++phase;
     };
     auto first = [](int k) { std::vector<int> v(k); for (int a = 0; a < k; ++a) v[a] = a; return v; };
@@ -516,13 +521,20 @@ int dfp_batch_project(dfp_batch* b, int n, dfp_plan* const* plans, double* const
     unsigned char* D = b->d_buf;
     const int* d_counts = reinterpret_cast<const int*>(D + L.counts);
     const int* d_pool = reinterpret_cast<const int*>(D + L.lists);
-    const int gx = b->n_cu * b->occ_x, gz = b->n_cu * b->occ_z, gs = b->n_cu * b->occ_s;
+    const int gz = b->n_cu * b->occ_z;
     // one launch on stream st
     auto run_one = [&](const Launch& l, hipStream_t st) -> hipError_t {
         {
             const int* o = d_pool + (size_t)l.list * list_stride;
             const int* ix = o + b->cap + 1;
             const int* nc = d_counts + l.list;
+            // one workgroup per tile, unless the grid has to serve any batch
+            // (a graph) or the caller chose it: a persistent workgroup waits
+            // for its last tile's stores before the next one's loads (48
+            // uneven channels: correction 238 -> 211 us, forward x 165 -> 156).  The z
+            // kernels load ahead across their items and stay persistent.
+            const bool each = !b->use_graphs && !b->fixed_grid && l.items > 0;
+            const int gx = each ? -l.items : b->n_cu * b->occ_x, gs = each ? -l.items : b->n_cu * b->occ_s;
             hipError_t e = hipSuccess;
             switch (l.kind) {
                 case Launch::XF:
@@ -539,9 +551,9 @@ int dfp_batch_project(dfp_batch* b, int n, dfp_plan* const* plans, double* const
                     break;
                 case Launch::ZFB:
                     e = l.f32 ? launch_zsolve_batch(st, l.R, reinterpret_cast<const ZPar<float2>*>(D + l.tab), o,
-                                                    ix, nc, gz, l.lds)
+                                                    ix, nc, gz, l.lds, l.mode)
                               : launch_zsolve_batch(st, l.R, reinterpret_cast<const ZPar<double2>*>(D + l.tab), o,
-                                                    ix, nc, gz, l.lds);
+                                                    ix, nc, gz, l.lds, l.mode);
                     break;
                 case Launch::ZFUSED:
                     e = l.f32 ? launch_zfused_batch(st, reinterpret_cast<const ZPar<float2>*>(D + l.tab), o, ix, nc,

@@ -270,6 +270,7 @@ struct dfp_plan {
     // launch shapes
     int tk_x = 8;   // z columns per block of the forward x kernel (zr lines each)
     int tk_xi = 8;  // z columns per block of the inverse x kernel
+    bool tuned_columns = false;  // the caller chose them (else small grids launch narrower tiles)
     int g_zs = 4;   // rows per group of the split z kernels, or rows per FFT call of the fused one
     int zfused = 0; // 1: one fused z kernel (whole sub-plane in LDS); 0: the split pair
     int zn1 = 0, zn2 = 0;  // two-pass z transforms of the split pair (0: staged transform)
@@ -312,6 +313,11 @@ constexpr int zplane_threads(int n, int nb) {
     if (nb == 1) return 384;
     return n == 18 || n == 27 || n == 36 || n == 54 || n == 81 || n == 96 || n == 108 || n == 128 ? 512 : 768;
 }
+// Threads of a batched register-plane workgroup (as many planes as fill them),
+// or zplane_threads where one plane needs more (wide).  With 256 a CU holds four
+// such workgroups by their LDS (16 waves), with 384 two (12): 48 uneven channels'
+// z stage 181 -> 170 us.
+constexpr int kZpBatchThreads = 256;
 // rows whose second exchange stays within a wave (16, 32, 64 modes), and the LDS slots per N2 elements of a row
 __host__ __device__ constexpr bool zplane_lane(int n1, int n2, int br) { return br == 8 && n2 == 8 && 64 % (n1 * n2) == 0; }
 __host__ __device__ constexpr int zplane_pad(int n1, int n2, int br) { return zplane_lane(n1, n2, br) ? n2 + 1 : n2; }
@@ -325,7 +331,7 @@ template <typename C>
 hipError_t launch_zplane(dfp_plan* p, const ZPar<C>& zp);
 template <typename C>
 hipError_t launch_zplane_batch(hipStream_t s, int variant, const ZPar<C>* cs, const int* off, const int* idx,
-                               const int* nc, int grid, size_t lds);
+                               const int* nc, int grid, size_t lds, int wide);
 hipError_t launch_irfft_x(dfp_plan* p, double* rhs, double* P, double dtc, int save_p);
 // fused z transform + y solve (whole sub-plane in LDS)
 template <typename C> hipError_t launch_zfused(dfp_plan* p, const ZPar<C>& zp);
@@ -401,7 +407,9 @@ hipError_t launch_xinv_batch(hipStream_t s, int R, int accum, const XPar<C>* cs,
                              const int* nc, int grid, size_t lds);
 template <typename C>
 hipError_t launch_zsolve_batch(hipStream_t s, int variant, const ZPar<C>* cs, const int* off, const int* idx,
-                               const int* nc, int grid, size_t lds);
+                               const int* nc, int grid, size_t lds, int wide);
+// the register planes of a plan need more than kZpBatchThreads threads: a wide batched workgroup
+int zplane_wide(const dfp_plan* p);
 hipError_t launch_correct_batch(hipStream_t s, const CPar* cs, const int* off, const int* idx, const int* nc,
                                 int grid);
 hipError_t launch_mode00_batch(hipStream_t s, const MPar* cs, const int* idx, const int* nc, int grid);
@@ -419,13 +427,15 @@ inline int ceil_div(long a, long b) { return (int)((a + b - 1) / b); }
 // transform: its kernel takes four slots each (FP32 form only).
 bool xfwd_wide(const FftDesc& fx, int R, int T);
 
-// Workgroups of a persistent (batched) launch: the caller's count, capped at
-// what the device holds at once of this kernel with this LDS.  A workgroup
-// beyond that would start only once another has finished all of its work
-// items, and then run its own items with the GPU mostly idle.
+// Workgroups of a batched launch.  grid > 0: a persistent launch, the caller's
+// count, capped at what the device holds at once of this kernel with this LDS
+// (a workgroup beyond that would start only once another has finished all of
+// its work items, and then run its own items with the GPU mostly idle).
+// grid < 0: -grid work items, one workgroup each.
 int resident_limit(const void* kernel, int threads, size_t lds);  // per device, cached; 0 if unknown
 template <typename K>
 inline int resident_grid(K kernel, int grid, int threads, size_t lds) {
+    if (grid < 0) return -grid;
     const int cap = resident_limit(reinterpret_cast<const void*>(kernel), threads, lds);
     return cap > 0 && cap < grid ? cap : grid;
 }

@@ -46,6 +46,24 @@ void xpar_columns(XPar<C>& q, const dfp_plan* p, int inv) {
 template void xpar_columns<double2>(XPar<double2>&, const dfp_plan*, int);
 template void xpar_columns<float2>(XPar<float2>&, const dfp_plan*, int);
 
+// A single launch on a small grid: narrower tiles while the launch has fewer
+// than two workgroups per CU, down to four columns (64-byte FP64 spectrum
+// segments).  64x64x64 (16 columns in 64 workgroups -> 4 in
+// 256): forward 10.2 -> 7.6 us, inverse 10.6 -> 7.5.  The FP32
+// form keeps its tiles, whose sums per workgroup set the order of its row
+// sums, and batched launches theirs, since the other cases fill the GPU.
+static void narrow_columns(XPar<double2>& q) {
+    const int nz2 = q.g.nzp / q.R;
+    int T = q.T;
+    for (int t = T - 1; t >= 4 && (long)(nz2 / T) * q.g.nym < 512; --t)
+        if (nz2 % t == 0) T = t;
+    q.T = T;
+    q.nbx = nz2 / T;
+    q.strip = q.g.nxp >= 512 ? std::min(q.nbx, 8) : q.nbx;  // as xpar_columns
+    q.div_t = FastDiv(T);
+}
+static void narrow_columns(XPar<float2>&) {}
+
 template <typename C>
 XPar<C> make_xpar(const dfp_plan* p, int inv) {
     XPar<C> q{};
@@ -80,14 +98,16 @@ XPar<C> make_xpar(const dfp_plan* p, int inv) {
 template XPar<double2> make_xpar<double2>(const dfp_plan*, int);
 template XPar<float2> make_xpar<float2>(const dfp_plan*, int);
 
-// dynamic LDS of the forward (inv = 0) or inverse (inv = 1) x kernel of a plan
-size_t x_lds_bytes(const dfp_plan* p, int inv, int f32) {
-    const int R = p->zr, T = inv ? p->tk_xi : p->tk_x, nz2 = p->geo.nzp / R, M = p->fx.n;
+// dynamic LDS of an x kernel with T columns per workgroup
+static size_t x_lds_bytes_t(const dfp_plan* p, int T, int f32) {
+    const int R = p->zr, nz2 = p->geo.nzp / R, M = p->fx.n;
     const size_t cs = f32 ? sizeof(float2) : sizeof(double2);
     if (p->geo.xbc == 1)  // DCT-IV: M packed points per line, pre- and post-twiddles
         return cs * ((size_t)R * T * M + twiddle_count(p->fx) + 2 * M + (size_t)nz2 * (R - 1));
     return cs * ((size_t)R * T * (M + 1) + twiddle_count(p->fx) + M + 1 + (size_t)nz2 * (R - 1));
 }
+// of a plan's forward (inv = 0) or inverse (inv = 1) x kernel
+size_t x_lds_bytes(const dfp_plan* p, int inv, int f32) { return x_lds_bytes_t(p, inv ? p->tk_xi : p->tk_x, f32); }
 
 static const char* xname(int mode, bool f32) {
     static const char* names[2][3] = {{"div_rfft_x", "rfft_x_rhs", "res_rfft_x"},
@@ -160,9 +180,10 @@ static hipError_t xdct_inv_any(int R, hipStream_t s, const XPar<double2>& q, dim
 }
 
 template <typename C>
-static hipError_t launch_xfwd(dfp_plan* p, int mode, const XPar<C>& q) {
+static hipError_t launch_xfwd(dfp_plan* p, int mode, XPar<C> q) {
+    if (!p->tuned_columns) narrow_columns(q);
     const dim3 grid(q.nbx, q.g.nym);
-    const size_t lds = x_lds_bytes(p, 0, sizeof(C) == 8);
+    const size_t lds = x_lds_bytes_t(p, q.T, sizeof(C) == 8);
     const int slot = prof_begin(p, xname(mode, sizeof(C) == 8));
     const hipError_t e = xfwd_any<C>(p->zr, p->stream, mode, q, grid, lds);
     prof_end(p, slot);
@@ -176,8 +197,9 @@ hipError_t launch_div_rfft_x(dfp_plan* p, const double* U, const double* V, cons
     if (p->geo.xbc == 1) {
         q.a.phib = from_rhs ? nullptr : phib;
         q.a.idx2 = 1.0 / std::pow(p->dx, 2.0);
+        if (!p->tuned_columns) narrow_columns(q);
         const dim3 grid(q.nbx, q.g.nym);
-        const size_t lds = x_lds_bytes(p, 0, 0);
+        const size_t lds = x_lds_bytes_t(p, q.T, 0);
         const int slot = prof_begin(p, from_rhs ? "dct_x_rhs" : "div_dct_x");
         const hipError_t e = xdct_fwd_any(p->zr, p->stream, from_rhs ? 1 : 0, q, grid, lds);
         prof_end(p, slot);
@@ -193,9 +215,10 @@ hipError_t launch_rfft_x32(dfp_plan* p, int mode, const XArgs& a) {
 }
 
 template <typename C, int ACCUM>
-static hipError_t launch_xinv(dfp_plan* p, const XPar<C>& q) {
+static hipError_t launch_xinv(dfp_plan* p, XPar<C> q) {
+    if (!p->tuned_columns) narrow_columns(q);
     const dim3 grid(q.nbx, q.g.nym);
-    const size_t lds = x_lds_bytes(p, 1, sizeof(C) == 8);
+    const size_t lds = x_lds_bytes_t(p, q.T, sizeof(C) == 8);
     const int slot = prof_begin(p, sizeof(C) == 8 ? "irfft_x32" : "irfft_x");
     const hipError_t e = xinv_any<C>(p->zr, p->stream, ACCUM, q, grid, lds);
     prof_end(p, slot);
@@ -206,8 +229,9 @@ hipError_t launch_irfft_x(dfp_plan* p, double* rhs, double* P, double dtc, int s
     XPar<double2> q = make_xpar<double2>(p, 1);
     q.rhs = rhs; q.P = P; q.dtc = dtc; q.save_p = save_p;
     if (p->geo.xbc == 1) {
+        if (!p->tuned_columns) narrow_columns(q);
         const dim3 grid(q.nbx, q.g.nym);
-        const size_t lds = x_lds_bytes(p, 1, 0);
+        const size_t lds = x_lds_bytes_t(p, q.T, 0);
         const int slot = prof_begin(p, "idct_x");
         const hipError_t e = xdct_inv_any(p->zr, p->stream, q, grid, lds);
         prof_end(p, slot);

@@ -33,9 +33,9 @@ template hipError_t launch_zplane<float2>(dfp_plan*, const ZPar<float2>&);
 
 template <typename C>
 hipError_t launch_zplane_batch(hipStream_t s, int variant, const ZPar<C>* cs, const int* off, const int* idx,
-                               const int* nc, int grid, size_t lds) {
+                               const int* nc, int grid, size_t lds, int wide) {
     const int nb = (variant - kZvPlane) / 1024, n1 = (variant & 1023) / 32, n2 = variant & 31;
-    const int threads = zplane_threads(n1 * n2, nb);
+    const int threads = wide ? zplane_threads(n1 * n2, nb) : kZpBatchThreads;
     switch (n1 * n2) {
 #define DFP_ZP_CASE(a, b, r) \
     case a * b: return launch_zplane_batch_n<C, a, b, r>(s, nb, cs, off, idx, nc, grid, threads, lds);
@@ -46,8 +46,8 @@ hipError_t launch_zplane_batch(hipStream_t s, int variant, const ZPar<C>* cs, co
     return hipErrorInvalidValue;
 }
 template hipError_t launch_zplane_batch<double2>(hipStream_t, int, const ZPar<double2>*, const int*, const int*,
-                                                 const int*, int, size_t);
+                                                 const int*, int, size_t, int);
 template hipError_t launch_zplane_batch<float2>(hipStream_t, int, const ZPar<float2>*, const int*, const int*,
-                                                const int*, int, size_t);
+                                                const int*, int, size_t, int);
 
 }  // namespace dfp

@@ -593,8 +593,10 @@ __global__ void __launch_bounds__(kZsThreads) kb_zsolve(const ZPar<C>* __restric
 // planes per workgroup of the register-plane kernel: enough to fill a
 // wavefront, or a batched launch's fixed workgroup
 static int zplane_planes(const dfp_plan* p, int batch) {
-    return std::max(1, (batch ? zplane_threads(p->fz.n, p->zp_nb) : 64) / (p->fz.n * p->zp_nch));
+    return std::max(1, (batch ? kZpBatchThreads : 64) / (p->fz.n * p->zp_nch));
 }
+
+int zplane_wide(const dfp_plan* p) { return p->zp_nb && p->fz.n * p->zp_nch > kZpBatchThreads; }
 
 static size_t zplane_lds(int threads, int n1, int n2, int nch, int br, int nb, bool f32) {
     const size_t cs = f32 ? sizeof(float2) : sizeof(double2);
@@ -617,7 +619,7 @@ bool zplane_shape(int n, int nym, bool f32, size_t lds_limit, int& nb, int& nch,
         if (threads > zplane_threads(n, q)) continue;
         nb = q;
         nch = (int)(threads / n);
-        // a batched workgroup holds up to zplane_threads threads of planes
+        // a wide batched workgroup holds up to zplane_threads threads of planes
         return zplane_lds(zplane_threads(n, q), n1, n2, nch, br, nb, f32) <= lds_limit;
     }
     return false;
@@ -703,11 +705,11 @@ hipError_t launch_zsolve32(dfp_plan* p) {
     return p->zp_nb ? launch_zplane(p, zp) : launch_zsolve_t<float2>(p, zp);
 }
 
-// variant: z_variant of the cases of the list (all alike)
+// variant, wide: z_variant and zplane_wide of the cases of the list (all alike)
 template <typename C>
 hipError_t launch_zsolve_batch(hipStream_t s, int variant, const ZPar<C>* cs, const int* off, const int* idx,
-                               const int* nc, int grid, size_t lds) {
-    if (variant >= kZvPlane) return launch_zplane_batch<C>(s, variant, cs, off, idx, nc, grid, lds);
+                               const int* nc, int grid, size_t lds, int wide) {
+    if (variant >= kZvPlane) return launch_zplane_batch<C>(s, variant, cs, off, idx, nc, grid, lds, wide);
     const dim3 blk(kZsThreads);
     auto go = [&](auto k) {
         hipLaunchKernelGGL(k, dim3(resident_grid(k, grid, kZsThreads, lds)), blk, lds, s, cs, off, idx, nc);
@@ -725,9 +727,9 @@ hipError_t launch_zsolve_batch(hipStream_t s, int variant, const ZPar<C>* cs, co
     return hipGetLastError();
 }
 template hipError_t launch_zsolve_batch<double2>(hipStream_t, int, const ZPar<double2>*, const int*, const int*,
-                                                 const int*, int, size_t);
+                                                 const int*, int, size_t, int);
 template hipError_t launch_zsolve_batch<float2>(hipStream_t, int, const ZPar<float2>*, const int*, const int*,
-                                                const int*, int, size_t);
+                                                const int*, int, size_t, int);
 
 // rows per group: the group (its rows in each of the block's planes) fits
 // the block's threads (one row coefficient each), the prefetch registers
