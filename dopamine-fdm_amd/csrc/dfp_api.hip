@@ -799,10 +799,15 @@ int dfp_plan_create_tuned(const dfp_grid* g, int precision, int device, const df
     const size_t o_ty2 = tw.size();
     if (G.ybc == 0)
         for (int e = 0; e < G.nym - 1; ++e) tw.push_back(expi(e, G.nym - 1));
+    FftDesc xrd{};
+    const bool xr = !dct && xr_steps(G.nxp / 2, xrd);  // the inverse x lines in registers
+    const size_t o_xr = tw.size();
+    if (xr) stage_twiddles(xrd, tw);
     if (hipMalloc(&p->d_tw, sizeof(double2) * tw.size()) != hipSuccess) return bail(DFP_E_NOMEM);
     if (hipMemcpy(p->d_tw, tw.data(), sizeof(double2) * tw.size(), hipMemcpyHostToDevice) != hipSuccess)
         return bail(DFP_E_HIP);
     p->tw_x = p->d_tw;
+    p->tw_xr = xr ? p->d_tw + o_xr : nullptr;
     p->tw_z = p->d_tw + o_tz;
     p->tw_r2c = p->d_tw + o_r2c;
     p->tw_zs = p->d_tw + o_zs;
@@ -816,6 +821,7 @@ int dfp_plan_create_tuned(const dfp_grid* g, int precision, int device, const df
         if (hipMemcpy(p->d_tw32, tw32.data(), sizeof(float2) * tw32.size(), hipMemcpyHostToDevice) != hipSuccess)
             return bail(DFP_E_HIP);
         p->tw_x32 = p->d_tw32;
+        p->tw_xr32 = xr ? p->d_tw32 + o_xr : nullptr;
         p->tw_z32 = p->d_tw32 + o_tz;
         p->tw_z2_32 = p->d_tw32 + o_t2;
     }

@@ -159,7 +159,7 @@ int bfail(dfp_batch* b, int code, const char* fmt, ...) {
 struct Launch {
     enum Kind { XF, XI, ZFB, ZFUSED, M00, SAVE, CORR } kind;
     int f32;      // spectrum precision
-    int mode;     // x forward mode, or ACCUM for the inverse
+    int mode;     // x forward mode, ACCUM + 16 M (register lines) for the inverse, zplane_wide
     int R;        // z-split radix (x kernels)
     size_t tab;   // offset of the case records
     int list;     // case list
@@ -445,19 +445,23 @@ int dfp_batch_project(dfp_batch* b, int n, dfp_plan* const* plans, double* const
     // for its fused and split members
     auto x_launches = [&](Launch::Kind k, int f32, int mode, size_t tab, const std::vector<int>& recs,
                           const std::vector<int>& Rs, const std::vector<size_t>& w, int inv) {
-        for (int R : kRadixList) {
-            std::vector<int> sel;
-            size_t lds = 0;
-            bool wide = false;  // a forward tile too large for two butterfly slots: the four-slot kernel
-            for (int a : recs)
-                if (Rs[a] == R) {
+        // inverse: one launch per line length of the register kernel, one for the other lengths
+        for (int R : kRadixList)
+            for (int M : {0, 16, 24, 32, 48, 64, 96, 128, 192, 256}) {
+                std::vector<int> sel;
+                size_t lds = 0;
+                bool wide = false;  // a forward tile too large for two butterfly slots: the four-slot kernel
+                for (int a : recs) {
+                    if (Rs[a] != R) continue;
                     const dfp_plan* p = plans[f32 ? i32[a] : i64[a]];
+                    const size_t reg = inv ? xinv_reg_lds(p, f32) : 0;
+                    if (M != (reg ? p->fx.n : 0)) continue;
                     sel.push_back(a);
-                    lds = std::max(lds, x_lds_bytes(p, inv, f32));
+                    lds = std::max(lds, reg ? reg : x_lds_bytes(p, inv, f32));
                     wide = wide || (!inv && xfwd_wide(p->fx, R, p->tk_x));
                 }
-            if (!sel.empty()) add(k, f32, wide ? mode | 8 : mode, R, tab, make_list(sel, w), lds);
-        }
+                if (!sel.empty()) add(k, f32, (wide ? mode | 8 : mode) | M << 4, R, tab, make_list(sel, w), lds);
+            }
         ++phase;
     };
     auto z_launches = [&](int f32, size_t tab, const std::vector<int>& recs, const std::vector<int>& Fs,
@@ -544,10 +548,10 @@ int dfp_batch_project(dfp_batch* b, int n, dfp_plan* const* plans, double* const
                                                   o, ix, nc, gx, l.lds);
                     break;
                 case Launch::XI:
-                    e = l.f32 ? launch_xinv_batch(st, l.R, l.mode, reinterpret_cast<const XPar<float2>*>(D + l.tab),
-                                                  o, ix, nc, gx, l.lds)
-                              : launch_xinv_batch(st, l.R, l.mode, reinterpret_cast<const XPar<double2>*>(D + l.tab),
-                                                  o, ix, nc, gx, l.lds);
+                    e = l.f32 ? launch_xinv_batch(st, l.R, l.mode & 15, reinterpret_cast<const XPar<float2>*>(D + l.tab),
+                                                  o, ix, nc, gx, l.lds, l.mode >> 4)
+                              : launch_xinv_batch(st, l.R, l.mode & 15, reinterpret_cast<const XPar<double2>*>(D + l.tab),
+                                                  o, ix, nc, gx, l.lds, l.mode >> 4);
                     break;
                 case Launch::ZFB:
                     e = l.f32 ? launch_zsolve_batch(st, l.R, reinterpret_cast<const ZPar<float2>*>(D + l.tab), o,
@@ -610,7 +614,7 @@ int dfp_batch_project(dfp_batch* b, int n, dfp_plan* const* plans, double* const
         std::vector<long> key;
         for (const Launch& l : ls) {
             key.push_back(l.kind);
-            key.push_back(l.f32 * 16 + l.mode);
+            key.push_back(l.f32 * 8192 + l.mode);
             key.push_back(l.R);
             key.push_back((long)l.tab);
             key.push_back(l.list);

@@ -105,6 +105,7 @@ struct XPar {
     Ops o;
     FftDesc fd;          // x FFT of length nxp/2
     const C* tw;         // x stages | R2C packing (nxp/2+1) | first z stage (nz2*(R-1))
+    const C* twr;        // step twiddles of the register lines (k_xinv_reg.h), or null
     C* spec;
     int ntw, R, T, nbx;  // stage-twiddle count, z split radix, columns per block, blocks per row
     int strip;           // column blocks per strip of the workgroup order (nbx: row-major)
@@ -227,12 +228,14 @@ struct dfp_plan {
     double2* d_z00 = nullptr;
     int zr = 1;                  // radix of the z stage applied by the x kernels (z split)
     const double2* tw_x = nullptr;
+    const double2* tw_xr = nullptr;   // step twiddles of the x lines in registers (k_xinv_reg.h), or null
     const double2* tw_z = nullptr;
     const double2* tw_z2 = nullptr;   // exp(-2 pi i e / n), e < n = nzp/zr (two-pass z transforms)
     const double2* tw_r2c = nullptr;  // exp(-2 pi i k / nxp), k = 0..nxp/2
     const double2* tw_zs = nullptr;   // exp(-2 pi i k' u / nzp), [k'*(zr-1) + u-1], k' < nzp/zr, 1 <= u < zr
     float2* d_tw32 = nullptr;         // the same table rounded to FP32 (FP32 form)
     const float2* tw_x32 = nullptr;
+    const float2* tw_xr32 = nullptr;
     const float2* tw_z32 = nullptr;
     const float2* tw_z2_32 = nullptr;
     // device work arrays
@@ -404,7 +407,11 @@ hipError_t launch_xfwd_batch(hipStream_t s, int R, int mode, const XPar<C>* cs, 
                              const int* nc, int grid, size_t lds);
 template <typename C>
 hipError_t launch_xinv_batch(hipStream_t s, int R, int accum, const XPar<C>* cs, const int* off, const int* idx,
-                             const int* nc, int grid, size_t lds);
+                             const int* nc, int grid, size_t lds, int M);
+// LDS of the inverse x kernel with the lines in registers (k_xinv_reg.h) for
+// a plan, 0 if it does not take the plan's lines; M of launch_xinv_batch: the
+// lines of every case where that kernel runs them, else 0
+size_t xinv_reg_lds(const dfp_plan* p, int f32);
 template <typename C>
 hipError_t launch_zsolve_batch(hipStream_t s, int variant, const ZPar<C>* cs, const int* off, const int* idx,
                                const int* nc, int grid, size_t lds, int wide);

@@ -444,4 +444,33 @@ inline int twiddle_count(const FftDesc& d) {
     return t;
 }
 
+// The x lines in registers (k_xinv_reg.h): points per lane and radix steps of
+// M-point lines
+template <int M> struct XrSteps;
+template <> struct XrSteps<16> { static constexpr int e = 8, r[3] = {8, 2, 1}; };
+template <> struct XrSteps<24> { static constexpr int e = 12, r[3] = {12, 2, 1}; };
+template <> struct XrSteps<32> { static constexpr int e = 8, r[3] = {8, 4, 1}; };
+template <> struct XrSteps<48> { static constexpr int e = 12, r[3] = {12, 4, 1}; };
+template <> struct XrSteps<64> { static constexpr int e = 8, r[3] = {8, 8, 1}; };
+template <> struct XrSteps<96> { static constexpr int e = 12, r[3] = {12, 4, 2}; };
+template <> struct XrSteps<128> { static constexpr int e = 8, r[3] = {8, 4, 4}; };
+template <> struct XrSteps<192> { static constexpr int e = 12, r[3] = {12, 4, 4}; };
+template <> struct XrSteps<256> { static constexpr int e = 8, r[3] = {8, 8, 4}; };
+#define DFP_XR_LINES(X) X(16) X(24) X(32) X(48) X(64) X(96) X(128) X(192) X(256)
+// the steps for the host's twiddles; false if no kernel takes M-point lines
+inline bool xr_steps(int M, FftDesc& d) {
+    d = FftDesc{};
+    d.n = M;
+    switch (M) {
+#define DFP_XR_CASE(m)                      \
+    case m:                                 \
+        for (int r : XrSteps<m>::r)         \
+            if (r > 1) d.rad[d.nst++] = r;  \
+        return true;
+        DFP_XR_LINES(DFP_XR_CASE)
+#undef DFP_XR_CASE
+    }
+    return false;
+}
+
 }  // namespace dfp

@@ -16,7 +16,9 @@ hipError_t launch_xfwd_batch_r(hipStream_t s, int mode, const XPar<C>* cs, const
                                const int* nc, int grid, size_t lds);
 template <int R, typename C>
 hipError_t launch_xinv_batch_r(hipStream_t s, int accum, const XPar<C>* cs, const int* off, const int* idx,
-                               const int* nc, int grid, size_t lds);
+                               const int* nc, int grid, size_t lds, int M);
+template <typename C>
+size_t xr_lds_any(int M, int R, int T);
 template <int R>
 hipError_t launch_xdct_fwd_r(hipStream_t s, int mode, const XPar<double2>& q, dim3 grid, size_t lds);
 template <int R>
@@ -88,9 +90,11 @@ XPar<C> make_xpar(const dfp_plan* p, int inv) {
     q.dtc = 1.0;
     if (sizeof(C) == sizeof(double2)) {
         q.tw = reinterpret_cast<const C*>(p->tw_x);
+        q.twr = reinterpret_cast<const C*>(p->tw_xr);
         q.spec = reinterpret_cast<C*>(p->d_spec);
     } else {
         q.tw = reinterpret_cast<const C*>(p->tw_x32);
+        q.twr = reinterpret_cast<const C*>(p->tw_xr32);
         q.spec = reinterpret_cast<C*>(p->d_spec);
     }
     return q;
@@ -108,6 +112,11 @@ static size_t x_lds_bytes_t(const dfp_plan* p, int T, int f32) {
 }
 // of a plan's forward (inv = 0) or inverse (inv = 1) x kernel
 size_t x_lds_bytes(const dfp_plan* p, int inv, int f32) { return x_lds_bytes_t(p, inv ? p->tk_xi : p->tk_x, f32); }
+
+size_t xinv_reg_lds(const dfp_plan* p, int f32) {
+    if (!p->tw_xr) return 0;
+    return f32 ? xr_lds_any<float2>(p->fx.n, p->zr, p->tk_xi) : xr_lds_any<double2>(p->fx.n, p->zr, p->tk_xi);
+}
 
 static const char* xname(int mode, bool f32) {
     static const char* names[2][3] = {{"div_rfft_x", "rfft_x_rhs", "res_rfft_x"},
@@ -157,15 +166,15 @@ template hipError_t launch_xfwd_batch<float2>(hipStream_t, int, int, const XPar<
 
 template <typename C>
 hipError_t launch_xinv_batch(hipStream_t s, int R, int accum, const XPar<C>* cs, const int* off, const int* idx,
-                             const int* nc, int grid, size_t lds) {
-#define DFP_CALL(RV) launch_xinv_batch_r<RV, C>(s, accum, cs, off, idx, nc, grid, lds)
+                             const int* nc, int grid, size_t lds, int M) {
+#define DFP_CALL(RV) launch_xinv_batch_r<RV, C>(s, accum, cs, off, idx, nc, grid, lds, M)
     DFP_R_SWITCH(R, DFP_CALL)
 #undef DFP_CALL
 }
 template hipError_t launch_xinv_batch<double2>(hipStream_t, int, int, const XPar<double2>*, const int*, const int*,
-                                               const int*, int, size_t);
+                                               const int*, int, size_t, int);
 template hipError_t launch_xinv_batch<float2>(hipStream_t, int, int, const XPar<float2>*, const int*, const int*,
-                                              const int*, int, size_t);
+                                              const int*, int, size_t, int);
 
 static hipError_t xdct_fwd_any(int R, hipStream_t s, int mode, const XPar<double2>& q, dim3 grid, size_t lds) {
 #define DFP_CALL(RV) launch_xdct_fwd_r<RV>(s, mode, q, grid, lds)

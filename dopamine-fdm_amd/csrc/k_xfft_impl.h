@@ -451,6 +451,10 @@ __global__ void __launch_bounds__(kXThreads) kb_irfft_x(const XPar<C>* __restric
 }
 
 
+}  // namespace dfp
+#include "k_xinv_reg.h"
+namespace dfp {
+
 // launches of the kernels above for one z-split radix R (instantiated per R
 // in k_xfft_r<R>.hip, so the radices compile in parallel)
 template <int R, typename C>
@@ -480,6 +484,8 @@ hipError_t launch_xfwd_r(hipStream_t s, int mode, const XPar<C>& q, dim3 grid, s
 
 template <int R, typename C>
 hipError_t launch_xinv_r(hipStream_t s, int accum, const XPar<C>& q, dim3 grid, size_t lds) {
+    if (accum ? launch_xinv_reg<C, sizeof(C) == sizeof(float2), R>(s, q, grid) : launch_xinv_reg<C, 0, R>(s, q, grid))
+        return hipGetLastError();
     if (!accum) {
         hipLaunchKernelGGL((k_irfft_x<C, 0, R>), grid, dim3(kXThreads), lds, s, q);
     } else {
@@ -527,7 +533,12 @@ hipError_t launch_xfwd_batch_r(hipStream_t s, int mode, const XPar<C>* cs, const
 
 template <int R, typename C>
 hipError_t launch_xinv_batch_r(hipStream_t s, int accum, const XPar<C>* cs, const int* off, const int* idx,
-                               const int* nc, int grid, size_t lds) {
+                               const int* nc, int grid, size_t lds, int M) {
+    if (M > 0) {
+        constexpr int A1 = sizeof(C) == sizeof(float2);
+        return accum ? launch_xinv_reg_batch<C, A1, R>(s, M, cs, off, idx, nc, grid, lds)
+                     : launch_xinv_reg_batch<C, 0, R>(s, M, cs, off, idx, nc, grid, lds);
+    }
     if (!accum) {
         const auto k = kb_irfft_x<C, 0, R>;
         hipLaunchKernelGGL(k, dim3(resident_grid(k, grid, kXThreads, lds)), dim3(kXThreads), lds, s, cs, off, idx, nc);
@@ -547,6 +558,8 @@ hipError_t launch_xinv_batch_r(hipStream_t s, int accum, const XPar<C>* cs, cons
 
 #define DFP_INSTANTIATE_XFFT(RV)                                                                                   \
     namespace dfp {                                                                                                \
+    template size_t xr_lds_any<double2>(int, int, int);                                                            \
+    template size_t xr_lds_any<float2>(int, int, int);                                                             \
     template hipError_t launch_xfwd_r<RV, double2>(hipStream_t, int, const XPar<double2>&, dim3, size_t);         \
     template hipError_t launch_xfwd_r<RV, float2>(hipStream_t, int, const XPar<float2>&, dim3, size_t);           \
     template hipError_t launch_xinv_r<RV, double2>(hipStream_t, int, const XPar<double2>&, dim3, size_t);         \
@@ -556,7 +569,7 @@ hipError_t launch_xinv_batch_r(hipStream_t s, int accum, const XPar<C>* cs, cons
     template hipError_t launch_xfwd_batch_r<RV, float2>(hipStream_t, int, const XPar<float2>*, const int*,        \
                                                         const int*, const int*, int, size_t);                                  \
     template hipError_t launch_xinv_batch_r<RV, double2>(hipStream_t, int, const XPar<double2>*, const int*,      \
-                                                         const int*, const int*, int, size_t);                                 \
+                                                         const int*, const int*, int, size_t, int);                            \
     template hipError_t launch_xinv_batch_r<RV, float2>(hipStream_t, int, const XPar<float2>*, const int*,        \
-                                                        const int*, const int*, int, size_t);                                  \
+                                                        const int*, const int*, int, size_t, int);                             \
     }

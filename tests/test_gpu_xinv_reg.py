@@ -1,0 +1,71 @@
+"""The inverse x kernel with the lines in registers (nxp = 2^n and 3 2^n from 32
+to 512; z splits 1, 2, 4, 8): each line length with each split, tiles of one
+column, of a column count that is no power of two and partial ones, a single
+y row, the duplicate row of a periodic y, z walls, P with its ghosts.
+
+FP64: the parity bar against the C oracle.  FP32+refine: one sweep leaves the
+square of the FP32 solve's error (below 1e-5 on these grids), 1e-10.  A batch
+runs the same arithmetic as the plans one by one: equal bits."""
+from __future__ import annotations
+
+import pytest
+
+import dfp
+from _cases import fields, make_grid, oracle_project, rel_linf
+
+pytestmark = pytest.mark.gpu
+
+DT, C3 = 1e-3, 0.75
+
+
+def _check(g, tuning=None, precision=dfp.DFP_FP64, bar=1e-12):
+    U, V, W, P, rhs = fields(g, 3, 0.1)
+    o = [a.copy(order="F") for a in (U, V, W, P, rhs)]
+    oracle_project(g, *o, DT, C3, save_p=True)
+    plan = dfp.Plan(g, precision=precision, tuning=tuning)
+    plan.project(U, V, W, rhs, P, DT, C3, save_p=True)
+    plan.close()
+    for lab, a, b in zip(("U", "V", "W", "P", "phi"), (U, V, W, P, rhs), o):
+        assert rel_linf(a, b) <= bar, lab
+
+
+@pytest.mark.parametrize("nxp", [32, 48, 64, 96, 128, 192, 256, 384, 512])
+@pytest.mark.parametrize("nym,nzp,R,T", [(1, 16, 1, 0), (3, 16, 2, 0), (9, 16, 4, 0), (4, 24, 8, 0), (6, 12, 4, 3),
+                                         (5, 16, 4, 1), (7, 6, 1, 2)])
+def test_lines_in_registers_match_oracle(nxp, nym, nzp, R, T):
+    print(f"{nxp}x{nym}x{nzp}, split {R}, columns {T}", flush=True)
+    g = make_grid(nxp, nym, nzp, 1.5)
+    _check(g, (R, T, 0, 0))
+    _check(g, (R, T, 0, 0), dfp.DFP_FP32_REFINE, 1e-10)
+
+
+@pytest.mark.parametrize("nxp", [32, 96, 128, 512])
+def test_lines_in_registers_periodic_y_and_z_walls(nxp):
+    print(f"nxp {nxp}", flush=True)
+    _check(dfp.periodic_y_grid(nxp, 9, 16))
+    _check(dfp.duct_grid(nxp, 6, 10, 1.0, 0.7))
+
+
+@pytest.mark.parametrize("precision", [dfp.DFP_FP64, dfp.DFP_FP32_REFINE])
+def test_batch_of_register_lines_equals_single_plans(precision):
+    import torch
+
+    from dfp.batch import Batch, Case
+
+    sizes = [(32, 5, 12), (64, 7, 16), (128, 4, 24), (256, 3, 16), (512, 2, 16), (48, 6, 12), (96, 5, 24), (36, 4, 12)]
+    batch, cases, singles = Batch(max_cases=len(sizes)), [], []
+    for n in sizes:
+        g = make_grid(*n, 1.5)
+        host = fields(g, sum(n), 0.1)
+        dev = [[torch.from_numpy(a.T.copy()).cuda() for a in host] for _ in range(2)]
+        U, V, W, P, rhs = dev[0]
+        plan = dfp.Plan(g, precision=precision)
+        plan.project(U, V, W, rhs, P, DT, C3, save_p=True)
+        plan.close()
+        singles.append(dev[0])
+        U, V, W, P, rhs = dev[1]
+        cases.append(Case(dfp.Plan(g, precision=precision), U, V, W, rhs, P, DT, C3, save_p=True))
+    batch.project(cases)
+    for n, c, s in zip(sizes, cases, singles):
+        for lab, a, b in zip(("U", "V", "W", "P", "phi"), (c.U, c.V, c.W, c.P, c.rhs), s):
+            assert torch.equal(a, b), (n, lab)
