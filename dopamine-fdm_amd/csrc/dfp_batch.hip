@@ -4,8 +4,8 @@
 // Every stage kernel has a batched form (kb_*) whose workgroups walk the
 // concatenated work lists of all cases of the stage: the case records
 // (XPar/ZPar/CPar/MPar/SPar) and the per-case work offsets are written on the
-// host into one pinned staging buffer, copied to the device with one
-// asynchronous copy, and read by the kernels.  The kernels' own arguments are
+// host into one pinned staging buffer, copied to the device by one small
+// kernel, and read by the kernels.  The kernels' own arguments are
 // then only addresses inside that device buffer, the case counts live in it
 // too, and the grid is fixed (workgroups per CU x CUs, capped at what the
 // device holds at once of the kernel with its LDS), so a launch sequence
@@ -126,13 +126,18 @@ struct dfp_batch {
     // caller's stream and these, forked and joined with events
     std::vector<hipStream_t> aux;
     bool fixed_grid = false;  // dfp_batch_set_occupancy: persistent launches of that many workgroups
-    int n_par = 3;  // auxiliary streams in use (<= aux.size())
+    int n_par = 3;  // dfp_batch_set_parallel: at most this many of them are used
     hipEvent_t ev_fork = nullptr;
     std::vector<hipEvent_t> ev_join;
     std::string last_error;
 };
 
-constexpr int kAuxStreams = 3;  // with the caller's stream: four, the process's hardware queues
+// dfp_batch_set_parallel takes 0..3.  One auxiliary stream is what helps: a
+// fork and its join cost 10-30 us for each stream that takes part (48 uneven
+// channels, FP64 / FP32+refine: none 895 / 1268 us, one 836 / 1165, two
+// 859 / 1158, three 872 / 1217; the largest launches first instead of in turn: 868 / 1229).
+constexpr int kMaxParallel = 3;
+constexpr int kAuxStreams = 1;
 
 namespace {
 
@@ -180,6 +185,19 @@ void release_streams(dfp_batch* b) {
 void destroy_graphs(dfp_batch* b) {
     for (auto& kv : b->graphs) (void)hipGraphExecDestroy(kv.second);
     b->graphs.clear();
+}
+
+// Tables in use, in 16-byte units of the staging buffer (whose tables start
+// at multiples of 256 bytes), copied by a kernel that reads the pinned buffer: an
+// asynchronous copy runs on another queue, and the stream waited 34 us between
+// the work before it and the first launch after it.
+struct Segments {
+    uint32_t at[13], len[13];
+    int n;
+};
+__global__ void __launch_bounds__(256) k_stage_tables(const uint4* __restrict__ src, uint4* __restrict__ dst, Segments sg) {
+    const uint32_t at = sg.at[blockIdx.y], len = sg.len[blockIdx.y];
+    for (uint32_t e = blockIdx.x * 256 + threadIdx.x; e < len; e += gridDim.x * 256) dst[at + e] = src[at + e];
 }
 
 // LDS of a batched launch rounded up to a power of two of at least 4 KiB
@@ -274,8 +292,8 @@ int dfp_batch_use_graphs(dfp_batch* b, int enable) {
 
 int dfp_batch_set_parallel(dfp_batch* b, int aux_streams) {
     if (!b) return DFP_E_ARG;
-    if (aux_streams < 0 || aux_streams > (int)b->aux.size())
-        return bfail(b, DFP_E_ARG, "auxiliary streams out of range (0..%d)", (int)b->aux.size());
+    if (aux_streams < 0 || aux_streams > kMaxParallel)
+        return bfail(b, DFP_E_ARG, "auxiliary streams out of range (0..%d)", kMaxParallel);
     if (aux_streams != b->n_par) destroy_graphs(b);
     b->n_par = aux_streams;
     return DFP_OK;
@@ -516,9 +534,28 @@ int dfp_batch_project(dfp_batch* b, int n, dfp_plan* const* plans, double* const
     if (!solve) add(Launch::CORR, 0, 0, 0, L.c, make_list(first(n), wc), 0);
     if (overflow) return bfail(b, DFP_E_UNSUPPORTED, "too many case lists in one call");
 
-    // tables to the device (up to the last list used), then the launches (or their graph)
-    const size_t used = L.lists + sizeof(int) * (size_t)nlists * list_stride;
-    BCHK(b, hipMemcpyAsync(b->d_buf, b->h_buf, used, hipMemcpyHostToDevice, b->stream));
+    // tables to the device, then the launches (or their graph)
+    Segments sg{};
+    auto seg = [&](size_t at, size_t bytes) {
+        if (bytes) sg.at[sg.n] = (uint32_t)(at / 16), sg.len[sg.n++] = (uint32_t)((bytes + 15) / 16);
+    };
+    seg(L.x64, sizeof(XPar<double2>) * n64);
+    seg(L.x64i, sizeof(XPar<double2>) * n64);
+    seg(L.z64, sizeof(ZPar<double2>) * n64);
+    seg(L.x32, sizeof(XPar<float2>) * n32);
+    seg(L.x32i, sizeof(XPar<float2>) * n32);
+    seg(L.x32s, sizeof(XPar<float2>) * n32);
+    seg(L.x32si, sizeof(XPar<float2>) * n32);
+    seg(L.z32, sizeof(ZPar<float2>) * n32);
+    seg(L.m32, sizeof(MPar) * n32);
+    seg(L.s32, sizeof(SPar) * ns);
+    seg(L.c, solve ? 0 : sizeof(CPar) * n);
+    seg(L.counts, sizeof(int) * nlists);
+    seg(L.lists, sizeof(int) * (size_t)nlists * list_stride);
+    void* h_dev = nullptr;
+    BCHK(b, hipHostGetDevicePointer(&h_dev, b->h_buf, 0));
+    hipLaunchKernelGGL(k_stage_tables, dim3(16, sg.n), dim3(256), 0, b->stream,
+                       reinterpret_cast<const uint4*>(h_dev), reinterpret_cast<uint4*>(b->d_buf), sg);
     BCHK(b, hipEventRecord(b->copied, b->stream));
     b->copy_pending = true;
 
@@ -589,7 +626,7 @@ int dfp_batch_project(dfp_batch* b, int n, dfp_plan* const* plans, double* const
             if (k - i == 1) {
                 if (hipError_t e = run_one(ls[i], st)) return e;
             } else {
-                const int ns = std::min((int)(k - i), b->n_par + 1);
+                const int ns = std::min({(int)(k - i), b->n_par + 1, (int)b->aux.size() + 1});
                 if (hipError_t e = hipEventRecord(b->ev_fork, st)) return e;
                 for (int q = 1; q < ns; ++q)
                     if (hipError_t e = hipStreamWaitEvent(b->aux[q - 1], b->ev_fork, 0)) return e;

@@ -266,7 +266,8 @@ int dfp_batch_set_occupancy(dfp_batch *batch, int x_per_cu, int z_per_cu, int st
 /* replay the launch sequence from hipGraphs keyed by its stage list */
 int dfp_batch_use_graphs(dfp_batch *batch, int enable);
 /* independent launches of one stage (different z splits or z kernels) run
- * side by side on up to 1 + aux_streams streams (0..3, default 3); callers
+ * side by side on up to 1 + aux_streams streams (0..3, default 3; the library
+ * takes no more than help, two in all); callers
  * that already overlap several batches on their own streams use 0 */
 int dfp_batch_set_parallel(dfp_batch *batch, int aux_streams);
 /* plans with x_bc_type = 1 are refused (DFP_E_UNSUPPORTED) */
