@@ -37,7 +37,7 @@
 
 #include <mutex>
 
-#include "dfp_internal.h"
+#include "fft_lds.h"
 
 using namespace dfp;
 
@@ -465,7 +465,11 @@ int dfp_batch_project(dfp_batch* b, int n, dfp_plan* const* plans, double* const
                           const std::vector<int>& Rs, const std::vector<size_t>& w, int inv) {
         // inverse: one launch per line length of the register kernel, one for the other lengths
         for (int R : kRadixList)
-            for (int M : {0, 16, 24, 32, 48, 64, 96, 128, 192, 256}) {
+            for (int M : {0
+#define DFP_XR_LINE(m) , m
+                          DFP_XR_LINES(DFP_XR_LINE)
+#undef DFP_XR_LINE
+                 }) {
                 std::vector<int> sel;
                 size_t lds = 0;
                 bool wide = false;  // a forward tile too large for two butterfly slots: the four-slot kernel

@@ -449,14 +449,25 @@ inline int twiddle_count(const FftDesc& d) {
 template <int M> struct XrSteps;
 template <> struct XrSteps<16> { static constexpr int e = 8, r[3] = {8, 2, 1}; };
 template <> struct XrSteps<24> { static constexpr int e = 12, r[3] = {12, 2, 1}; };
+template <> struct XrSteps<27> { static constexpr int e = 9, r[3] = {9, 3, 1}; };
 template <> struct XrSteps<32> { static constexpr int e = 8, r[3] = {8, 4, 1}; };
+template <> struct XrSteps<36> { static constexpr int e = 12, r[3] = {12, 3, 1}; };
 template <> struct XrSteps<48> { static constexpr int e = 12, r[3] = {12, 4, 1}; };
+template <> struct XrSteps<54> { static constexpr int e = 18, r[3] = {9, 6, 1}; };
 template <> struct XrSteps<64> { static constexpr int e = 8, r[3] = {8, 8, 1}; };
+template <> struct XrSteps<72> { static constexpr int e = 12, r[3] = {12, 6, 1}; };
+template <> struct XrSteps<81> { static constexpr int e = 9, r[3] = {9, 9, 1}; };
 template <> struct XrSteps<96> { static constexpr int e = 12, r[3] = {12, 4, 2}; };
+template <> struct XrSteps<108> { static constexpr int e = 12, r[3] = {12, 3, 3}; };
 template <> struct XrSteps<128> { static constexpr int e = 8, r[3] = {8, 4, 4}; };
+template <> struct XrSteps<144> { static constexpr int e = 12, r[3] = {12, 12, 1}; };
+template <> struct XrSteps<162> { static constexpr int e = 18, r[3] = {9, 9, 2}; };
 template <> struct XrSteps<192> { static constexpr int e = 12, r[3] = {12, 4, 4}; };
+template <> struct XrSteps<216> { static constexpr int e = 12, r[3] = {12, 6, 3}; };
 template <> struct XrSteps<256> { static constexpr int e = 8, r[3] = {8, 8, 4}; };
-#define DFP_XR_LINES(X) X(16) X(24) X(32) X(48) X(64) X(96) X(128) X(192) X(256)
+#define DFP_XR_LINES(X)                                                                            \
+    X(16) X(24) X(27) X(32) X(36) X(48) X(54) X(64) X(72) X(81) X(96) X(108) X(128) X(144) X(162)  \
+    X(192) X(216) X(256)
 // the steps for the host's twiddles; false if no kernel takes M-point lines
 inline bool xr_steps(int M, FftDesc& d) {
     d = FftDesc{};

@@ -1,24 +1,28 @@
-// Inverse x transform with the lines in registers, for lines of M = nxp/2 = 16,
-// 24, 32, 48, 64, 96, 128, 192 or 256 packed points.
+// Inverse x transform with the lines in registers, for the lines of M = nxp/2
+// packed points of DFP_XR_LINES (16 ... 256, 3-smooth).
 //
 // The staged kernel (xinv_body) takes every step through LDS: the gathered
 // modes, the C2R packing and each radix-4 or -2 stage are a pass over the tile
 // with a workgroup barrier on both sides, 12 accesses a point.  Here a thread
 // gathers the modes k and M-k of its column at all R sub-lines, so it undoes
 // the z split and packs Z[k] and Z[M-k] without an exchange; the lines are then
-// transformed in radix-8 (or -12), -4 and -2 steps, E = 8 (12) points a lane and
-// M/E, a power of two, neighbouring lanes a line, so each exchange stays within
-// a wave and needs no barrier; the last step stores phi (and P) from registers.
+// transformed in two or three radix steps, E = 8 to 18 points a lane and PT = M/E
+// neighbouring lanes a line (64/PT whole lines a wave), so each exchange stays
+// within a wave and needs no barrier; the last step stores phi (and P) from
+// registers.
 // Six accesses a point and two barriers a tile.  Bound by HBM with P (303 MB at
 // 256x192x256 in 62 us, 4.9 TB/s); measured, staged -> registers: 256x192x256
 // 74 -> 62 us, FP32 46 -> 30 and (phi read) 86 -> 67, 512x384x512 486 -> 402,
 // 256x257x256 86 -> 76, 64x64x64 7.5 -> 5.5.
 //
-// LDS position of point e of line l (column c of the tile): e ^ (e/8 mod 8) ^
-// lx(c), lx = c * (8/T) mod 8, which spreads the radix-8 step's stride-8
-// writes, and the packing's writes of one mode in T neighbouring lines, over
-// the banks; the reads run along the lines.
+// LDS position of point e of line l (column c of the tile): for M a multiple of
+// 8, e ^ (e/8 mod 8) ^ lx(c), lx = c * (8/T) mod 8, which spreads the first step's
+// strided writes, and the packing's writes of one mode in T neighbouring lines,
+// over the banks (the reads run along the lines); for other M, e in lines of an
+// odd pitch.
 #pragma once
+
+#include <algorithm>
 
 #include "fft_lds.h"
 
@@ -28,13 +32,22 @@ namespace dfp {
 template <typename C>
 constexpr int xr_threads(int M) { return M >= (sizeof(C) == sizeof(float2) ? 128 : 256) ? 512 : 256; }
 
+// pitch of the lines in LDS, and position of point e in its line
+template <int M>
+constexpr int xr_pitch() { return M % 8 == 0 ? M : M | 1; }
+template <int M>
+__device__ __forceinline__ int xr_pos(int e, int lx) {
+    if constexpr (M % 8 == 0) return e ^ (e >> 3 & 7) ^ lx;
+    else return e;
+}
+
 // One step of radix r and stride s on a line: this lane's 8/r butterflies.
 // out(n, z) takes the results of the last step, the others stay in the line.
 template <int M, int r, int s, typename C, typename Out>
 __device__ __forceinline__ void xr_step(C* line, int lx, int b0, const C* tws, bool act, Out out) {
     constexpr int NB = XrSteps<M>::e / r, PT = M / XrSteps<M>::e;
     constexpr bool kLast = r * s == M;
-    auto sw = [&](int e) { return e ^ (e >> 3 & 7) ^ lx; };
+    auto sw = [&](int e) { return xr_pos<M>(e, lx); };
     C v[NB][r];
 #pragma unroll
     for (int h = 0; h < NB; ++h)
@@ -66,7 +79,7 @@ __device__ __forceinline__ void xr_step(C* line, int lx, int b0, const C* tws, b
 template <typename C, int ACCUM, int R, int M>
 __device__ __forceinline__ void xinv_reg_body(const XPar<C>& q, int bx, int j, unsigned char* smem_raw) {
     constexpr int NT = xr_threads<C>(M);
-    constexpr int H = M / 2, E = XrSteps<M>::e, PT = M / E;
+    constexpr int H = M / 2, KI = (M + 1) / 2, E = XrSteps<M>::e, PT = M / E, LD = xr_pitch<M>();
     constexpr int GI = R <= 4 ? 4 / R : 1;  // gathered items (mode pair, column) per thread
     constexpr int r0 = XrSteps<M>::r[0], r1 = XrSteps<M>::r[1], r2 = XrSteps<M>::r[2];
     constexpr int n0 = M / r0 * (r0 - 1), n1 = r2 > 1 ? M / (r0 * r1) * (r1 - 1) : 0;  // twiddles of all steps but the last
@@ -75,20 +88,20 @@ __device__ __forceinline__ void xinv_reg_body(const XPar<C>& q, int bx, int j, u
     const int nz2 = g.nzp / R;
     const int T = q.T, nl = R * T, k0 = bx * T;
     const int tid = threadIdx.x;
-    C* A = reinterpret_cast<C*>(smem_raw);  // nl * M
-    C* tws = A + nl * M;                    // step twiddles
+    C* A = reinterpret_cast<C*>(smem_raw);  // nl lines
+    C* tws = A + nl * LD;                   // step twiddles
     C* rtl = tws + n0 + n1;                 // packing twiddles, M+1
     C* tzl = rtl + M + 1;                   // this tile's last z stage twiddles, T*(R-1)
     const int swm = T < 8 ? 8 / T : 1;
 
     // a periodic y's duplicate row nym-1 reads row 0 (projection.f90:350-354)
     const int js = (g.ybc == 0 && j == g.nym - 1) ? 0 : j;
-    const int nitems = H * T;
+    const int nitems = KI * T;
     const long plane = (long)g.nym * nz2;
-    // item: column c and modes (k, M-k); k = 0 takes (0, M), and in xm the mode M/2 that pairs with itself
+    // item: column c and modes (k, M-k); k = 0 takes (0, M), and, of an even M, in xm the mode M/2 that pairs with itself
     C xa[GI][R], xb[GI][R], xm[R];
     const auto base = gptr(q.spec) + (long)js * nz2 + k0;
-    if (tid < T) {
+    if (M % 2 == 0 && tid < T) {
 #pragma unroll
         for (int u = 0; u < R; ++u) xm[u] = gld<C>(base + ((long)H * R + u) * plane + tid);
     }
@@ -128,36 +141,38 @@ __device__ __forceinline__ void xinv_reg_body(const XPar<C>& q, int bx, int j, u
             if (it < nitems) {
                 const int k = (int)q.div_t.div((uint32_t)it), c = it - k * T;
                 const int lx = c * swm & 7;
-                auto sw = [&](int e) { return e ^ (e >> 3 & 7) ^ lx; };
+                auto sw = [&](int e) { return xr_pos<M>(e, lx); };
                 undo_z(xa[i], c);
                 undo_z(xb[i], c);
                 const C wa = rtl[k], wb = rtl[M - k];
-                C* const Z = A + c * M;
+                C* const Z = A + c * LD;
 #pragma unroll
-                for (int t = 0; t < R; ++t) Z[t * T * M + sw(k)] = pack(xa[i][t], xb[i][t], wa);
+                for (int t = 0; t < R; ++t) Z[t * T * LD + sw(k)] = pack(xa[i][t], xb[i][t], wa);
                 if (k > 0) {
 #pragma unroll
-                    for (int t = 0; t < R; ++t) Z[t * T * M + sw(M - k)] = pack(xb[i][t], xa[i][t], wb);
+                    for (int t = 0; t < R; ++t) Z[t * T * LD + sw(M - k)] = pack(xb[i][t], xa[i][t], wb);
                 }
             }
         }
-        if (tid < T) {
+        if (M % 2 == 0 && tid < T) {
             const int lx = tid * swm & 7;
             undo_z(xm, tid);
             const C w = rtl[H];
 #pragma unroll
-            for (int t = 0; t < R; ++t) A[(t * T + tid) * M + (H ^ (H >> 3 & 7) ^ lx)] = pack(xm[t], xm[t], w);
+            for (int t = 0; t < R; ++t) A[(t * T + tid) * LD + xr_pos<M>(H, lx)] = pack(xm[t], xm[t], w);
         }
     }
     __syncthreads();
 
-    // this lane's line: PT neighbouring lanes of one wave
-    const int l0 = tid / PT, b0 = tid - l0 * PT;
-    const bool act = l0 < nl;
+    // this lane's line: PT neighbouring lanes of one wave (lanes past a wave's whole lines repeat the last one's)
+    constexpr int LW = 64 / PT;
+    const int lane = tid & 63, lw = min(lane / PT, LW - 1);
+    const int l0 = (tid >> 6) * LW + lw, b0 = min(lane - lw * PT, PT - 1);
+    const bool act = l0 < nl && lane < LW * PT;
     const int l = min(l0, nl - 1);
     const int t = (int)q.div_t.div((uint32_t)l), c = l - t * T;
     const int k = k0 + c + t * nz2, lx = c * swm & 7;
-    C* const line = A + l * M;
+    C* const line = A + l * LD;
     const long pr_j = (long)(g.nxg - 1), pr_k = pr_j * g.nym;
     const auto rr = gptr(q.rhs) + (long)j * pr_j + k * pr_k;
     double2 ph[E];
@@ -249,7 +264,7 @@ __device__ __forceinline__ void xinv_reg_body(const XPar<C>& q, int bx, int j, u
 template <typename C, int M>
 constexpr size_t xr_lds(int R, int T) {
     constexpr int r0 = XrSteps<M>::r[0], r1 = XrSteps<M>::r[1], r2 = XrSteps<M>::r[2];
-    return sizeof(C) * ((size_t)R * T * M + M / r0 * (r0 - 1) + (r2 > 1 ? M / (r0 * r1) * (r1 - 1) : 0) + M + 1 +
+    return sizeof(C) * ((size_t)R * T * xr_pitch<M>() + M / r0 * (r0 - 1) + (r2 > 1 ? M / (r0 * r1) * (r1 - 1) : 0) + M + 1 +
                         (size_t)T * (R - 1));
 }
 
@@ -288,9 +303,12 @@ template <typename C>
 size_t xr_lds_any(int M, int R, int T) {
     if (R != 1 && R != 2 && R != 4 && R != 8) return 0;
     if ((long)R * T * M > 8 * xr_threads<C>(M)) return 0;
+    // the items of the gather, and the lines of the waves
+    if ((long)(M + 1) / 2 * T > (long)std::max(4 / R, 1) * xr_threads<C>(M)) return 0;
     switch (M) {
-#define DFP_XR_CASE(m) \
-    case m: return xr_lds<C, m>(R, T);
+#define DFP_XR_CASE(m)                                                                                       \
+    case m:                                                                                                  \
+        return R * T <= 64 / (m / XrSteps<m>::e) * (xr_threads<C>(m) / 64) ? xr_lds<C, m>(R, T) : 0;
         DFP_XR_LINES(DFP_XR_CASE)
 #undef DFP_XR_CASE
     }

@@ -1,5 +1,5 @@
-"""The inverse x kernel with the lines in registers (nxp = 2^n and 3 2^n from 32
-to 512; z splits 1, 2, 4, 8): each line length with each split, tiles of one
+"""The inverse x kernel with the lines in registers (nxp/2 = 2^a 3^b from 16 to
+256; z splits 1, 2, 4, 8): each line length with each split, tiles of one
 column, of a column count that is no power of two and partial ones, a single
 y row, the duplicate row of a periodic y, z walls, P with its ghosts.
 
@@ -29,17 +29,19 @@ def _check(g, tuning=None, precision=dfp.DFP_FP64, bar=1e-12):
         assert rel_linf(a, b) <= bar, lab
 
 
-@pytest.mark.parametrize("nxp", [32, 48, 64, 96, 128, 192, 256, 384, 512])
+@pytest.mark.parametrize("nxp", [32, 48, 54, 64, 72, 96, 108, 128, 144, 162, 192, 216, 256, 288, 324, 384, 432, 512])
 @pytest.mark.parametrize("nym,nzp,R,T", [(1, 16, 1, 0), (3, 16, 2, 0), (9, 16, 4, 0), (4, 24, 8, 0), (6, 12, 4, 3),
                                          (5, 16, 4, 1), (7, 6, 1, 2)])
 def test_lines_in_registers_match_oracle(nxp, nym, nzp, R, T):
+    if R * T * (nxp // 2) > 2048:
+        pytest.skip("a plan takes no tile of that many points")
     print(f"{nxp}x{nym}x{nzp}, split {R}, columns {T}", flush=True)
     g = make_grid(nxp, nym, nzp, 1.5)
     _check(g, (R, T, 0, 0))
     _check(g, (R, T, 0, 0), dfp.DFP_FP32_REFINE, 1e-10)
 
 
-@pytest.mark.parametrize("nxp", [32, 96, 128, 512])
+@pytest.mark.parametrize("nxp", [32, 54, 96, 108, 128, 162, 512])
 def test_lines_in_registers_periodic_y_and_z_walls(nxp):
     print(f"nxp {nxp}", flush=True)
     _check(dfp.periodic_y_grid(nxp, 9, 16))
@@ -52,7 +54,8 @@ def test_batch_of_register_lines_equals_single_plans(precision):
 
     from dfp.batch import Batch, Case
 
-    sizes = [(32, 5, 12), (64, 7, 16), (128, 4, 24), (256, 3, 16), (512, 2, 16), (48, 6, 12), (96, 5, 24), (36, 4, 12)]
+    sizes = [(32, 5, 12), (64, 7, 16), (128, 4, 24), (256, 3, 16), (512, 2, 16), (48, 6, 12), (96, 5, 24), (36, 4, 12), (54, 3, 16),
+             (162, 4, 16), (324, 2, 12), (432, 2, 12)]
     batch, cases, singles = Batch(max_cases=len(sizes)), [], []
     for n in sizes:
         g = make_grid(*n, 1.5)
