@@ -22,8 +22,6 @@
 // odd pitch.
 #pragma once
 
-#include <algorithm>
-
 #include "fft_lds.h"
 
 namespace dfp {
@@ -31,6 +29,10 @@ namespace dfp {
 // tiles of up to 8 NT points: 2048, or 4096 where the plan's tiles are that large (x_columns)
 template <typename C>
 constexpr int xr_threads(int M) { return M >= (sizeof(C) == sizeof(float2) ? 128 : 256) ? 512 : 256; }
+
+// z splits with a kernel, and the items (mode pair, column) that a thread gathers of a tile of up to 8 NT points
+constexpr bool xr_split(int R) { return R <= 4 || R == 6 || R == 8 || R == 9; }
+constexpr int xr_items(int R) { return (4 + R - 1) / R; }
 
 // pitch of the lines in LDS, and position of point e in its line
 template <int M>
@@ -80,7 +82,7 @@ template <typename C, int ACCUM, int R, int M>
 __device__ __forceinline__ void xinv_reg_body(const XPar<C>& q, int bx, int j, unsigned char* smem_raw) {
     constexpr int NT = xr_threads<C>(M);
     constexpr int H = M / 2, KI = (M + 1) / 2, E = XrSteps<M>::e, PT = M / E, LD = xr_pitch<M>();
-    constexpr int GI = R <= 4 ? 4 / R : 1;  // gathered items (mode pair, column) per thread
+    constexpr int GI = xr_items(R);  // gathered items (mode pair, column) per thread
     constexpr int r0 = XrSteps<M>::r[0], r1 = XrSteps<M>::r[1], r2 = XrSteps<M>::r[2];
     constexpr int n0 = M / r0 * (r0 - 1), n1 = r2 > 1 ? M / (r0 * r1) * (r1 - 1) : 0;  // twiddles of all steps but the last
     __shared__ double wsum[NT / 64];
@@ -301,10 +303,10 @@ kb_irfft_xr(const XPar<C>* __restrict__ cs, const int* __restrict__ off, const i
 // LDS of the kernel for a plan's tile of T columns, 0 if it does not take the plan's lines
 template <typename C>
 size_t xr_lds_any(int M, int R, int T) {
-    if (R != 1 && R != 2 && R != 4 && R != 8) return 0;
+    if (!xr_split(R)) return 0;
     if ((long)R * T * M > 8 * xr_threads<C>(M)) return 0;
     // the items of the gather, and the lines of the waves
-    if ((long)(M + 1) / 2 * T > (long)std::max(4 / R, 1) * xr_threads<C>(M)) return 0;
+    if ((long)(M + 1) / 2 * T > (long)xr_items(R) * xr_threads<C>(M)) return 0;
     switch (M) {
 #define DFP_XR_CASE(m)                                                                                       \
     case m:                                                                                                  \
@@ -319,7 +321,7 @@ size_t xr_lds_any(int M, int R, int T) {
 template <typename C, int ACCUM, int R>
 hipError_t launch_xinv_reg_batch(hipStream_t s, int M, const XPar<C>* cs, const int* off, const int* idx,
                                  const int* nc, int grid, size_t lds) {
-    if constexpr (R == 1 || R == 2 || R == 4 || R == 8) {
+    if constexpr (xr_split(R)) {
         auto go = [&](auto m) {
             constexpr int MV = decltype(m)::value;
             const auto k = kb_irfft_xr<C, ACCUM, R, MV>;
@@ -340,7 +342,7 @@ hipError_t launch_xinv_reg_batch(hipStream_t s, int M, const XPar<C>* cs, const 
 // false: the plan's lines or tile are not this kernel's
 template <typename C, int ACCUM, int R>
 bool launch_xinv_reg(hipStream_t s, const XPar<C>& q, dim3 grid) {
-    if constexpr (R == 1 || R == 2 || R == 4 || R == 8) {
+    if constexpr (xr_split(R)) {
         if (!q.twr || xr_lds_any<C>(q.fd.n, R, q.T) == 0) return false;
         auto go = [&](auto m) {
             constexpr int M = decltype(m)::value;

@@ -1,5 +1,5 @@
 """The inverse x kernel with the lines in registers (nxp/2 = 2^a 3^b from 16 to
-256; z splits 1, 2, 4, 8): each line length with each split, tiles of one
+256; z splits 1, 2, 3, 4, 6, 8, 9): each line length with each split, tiles of one
 column, of a column count that is no power of two and partial ones, a single
 y row, the duplicate row of a periodic y, z walls, P with its ghosts.
 
@@ -31,7 +31,8 @@ def _check(g, tuning=None, precision=dfp.DFP_FP64, bar=1e-12):
 
 @pytest.mark.parametrize("nxp", [32, 48, 54, 64, 72, 96, 108, 128, 144, 162, 192, 216, 256, 288, 324, 384, 432, 512])
 @pytest.mark.parametrize("nym,nzp,R,T", [(1, 16, 1, 0), (3, 16, 2, 0), (9, 16, 4, 0), (4, 24, 8, 0), (6, 12, 4, 3),
-                                         (5, 16, 4, 1), (7, 6, 1, 2)])
+                                         (5, 16, 4, 1), (7, 6, 1, 2),
+                                         (4, 12, 3, 0), (3, 24, 6, 0), (5, 27, 9, 0)])
 def test_lines_in_registers_match_oracle(nxp, nym, nzp, R, T):
     if R * T * (nxp // 2) > 2048:
         pytest.skip("a plan takes no tile of that many points")
