@@ -802,7 +802,14 @@ int dfp_plan_create_tuned(const dfp_grid* g, int precision, int device, const df
     FftDesc xrd{};
     const bool xr = !dct && xr_steps(G.nxp / 2, xrd);  // the inverse x lines in registers
     const size_t o_xr = tw.size();
-    if (xr) stage_twiddles(xrd, tw);
+    // their step twiddles are among the packing's (w_2M^k, k <= M) and their negatives
+    for (int st = 0, n = xrd.n; xr && st < xrd.nst; n /= xrd.rad[st++])
+        for (int e = 0; e < n / xrd.rad[st]; ++e)
+            for (int u = 1; u < xrd.rad[st]; ++u) {
+                const int k = e * u * (G.nxp / n), M = G.nxp / 2;
+                const double2 w = tw[o_r2c + (k <= M ? k : k - M)];
+                tw.push_back(k <= M ? w : make_double2(-w.x, -w.y));
+            }
     if (hipMalloc(&p->d_tw, sizeof(double2) * tw.size()) != hipSuccess) return bail(DFP_E_NOMEM);
     if (hipMemcpy(p->d_tw, tw.data(), sizeof(double2) * tw.size(), hipMemcpyHostToDevice) != hipSuccess)
         return bail(DFP_E_HIP);

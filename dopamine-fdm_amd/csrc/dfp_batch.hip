@@ -164,7 +164,7 @@ int bfail(dfp_batch* b, int code, const char* fmt, ...) {
 struct Launch {
     enum Kind { XF, XI, ZFB, ZFUSED, M00, SAVE, CORR } kind;
     int f32;      // spectrum precision
-    int mode;     // x forward mode, ACCUM + 16 M (register lines) for the inverse, zplane_wide
+    int mode;     // x forward mode or ACCUM, + 16 M (register lines); zplane_wide
     int R;        // z-split radix (x kernels)
     size_t tab;   // offset of the case records
     int list;     // case list
@@ -463,7 +463,7 @@ int dfp_batch_project(dfp_batch* b, int n, dfp_plan* const* plans, double* const
     // for its fused and split members
     auto x_launches = [&](Launch::Kind k, int f32, int mode, size_t tab, const std::vector<int>& recs,
                           const std::vector<int>& Rs, const std::vector<size_t>& w, int inv) {
-        // inverse: one launch per line length of the register kernel, one for the other lengths
+        // one launch per line length of the register kernels, one for the other lengths
         for (int R : kRadixList)
             for (int M : {0
 #define DFP_XR_LINE(m) , m
@@ -476,7 +476,7 @@ int dfp_batch_project(dfp_batch* b, int n, dfp_plan* const* plans, double* const
                 for (int a : recs) {
                     if (Rs[a] != R) continue;
                     const dfp_plan* p = plans[f32 ? i32[a] : i64[a]];
-                    const size_t reg = inv ? xinv_reg_lds(p, f32) : 0;
+                    const size_t reg = x_reg_lds(p, inv, mode, f32);
                     if (M != (reg ? p->fx.n : 0)) continue;
                     sel.push_back(a);
                     lds = std::max(lds, reg ? reg : x_lds_bytes(p, inv, f32));
@@ -583,10 +583,10 @@ int dfp_batch_project(dfp_batch* b, int n, dfp_plan* const* plans, double* const
             hipError_t e = hipSuccess;
             switch (l.kind) {
                 case Launch::XF:
-                    e = l.f32 ? launch_xfwd_batch(st, l.R, l.mode, reinterpret_cast<const XPar<float2>*>(D + l.tab),
-                                                  o, ix, nc, gx, l.lds)
-                              : launch_xfwd_batch(st, l.R, l.mode, reinterpret_cast<const XPar<double2>*>(D + l.tab),
-                                                  o, ix, nc, gx, l.lds);
+                    e = l.f32 ? launch_xfwd_batch(st, l.R, l.mode & 15, reinterpret_cast<const XPar<float2>*>(D + l.tab),
+                                                  o, ix, nc, gx, l.lds, l.mode >> 4)
+                              : launch_xfwd_batch(st, l.R, l.mode & 15, reinterpret_cast<const XPar<double2>*>(D + l.tab),
+                                                  o, ix, nc, gx, l.lds, l.mode >> 4);
                     break;
                 case Launch::XI:
                     e = l.f32 ? launch_xinv_batch(st, l.R, l.mode & 15, reinterpret_cast<const XPar<float2>*>(D + l.tab),

@@ -13,12 +13,14 @@ template <int R, typename C>
 hipError_t launch_xinv_r(hipStream_t s, int accum, const XPar<C>& q, dim3 grid, size_t lds);
 template <int R, typename C>
 hipError_t launch_xfwd_batch_r(hipStream_t s, int mode, const XPar<C>* cs, const int* off, const int* idx,
-                               const int* nc, int grid, size_t lds);
+                               const int* nc, int grid, size_t lds, int M);
 template <int R, typename C>
 hipError_t launch_xinv_batch_r(hipStream_t s, int accum, const XPar<C>* cs, const int* off, const int* idx,
                                const int* nc, int grid, size_t lds, int M);
 template <typename C>
 size_t xr_lds_any(int M, int R, int T);
+template <typename C>
+size_t xf_lds_any(int M, int R, int T);
 template <int R>
 hipError_t launch_xdct_fwd_r(hipStream_t s, int mode, const XPar<double2>& q, dim3 grid, size_t lds);
 template <int R>
@@ -113,8 +115,9 @@ static size_t x_lds_bytes_t(const dfp_plan* p, int T, int f32) {
 // of a plan's forward (inv = 0) or inverse (inv = 1) x kernel
 size_t x_lds_bytes(const dfp_plan* p, int inv, int f32) { return x_lds_bytes_t(p, inv ? p->tk_xi : p->tk_x, f32); }
 
-size_t xinv_reg_lds(const dfp_plan* p, int f32) {
-    if (!p->tw_xr) return 0;
+size_t x_reg_lds(const dfp_plan* p, int inv, int mode, int f32) {
+    if (!p->tw_xr || (!inv && (f32 || mode != 1))) return 0;
+    if (!inv) return xf_lds_any<double2>(p->fx.n, p->zr, p->tk_x);
     return f32 ? xr_lds_any<float2>(p->fx.n, p->zr, p->tk_xi) : xr_lds_any<double2>(p->fx.n, p->zr, p->tk_xi);
 }
 
@@ -154,15 +157,15 @@ static hipError_t xinv_any(int R, hipStream_t s, int accum, const XPar<C>& q, di
 
 template <typename C>
 hipError_t launch_xfwd_batch(hipStream_t s, int R, int mode, const XPar<C>* cs, const int* off, const int* idx,
-                             const int* nc, int grid, size_t lds) {
-#define DFP_CALL(RV) launch_xfwd_batch_r<RV, C>(s, mode, cs, off, idx, nc, grid, lds)
+                             const int* nc, int grid, size_t lds, int M) {
+#define DFP_CALL(RV) launch_xfwd_batch_r<RV, C>(s, mode, cs, off, idx, nc, grid, lds, M)
     DFP_R_SWITCH(R, DFP_CALL)
 #undef DFP_CALL
 }
 template hipError_t launch_xfwd_batch<double2>(hipStream_t, int, int, const XPar<double2>*, const int*, const int*,
-                                               const int*, int, size_t);
+                                               const int*, int, size_t, int);
 template hipError_t launch_xfwd_batch<float2>(hipStream_t, int, int, const XPar<float2>*, const int*, const int*,
-                                              const int*, int, size_t);
+                                              const int*, int, size_t, int);
 
 template <typename C>
 hipError_t launch_xinv_batch(hipStream_t s, int R, int accum, const XPar<C>* cs, const int* off, const int* idx,

@@ -452,13 +452,16 @@ __global__ void __launch_bounds__(kXThreads) kb_irfft_x(const XPar<C>* __restric
 
 
 }  // namespace dfp
-#include "k_xinv_reg.h"
+#include "k_xfwd_reg.h"
 namespace dfp {
 
 // launches of the kernels above for one z-split radix R (instantiated per R
 // in k_xfft_r<R>.hip, so the radices compile in parallel)
 template <int R, typename C>
 hipError_t launch_xfwd_r(hipStream_t s, int mode, const XPar<C>& q, dim3 grid, size_t lds) {
+    if constexpr (sizeof(C) == sizeof(double2)) {
+        if (mode == 1 && launch_xfwd_reg<R>(s, q, grid)) return hipGetLastError();
+    }
     auto go = [&](auto k) { hipLaunchKernelGGL(k, grid, dim3(kXThreads), lds, s, q); };
     if constexpr (sizeof(C) == sizeof(float2)) {
         if (xfwd_wide(q.fd, R, q.T)) {
@@ -502,7 +505,10 @@ hipError_t launch_xinv_r(hipStream_t s, int accum, const XPar<C>& q, dim3 grid, 
 // forward tiles too large for two butterfly slots per thread (FP32 only)
 template <int R, typename C>
 hipError_t launch_xfwd_batch_r(hipStream_t s, int mode, const XPar<C>* cs, const int* off, const int* idx,
-                               const int* nc, int grid, size_t lds) {
+                               const int* nc, int grid, size_t lds, int M) {
+    if constexpr (sizeof(C) == sizeof(double2)) {
+        if (M > 0) return launch_xfwd_reg_batch<R>(s, M, cs, off, idx, nc, grid, lds);
+    }
     auto go = [&](auto k) {
         hipLaunchKernelGGL(k, dim3(resident_grid(k, grid, kXThreads, lds)), dim3(kXThreads), lds, s, cs, off, idx, nc);
     };
@@ -559,15 +565,16 @@ hipError_t launch_xinv_batch_r(hipStream_t s, int accum, const XPar<C>* cs, cons
 #define DFP_INSTANTIATE_XFFT(RV)                                                                                   \
     namespace dfp {                                                                                                \
     template size_t xr_lds_any<double2>(int, int, int);                                                            \
+    template size_t xf_lds_any<double2>(int, int, int);                                                            \
     template size_t xr_lds_any<float2>(int, int, int);                                                             \
     template hipError_t launch_xfwd_r<RV, double2>(hipStream_t, int, const XPar<double2>&, dim3, size_t);         \
     template hipError_t launch_xfwd_r<RV, float2>(hipStream_t, int, const XPar<float2>&, dim3, size_t);           \
     template hipError_t launch_xinv_r<RV, double2>(hipStream_t, int, const XPar<double2>&, dim3, size_t);         \
     template hipError_t launch_xinv_r<RV, float2>(hipStream_t, int, const XPar<float2>&, dim3, size_t);           \
     template hipError_t launch_xfwd_batch_r<RV, double2>(hipStream_t, int, const XPar<double2>*, const int*,      \
-                                                         const int*, const int*, int, size_t);                                 \
+                                                         const int*, const int*, int, size_t, int);                            \
     template hipError_t launch_xfwd_batch_r<RV, float2>(hipStream_t, int, const XPar<float2>*, const int*,        \
-                                                        const int*, const int*, int, size_t);                                  \
+                                                        const int*, const int*, int, size_t, int);                             \
     template hipError_t launch_xinv_batch_r<RV, double2>(hipStream_t, int, const XPar<double2>*, const int*,      \
                                                          const int*, const int*, int, size_t, int);                            \
     template hipError_t launch_xinv_batch_r<RV, float2>(hipStream_t, int, const XPar<float2>*, const int*,        \

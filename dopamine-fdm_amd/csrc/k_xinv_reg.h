@@ -43,9 +43,15 @@ __device__ __forceinline__ int xr_pos(int e, int lx) {
     else return e;
 }
 
+// orders a wave's LDS accesses across the call, for exchanges among its lanes (which LDS serves in order)
+__device__ __forceinline__ void wave_exchange() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // One step of radix r and stride s on a line: this lane's 8/r butterflies.
 // out(n, z) takes the results of the last step, the others stay in the line.
-template <int M, int r, int s, typename C, typename Out>
+template <int SIGN, int M, int r, int s, typename C, typename Out>
 __device__ __forceinline__ void xr_step(C* line, int lx, int b0, const C* tws, bool act, Out out) {
     constexpr int NB = XrSteps<M>::e / r, PT = M / XrSteps<M>::e;
     constexpr bool kLast = r * s == M;
@@ -55,25 +61,23 @@ __device__ __forceinline__ void xr_step(C* line, int lx, int b0, const C* tws, b
     for (int h = 0; h < NB; ++h)
 #pragma unroll
         for (int t = 0; t < r; ++t) v[h][t] = line[sw(b0 + h * PT + t * (M / r))];
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
+    wave_exchange();
 #pragma unroll
     for (int h = 0; h < NB; ++h) {
         const int b = b0 + h * PT;
         const int p = b / s, q = b - p * s;
-        dft_reg<1, r>(v[h]);
+        dft_reg<SIGN, r>(v[h]);
 #pragma unroll
         for (int u = 0; u < r; ++u) {
             if constexpr (kLast) {
                 out(h * r + u, q + s * u, v[h][u]);
             } else {
-                const C z = u == 0 ? v[h][0] : cmulc(v[h][u], tws[p * (r - 1) + (u - 1)]);
+                const C z = u == 0 ? v[h][0] : twiddle<SIGN>(v[h][u], tws[p * (r - 1) + (u - 1)]);
                 if (act) line[sw(q + s * (r * p + u))] = z;
             }
         }
     }
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
+    wave_exchange();
 }
 
 // As xinv_body: last inverse z stage, C2R, phi (ACCUM: added to phi) with its
@@ -184,12 +188,12 @@ __device__ __forceinline__ void xinv_reg_body(const XPar<C>& q, int bx, int j, u
         at[o] = 2 * n;
         ph[o] = make_double2((double)z.x * q.scale, (double)z.y * q.scale);
     };
-    xr_step<M, r0, 1>(line, lx, b0, tws, act, none);
+    xr_step<1, M, r0, 1>(line, lx, b0, tws, act, none);
     if constexpr (r2 > 1) {
-        xr_step<M, r1, r0>(line, lx, b0, tws + n0, act, none);
-        xr_step<M, r2, r0 * r1>(line, lx, b0, tws, act, take);
+        xr_step<1, M, r1, r0>(line, lx, b0, tws + n0, act, none);
+        xr_step<1, M, r2, r0 * r1>(line, lx, b0, tws, act, take);
     } else {
-        xr_step<M, r1, r0>(line, lx, b0, tws, act, take);
+        xr_step<1, M, r1, r0>(line, lx, b0, tws, act, take);
     }
 
     double psum = 0.0;

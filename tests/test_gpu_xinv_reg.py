@@ -73,3 +73,28 @@ def test_batch_of_register_lines_equals_single_plans(precision):
     for n, c, s in zip(sizes, cases, singles):
         for lab, a, b in zip(("U", "V", "W", "P", "phi"), (c.U, c.V, c.W, c.P, c.rhs), s):
             assert torch.equal(a, b), (n, lab)
+
+
+@pytest.mark.parametrize("nxp", [32, 54, 72, 108, 128, 162, 192, 324, 512])
+@pytest.mark.parametrize("nym,nzp,R,T", [(3, 16, 2, 0), (9, 16, 4, 0), (1, 16, 1, 0), (4, 24, 8, 0), (5, 27, 9, 0)])
+def test_solve_lines_in_registers_match_oracle(nxp, nym, nzp, R, T):
+    """The right-hand side's forward transform in registers: phi of a solve, alone and in a batch (equal bits)."""
+    import numpy as np
+    import torch
+
+    from dfp.batch import Batch, Case
+
+    print(f"solve {nxp}x{nym}x{nzp}, split {R}", flush=True)
+    g = make_grid(nxp, nym, nzp, 1.5)
+    U, V, W, P, rhs = fields(g, 5, 0.1)
+    o = [a.copy(order="F") for a in (U, V, W, P, rhs)]
+    oracle_project(g, *o, DT, C3, save_p=False)
+    plan = dfp.Plan(g, tuning=(R, T, 0, 0))
+    plan.divergence(U, V, W, rhs)
+    b = rhs.copy(order="F")
+    plan.solve(rhs)
+    assert rel_linf(rhs, o[4]) <= 1e-12
+    dev = torch.from_numpy(b.T.copy()).cuda()
+    Batch(max_cases=1).project([Case(plan, None, None, None, dev)], solve_only=True)
+    assert np.array_equal(dev.cpu().numpy().T, rhs)
+    plan.close()
