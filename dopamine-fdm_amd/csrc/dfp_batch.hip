@@ -77,7 +77,22 @@ struct Layout {
     size_t total;
 };
 
-constexpr int kMaxLists = 512;  // case lists per call (each launch reads one)
+// Case lists of one call (each launch reads one), at most: the lists of a
+// stage part its cases, by z split (forward FP32), by z split and line length
+// (inverse, and FP64 forward) or by z kernel, and every solve, the first one
+// and those of the sweeps, has its own.
+constexpr int kSplits = sizeof kRadixList / sizeof *kRadixList;
+#define DFP_ONE(...) +1
+constexpr int kXLists = kSplits * (1 DFP_XR_LINES(DFP_ONE));
+// register planes of one or two passes, narrow or wide; the streaming kernel, two-pass or staged; the LDS-resident one
+constexpr int kZLists = 4 * (0 DFP_ZP_SHORT(DFP_ONE) DFP_ZP_LONG(DFP_ONE)) + (1 DFP_ZV_LIST(DFP_ONE)) + 1;
+#undef DFP_ONE
+int max_lists(int cap) {
+    const int f = std::min(cap, kSplits), x = std::min(cap, kXLists), z = std::min(cap, kZLists);
+    const int fp32 = (1 + kMaxSweepStages) * (f + 1 + z + x) + 1;  // 1: the (0,0) modes; P
+    const int fp64 = x + z + x;
+    return fp32 + fp64 + 1;  // the correction
+}
 
 size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
@@ -101,8 +116,8 @@ Layout layout_for(int cap) {
     L.s32 = take(sizeof(SPar) * cap);
     L.c = take(sizeof(CPar) * cap);
     // list counts, then the lists: offsets (count + 1) and record indices (count)
-    L.counts = take(sizeof(int) * kMaxLists);
-    L.lists = take(sizeof(int) * (size_t)kMaxLists * (2 * cap + 1));
+    L.counts = take(sizeof(int) * max_lists(cap));
+    L.lists = take(sizeof(int) * (size_t)max_lists(cap) * (2 * cap + 1));
     L.total = o;
     return L;
 }
@@ -438,9 +453,10 @@ int dfp_batch_project(dfp_batch* b, int n, dfp_plan* const* plans, double* const
     // positions, so a launch (and a graph that captured it) reads the same
     // addresses whatever the list's length
     int nlists = 0;
+    const int most_lists = max_lists(b->cap);
     bool overflow = false;
     auto make_list = [&](const std::vector<int>& recs, const std::vector<size_t>& w) {
-        if (nlists >= kMaxLists) { overflow = true; return 0; }
+        if (nlists >= most_lists) { overflow = true; return 0; }
         int* o = pool + (size_t)nlists * list_stride;
         int* ix = o + b->cap + 1;
         o[0] = 0;

@@ -302,6 +302,10 @@ bool z_two_pass(int n, int& n1, int& n2);
 constexpr int kZvPlane = 1 << 16;
 int z_variant(const dfp_plan* p);
 
+// the streaming kernel's two-pass factorizations (N1, N2) with N1 * N2 = nzp / R;
+// others use the staged transform
+#define DFP_ZV_LIST(X) X(2, 4) X(3, 4) X(2, 8) X(3, 8) X(4, 8) X(9, 4) X(6, 8) X(8, 8) X(9, 8) X(12, 8) X(16, 8)
+
 // (N1, N2, rows per pass): n = N1*N2 modes per row; the rows per pass are a
 // multiple of N2, so that a thread's items fill its registers
 #define DFP_ZP_SHORT(X) X(2, 4, 8) X(3, 4, 8) X(2, 8, 8) X(9, 2, 8) X(3, 8, 8) X(9, 3, 9) X(4, 8, 8)

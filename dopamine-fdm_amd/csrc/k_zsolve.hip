@@ -529,10 +529,6 @@ __device__ __forceinline__ void zbwd2_body(const ZPar<C>& zp, int blk, unsigned 
     }
 }
 
-// the two-pass factorizations (N1, N2) with N1 * N2 = nzp / R; others use the
-// staged transform
-#define DFP_ZV_LIST(X) X(2, 4) X(3, 4) X(2, 8) X(3, 8) X(4, 8) X(9, 4) X(6, 8) X(8, 8) X(9, 8) X(12, 8) X(16, 8)
-
 bool z_two_pass(int n, int& n1, int& n2) {
 #define DFP_ZV_TRY(a, c) \
     if (a * c == n) { n1 = a; n2 = c; return true; }
