@@ -78,12 +78,12 @@ struct Layout {
 };
 
 // Case lists of one call (each launch reads one), at most: the lists of a
-// stage part its cases, by z split (forward FP32), by z split and line length
-// (inverse, and FP64 forward) or by z kernel, and every solve, the first one
-// and those of the sweeps, has its own.
+// stage part its cases, by z split (forward FP32), by z split and group of
+// line lengths (inverse, and FP64 forward) or by z kernel, and every solve, the
+// first one and those of the sweeps, has its own.
 constexpr int kSplits = sizeof kRadixList / sizeof *kRadixList;
 #define DFP_ONE(...) +1
-constexpr int kXLists = kSplits * (1 DFP_XR_LINES(DFP_ONE));
+constexpr int kXLists = kSplits * kXrGroups;
 // register planes of one or two passes, narrow or wide; the streaming kernel, two-pass or staged; the LDS-resident one
 constexpr int kZLists = 4 * (0 DFP_ZP_SHORT(DFP_ONE) DFP_ZP_LONG(DFP_ONE)) + (1 DFP_ZV_LIST(DFP_ONE)) + 1;
 #undef DFP_ONE
@@ -179,7 +179,7 @@ int bfail(dfp_batch* b, int code, const char* fmt, ...) {
 struct Launch {
     enum Kind { XF, XI, ZFB, ZFUSED, M00, SAVE, CORR } kind;
     int f32;      // spectrum precision
-    int mode;     // x forward mode or ACCUM, + 16 M (register lines); zplane_wide
+    int mode;     // x forward mode or ACCUM, + 16 times the group of register lines; zplane_wide
     int R;        // z-split radix (x kernels)
     size_t tab;   // offset of the case records
     int list;     // case list
@@ -479,26 +479,30 @@ int dfp_batch_project(dfp_batch* b, int n, dfp_plan* const* plans, double* const
     // for its fused and split members
     auto x_launches = [&](Launch::Kind k, int f32, int mode, size_t tab, const std::vector<int>& recs,
                           const std::vector<int>& Rs, const std::vector<size_t>& w, int inv) {
-        // one launch per line length of the register kernels, one for the other lengths
+        // and, of the register kernels, per group of line lengths.  A launch per length made so many small ones
+        // that sets of a dozen lengths lost what the kernels gain: 96 tiny FP32 cases 589 -> 520 us a graph
+        // replay (547 with every line staged), 16 FP64 solves 241 -> 219, 48 cases 669 -> 600 (FP32 1085 -> 967).
+        std::vector<int> group(recs.size());
+        std::vector<size_t> need(recs.size());
+        for (size_t i = 0; i < recs.size(); ++i) {
+            const dfp_plan* p = plans[f32 ? i32[recs[i]] : i64[recs[i]]];
+            const size_t reg = x_reg_lds(p, inv, mode, f32);
+            group[i] = reg ? x_reg_group(p, inv, f32) : 0;
+            need[i] = reg ? reg : x_lds_bytes(p, inv, f32);
+        }
         for (int R : kRadixList)
-            for (int M : {0
-#define DFP_XR_LINE(m) , m
-                          DFP_XR_LINES(DFP_XR_LINE)
-#undef DFP_XR_LINE
-                 }) {
+            for (int G = 0; G < kXrGroups; ++G) {
                 std::vector<int> sel;
                 size_t lds = 0;
                 bool wide = false;  // a forward tile too large for two butterfly slots: the four-slot kernel
-                for (int a : recs) {
-                    if (Rs[a] != R) continue;
-                    const dfp_plan* p = plans[f32 ? i32[a] : i64[a]];
-                    const size_t reg = x_reg_lds(p, inv, mode, f32);
-                    if (M != (reg ? p->fx.n : 0)) continue;
-                    sel.push_back(a);
-                    lds = std::max(lds, reg ? reg : x_lds_bytes(p, inv, f32));
+                for (size_t i = 0; i < recs.size(); ++i) {
+                    if (Rs[recs[i]] != R || group[i] != G) continue;
+                    const dfp_plan* p = plans[f32 ? i32[recs[i]] : i64[recs[i]]];
+                    sel.push_back(recs[i]);
+                    lds = std::max(lds, need[i]);
                     wide = wide || (!inv && xfwd_wide(p->fx, R, p->tk_x));
                 }
-                if (!sel.empty()) add(k, f32, (wide ? mode | 8 : mode) | M << 4, R, tab, make_list(sel, w), lds);
+                if (!sel.empty()) add(k, f32, (wide ? mode | 8 : mode) | G << 4, R, tab, make_list(sel, w), lds);
             }
         ++phase;
     };
@@ -671,7 +675,7 @@ int dfp_batch_project(dfp_batch* b, int n, dfp_plan* const* plans, double* const
         std::vector<long> key;
         for (const Launch& l : ls) {
             key.push_back(l.kind);
-            key.push_back(l.f32 * 8192 + l.mode);
+            key.push_back(l.f32 * 256 + l.mode);
             key.push_back(l.R);
             key.push_back((long)l.tab);
             key.push_back(l.list);

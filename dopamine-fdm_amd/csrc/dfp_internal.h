@@ -408,15 +408,16 @@ size_t x_lds_bytes(const dfp_plan* p, int inv, int f32);
 size_t z_lds_bytes(const dfp_plan* p, int f32, int batch = 0);
 template <typename C>
 hipError_t launch_xfwd_batch(hipStream_t s, int R, int mode, const XPar<C>* cs, const int* off, const int* idx,
-                             const int* nc, int grid, size_t lds, int M);
+                             const int* nc, int grid, size_t lds, int G);
 template <typename C>
 hipError_t launch_xinv_batch(hipStream_t s, int R, int accum, const XPar<C>* cs, const int* off, const int* idx,
-                             const int* nc, int grid, size_t lds, int M);
+                             const int* nc, int grid, size_t lds, int G);
 // LDS of the forward (inv = 0, of the given mode) or inverse x kernel with the
 // lines in registers (k_xfwd_reg.h, k_xinv_reg.h) for a plan, 0 if it does not
-// take the plan's lines; M of the batched launches: the lines of every case
-// where those kernels run them, else 0
+// take the plan's lines; G of the batched launches: the group (x_reg_group) of
+// the lines of every case where those kernels run them, else 0
 size_t x_reg_lds(const dfp_plan* p, int inv, int mode, int f32);
+int x_reg_group(const dfp_plan* p, int inv, int f32);
 template <typename C>
 hipError_t launch_zsolve_batch(hipStream_t s, int variant, const ZPar<C>* cs, const int* off, const int* idx,
                                const int* nc, int grid, size_t lds, int wide);

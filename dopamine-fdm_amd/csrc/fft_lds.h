@@ -484,4 +484,28 @@ inline bool xr_steps(int M, FftDesc& d) {
     return false;
 }
 
+// threads of their workgroups, for tiles of up to 8 points a thread: 2048
+// points, or 4096 where the plan's tiles are that large (x_columns)
+template <typename C>  // inverse
+constexpr int xr_threads(int M) { return M >= (sizeof(C) == sizeof(float2) ? 128 : 256) ? 512 : 256; }
+constexpr int xf_threads(int M) { return M >= 128 ? 512 : 256; }  // forward
+
+// Line lengths that share a batched kernel, which switches on the record's
+// length: those of alike register need and workgroup, so that no case is held
+// to another's occupancy (inverse, R = 4, FP64 / FP32 added to phi: 103 / 126,
+// 162 / 166 and 142 / 235 VGPRs for 8 or 9, 12 and 18 points a lane).  0: no kernel.
+constexpr int xr_class(int M) {
+    switch (M) {
+#define DFP_XR_CASE(m) \
+    case m: return XrSteps<m>::e <= 9 ? 1 : XrSteps<m>::e == 12 ? 2 : 3;
+        DFP_XR_LINES(DFP_XR_CASE)
+#undef DFP_XR_CASE
+    }
+    return 0;
+}
+template <typename C>
+constexpr int xr_group(int M) { return xr_class(M) | (xr_threads<C>(M) == 512 ? 4 : 0); }
+constexpr int xf_group(int M) { return xr_class(M) | (xf_threads(M) == 512 ? 4 : 0); }
+constexpr int kXrGroups = 8;  // 1..3: 256 threads, 5..7: 512
+
 }  // namespace dfp

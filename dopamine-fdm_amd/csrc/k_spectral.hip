@@ -13,10 +13,10 @@ template <int R, typename C>
 hipError_t launch_xinv_r(hipStream_t s, int accum, const XPar<C>& q, dim3 grid, size_t lds);
 template <int R, typename C>
 hipError_t launch_xfwd_batch_r(hipStream_t s, int mode, const XPar<C>* cs, const int* off, const int* idx,
-                               const int* nc, int grid, size_t lds, int M);
+                               const int* nc, int grid, size_t lds, int G);
 template <int R, typename C>
 hipError_t launch_xinv_batch_r(hipStream_t s, int accum, const XPar<C>* cs, const int* off, const int* idx,
-                               const int* nc, int grid, size_t lds, int M);
+                               const int* nc, int grid, size_t lds, int G);
 template <typename C>
 size_t xr_lds_any(int M, int R, int T);
 template <typename C>
@@ -121,6 +121,11 @@ size_t x_reg_lds(const dfp_plan* p, int inv, int mode, int f32) {
     return f32 ? xr_lds_any<float2>(p->fx.n, p->zr, p->tk_xi) : xr_lds_any<double2>(p->fx.n, p->zr, p->tk_xi);
 }
 
+int x_reg_group(const dfp_plan* p, int inv, int f32) {
+    if (!inv) return xf_group(p->fx.n);
+    return f32 ? xr_group<float2>(p->fx.n) : xr_group<double2>(p->fx.n);
+}
+
 static const char* xname(int mode, bool f32) {
     static const char* names[2][3] = {{"div_rfft_x", "rfft_x_rhs", "res_rfft_x"},
                                       {"div_rfft_x32", "rfft_x_rhs32", "res_rfft_x32"}};
@@ -157,8 +162,8 @@ static hipError_t xinv_any(int R, hipStream_t s, int accum, const XPar<C>& q, di
 
 template <typename C>
 hipError_t launch_xfwd_batch(hipStream_t s, int R, int mode, const XPar<C>* cs, const int* off, const int* idx,
-                             const int* nc, int grid, size_t lds, int M) {
-#define DFP_CALL(RV) launch_xfwd_batch_r<RV, C>(s, mode, cs, off, idx, nc, grid, lds, M)
+                             const int* nc, int grid, size_t lds, int G) {
+#define DFP_CALL(RV) launch_xfwd_batch_r<RV, C>(s, mode, cs, off, idx, nc, grid, lds, G)
     DFP_R_SWITCH(R, DFP_CALL)
 #undef DFP_CALL
 }
@@ -169,8 +174,8 @@ template hipError_t launch_xfwd_batch<float2>(hipStream_t, int, int, const XPar<
 
 template <typename C>
 hipError_t launch_xinv_batch(hipStream_t s, int R, int accum, const XPar<C>* cs, const int* off, const int* idx,
-                             const int* nc, int grid, size_t lds, int M) {
-#define DFP_CALL(RV) launch_xinv_batch_r<RV, C>(s, accum, cs, off, idx, nc, grid, lds, M)
+                             const int* nc, int grid, size_t lds, int G) {
+#define DFP_CALL(RV) launch_xinv_batch_r<RV, C>(s, accum, cs, off, idx, nc, grid, lds, G)
     DFP_R_SWITCH(R, DFP_CALL)
 #undef DFP_CALL
 }

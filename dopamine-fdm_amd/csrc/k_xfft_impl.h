@@ -505,9 +505,9 @@ hipError_t launch_xinv_r(hipStream_t s, int accum, const XPar<C>& q, dim3 grid, 
 // forward tiles too large for two butterfly slots per thread (FP32 only)
 template <int R, typename C>
 hipError_t launch_xfwd_batch_r(hipStream_t s, int mode, const XPar<C>* cs, const int* off, const int* idx,
-                               const int* nc, int grid, size_t lds, int M) {
+                               const int* nc, int grid, size_t lds, int G) {
     if constexpr (sizeof(C) == sizeof(double2)) {
-        if (M > 0) return launch_xfwd_reg_batch<R>(s, M, cs, off, idx, nc, grid, lds);
+        if (G > 0) return launch_xfwd_reg_batch<R>(s, G, cs, off, idx, nc, grid, lds);
     }
     auto go = [&](auto k) {
         hipLaunchKernelGGL(k, dim3(resident_grid(k, grid, kXThreads, lds)), dim3(kXThreads), lds, s, cs, off, idx, nc);
@@ -539,11 +539,11 @@ hipError_t launch_xfwd_batch_r(hipStream_t s, int mode, const XPar<C>* cs, const
 
 template <int R, typename C>
 hipError_t launch_xinv_batch_r(hipStream_t s, int accum, const XPar<C>* cs, const int* off, const int* idx,
-                               const int* nc, int grid, size_t lds, int M) {
-    if (M > 0) {
+                               const int* nc, int grid, size_t lds, int G) {
+    if (G > 0) {
         constexpr int A1 = sizeof(C) == sizeof(float2);
-        return accum ? launch_xinv_reg_batch<C, A1, R>(s, M, cs, off, idx, nc, grid, lds)
-                     : launch_xinv_reg_batch<C, 0, R>(s, M, cs, off, idx, nc, grid, lds);
+        return accum ? launch_xinv_reg_batch<C, A1, R>(s, G, cs, off, idx, nc, grid, lds)
+                     : launch_xinv_reg_batch<C, 0, R>(s, G, cs, off, idx, nc, grid, lds);
     }
     if (!accum) {
         const auto k = kb_irfft_x<C, 0, R>;

@@ -15,11 +15,8 @@
 
 namespace dfp {
 
-// tiles of up to 8 NT points: 4096 where the plan's tiles are that large (x_columns)
-constexpr int xf_threads(int M) { return M >= 128 ? 512 : 256; }
-
 template <int R, int M>
-__device__ __forceinline__ void xfwd_reg_body(const XPar<double2>& q, int bx, int j, unsigned char* smem_raw) {
+__device__ __forceinline__ void xfwd_reg_body(const XPar<double2>& q, int bx, int j, unsigned char* smem_raw, int tid) {
     using C = double2;
     constexpr int NT = xf_threads(M);
     constexpr int H = M / 2, KI = (M + 1) / 2, E = XrSteps<M>::e, PT = M / E, LD = xr_pitch<M>();
@@ -29,7 +26,6 @@ __device__ __forceinline__ void xfwd_reg_body(const XPar<double2>& q, int bx, in
     const Geo& g = q.g;
     const int nz2 = g.nzp / R;
     const int T = q.T, nl = R * T, k0 = bx * T;
-    const int tid = threadIdx.x;
     C* A = reinterpret_cast<C*>(smem_raw);  // nl lines, positions as in k_xinv_reg.h
     C* tws = A + nl * LD;                   // step twiddles
     C* rtl = tws + n0 + n1;                 // unpack twiddles, M+1
@@ -141,11 +137,11 @@ __global__ void __launch_bounds__(xf_threads(M)) k_rfft_xr(XPar<double2> q) {
     const int L = xcd_remap(blockIdx.x + gridDim.x * blockIdx.y, gridDim.x * gridDim.y);
     int bx, j;
     xtile(L, gridDim.x, gridDim.y, q.strip, bx, j);
-    xfwd_reg_body<R, M>(q, bx, j, smem_raw);
+    xfwd_reg_body<R, M>(q, bx, j, smem_raw, threadIdx.x);
 }
 
-template <int R, int M>
-__global__ void __launch_bounds__(xf_threads(M))
+template <int R, int G>
+__global__ void __launch_bounds__(G & 4 ? 512 : 256)
 kb_rfft_xr(const XPar<double2>* __restrict__ cs, const int* __restrict__ off, const int* __restrict__ idx,
            const int* __restrict__ pnc) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -159,7 +155,14 @@ kb_rfft_xr(const XPar<double2>* __restrict__ cs, const int* __restrict__ off, co
         const XPar<double2>& q = cs[idx[c]];
         int bx, j;
         xtile(w - off[c], q.nbx, q.g.nym, q.strip, bx, j);
-        xfwd_reg_body<R, M>(q, bx, j, smem_raw);
+        switch (__builtin_amdgcn_readfirstlane(q.fd.n)) {
+#define DFP_XR_CASE(m)                                                                              \
+    case m:                                                                                         \
+        if constexpr (xf_group(m) == G) xfwd_reg_body<R, m>(q, bx, j, smem_raw, thread_id());       \
+        break;
+            DFP_XR_LINES(DFP_XR_CASE)
+#undef DFP_XR_CASE
+        }
         __syncthreads();
     }
 }
@@ -178,43 +181,42 @@ size_t xf_lds_any(int M, int R, int T) {
     return 0;
 }
 
-template <typename F>
-hipError_t xf_dispatch(int M, F go) {
-    switch (M) {
-#define DFP_XR_CASE(m) \
-    case m: return go(std::integral_constant<int, m>{});
-        DFP_XR_LINES(DFP_XR_CASE)
-#undef DFP_XR_CASE
-    }
-    return hipErrorInvalidValue;
-}
-
 // false: the plan's lines or tile are not this kernel's
 template <int R>
 bool launch_xfwd_reg(hipStream_t s, const XPar<double2>& q, dim3 grid) {
     if constexpr (xr_split(R)) {
         const size_t lds = q.twr ? xf_lds_any<double2>(q.fd.n, R, q.T) : 0;
         if (lds == 0) return false;
-        return xf_dispatch(q.fd.n, [&](auto m) {
-            constexpr int M = decltype(m)::value;
-            hipLaunchKernelGGL((k_rfft_xr<R, M>), grid, dim3(xf_threads(M)), lds, s, q);
-            return hipSuccess;
-        }) == hipSuccess;
+        switch (q.fd.n) {
+#define DFP_XR_CASE(m)                                                                          \
+    case m:                                                                                     \
+        hipLaunchKernelGGL((k_rfft_xr<R, m>), grid, dim3(xf_threads(m)), lds, s, q);            \
+        return true;
+            DFP_XR_LINES(DFP_XR_CASE)
+#undef DFP_XR_CASE
+        }
     }
     return false;
 }
 
-// M: the lines of every case of the list
+// G: the group of the lines of every case of the list
 template <int R>
-hipError_t launch_xfwd_reg_batch(hipStream_t s, int M, const XPar<double2>* cs, const int* off, const int* idx,
+hipError_t launch_xfwd_reg_batch(hipStream_t s, int G, const XPar<double2>* cs, const int* off, const int* idx,
                                  const int* nc, int grid, size_t lds) {
     if constexpr (xr_split(R)) {
-        return xf_dispatch(M, [&](auto m) {
-            constexpr int MV = decltype(m)::value, NT = xf_threads(MV);
-            const auto k = kb_rfft_xr<R, MV>;
+        auto go = [&](auto k) {
+            const int NT = G & 4 ? 512 : 256;
             hipLaunchKernelGGL(k, dim3(resident_grid(k, grid, NT, lds)), dim3(NT), lds, s, cs, off, idx, nc);
             return hipGetLastError();
-        });
+        };
+        switch (G) {
+            case 1: return go(kb_rfft_xr<R, 1>);
+            case 2: return go(kb_rfft_xr<R, 2>);
+            case 3: return go(kb_rfft_xr<R, 3>);
+            case 5: return go(kb_rfft_xr<R, 5>);
+            case 6: return go(kb_rfft_xr<R, 6>);
+            case 7: return go(kb_rfft_xr<R, 7>);
+        }
     }
     return hipErrorInvalidValue;
 }

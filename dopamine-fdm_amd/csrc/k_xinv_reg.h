@@ -26,10 +26,6 @@
 
 namespace dfp {
 
-// tiles of up to 8 NT points: 2048, or 4096 where the plan's tiles are that large (x_columns)
-template <typename C>
-constexpr int xr_threads(int M) { return M >= (sizeof(C) == sizeof(float2) ? 128 : 256) ? 512 : 256; }
-
 // z splits with a kernel, and the items (mode pair, column) that a thread gathers of a tile of up to 8 NT points
 constexpr bool xr_split(int R) { return R <= 4 || R == 6 || R == 8 || R == 9; }
 constexpr int xr_items(int R) { return (4 + R - 1) / R; }
@@ -47,6 +43,15 @@ __device__ __forceinline__ int xr_pos(int e, int lx) {
 __device__ __forceinline__ void wave_exchange() {
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
+}
+
+// threadIdx.x for the bodies in a batched kernel, opaque to the compiler, so
+// that each item forms what depends on it anew: held over the loop for every
+// length, the LDS positions took up to 256 VGPRs and spilled
+__device__ __forceinline__ int thread_id() {
+    int t = threadIdx.x;
+    asm volatile("" : "+v"(t));
+    return t;
 }
 
 // One step of radix r and stride s on a line: this lane's 8/r butterflies.
@@ -83,17 +88,15 @@ __device__ __forceinline__ void xr_step(C* line, int lx, int b0, const C* tws, b
 // As xinv_body: last inverse z stage, C2R, phi (ACCUM: added to phi) with its
 // duplicates and, with save_p, P = phi/(dt*c) with its ghosts.
 template <typename C, int ACCUM, int R, int M>
-__device__ __forceinline__ void xinv_reg_body(const XPar<C>& q, int bx, int j, unsigned char* smem_raw) {
+__device__ __forceinline__ void xinv_reg_body(const XPar<C>& q, int bx, int j, unsigned char* smem_raw, double* wsum, int tid) {
     constexpr int NT = xr_threads<C>(M);
     constexpr int H = M / 2, KI = (M + 1) / 2, E = XrSteps<M>::e, PT = M / E, LD = xr_pitch<M>();
     constexpr int GI = xr_items(R);  // gathered items (mode pair, column) per thread
     constexpr int r0 = XrSteps<M>::r[0], r1 = XrSteps<M>::r[1], r2 = XrSteps<M>::r[2];
     constexpr int n0 = M / r0 * (r0 - 1), n1 = r2 > 1 ? M / (r0 * r1) * (r1 - 1) : 0;  // twiddles of all steps but the last
-    __shared__ double wsum[NT / 64];
     const Geo& g = q.g;
     const int nz2 = g.nzp / R;
     const int T = q.T, nl = R * T, k0 = bx * T;
-    const int tid = threadIdx.x;
     C* A = reinterpret_cast<C*>(smem_raw);  // nl lines
     C* tws = A + nl * LD;                   // step twiddles
     C* rtl = tws + n0 + n1;                 // packing twiddles, M+1
@@ -280,15 +283,17 @@ __global__ void __launch_bounds__(xr_threads<C>(M)) k_irfft_xr(XPar<C> q) {
     const int L = xcd_remap(blockIdx.x + gridDim.x * blockIdx.y, gridDim.x * gridDim.y);
     int bx, j;
     xtile(L, gridDim.x, gridDim.y, q.strip, bx, j);
-    xinv_reg_body<C, ACCUM, R, M>(q, bx, j, smem_raw);
+    __shared__ double wsum[xr_threads<C>(M) / 64];
+    xinv_reg_body<C, ACCUM, R, M>(q, bx, j, smem_raw, wsum, threadIdx.x);
 }
 
-// one workgroup per work item, or persistent, as the other batched kernels
-template <typename C, int ACCUM, int R, int M>
-__global__ void __launch_bounds__(xr_threads<C>(M))
+// one workgroup per work item, or persistent, as the other batched kernels; G: the group of its cases' lines
+template <typename C, int ACCUM, int R, int G>
+__global__ void __launch_bounds__(G & 4 ? 512 : 256)
 kb_irfft_xr(const XPar<C>* __restrict__ cs, const int* __restrict__ off, const int* __restrict__ idx,
             const int* __restrict__ pnc) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
+    __shared__ double wsum[8];
     const int nc = *pnc;
     const int total = off[nc];
     const int me = xcd_remap(blockIdx.x, gridDim.x);
@@ -299,7 +304,14 @@ kb_irfft_xr(const XPar<C>* __restrict__ cs, const int* __restrict__ off, const i
         const XPar<C>& q = cs[idx[c]];
         int bx, j;
         xtile(w - off[c], q.nbx, q.g.nym, q.strip, bx, j);
-        xinv_reg_body<C, ACCUM, R, M>(q, bx, j, smem_raw);
+        switch (__builtin_amdgcn_readfirstlane(q.fd.n)) {
+#define DFP_XR_CASE(m)                                                                                              \
+    case m:                                                                                                         \
+        if constexpr (xr_group<C>(m) == G) xinv_reg_body<C, ACCUM, R, m>(q, bx, j, smem_raw, wsum, thread_id());    \
+        break;
+            DFP_XR_LINES(DFP_XR_CASE)
+#undef DFP_XR_CASE
+        }
         __syncthreads();
     }
 }
@@ -321,23 +333,25 @@ size_t xr_lds_any(int M, int R, int T) {
     return 0;
 }
 
-// M: the lines of every case of the list
+// G: the group of the lines of every case of the list
 template <typename C, int ACCUM, int R>
-hipError_t launch_xinv_reg_batch(hipStream_t s, int M, const XPar<C>* cs, const int* off, const int* idx,
+hipError_t launch_xinv_reg_batch(hipStream_t s, int G, const XPar<C>* cs, const int* off, const int* idx,
                                  const int* nc, int grid, size_t lds) {
     if constexpr (xr_split(R)) {
-        auto go = [&](auto m) {
-            constexpr int MV = decltype(m)::value;
-            const auto k = kb_irfft_xr<C, ACCUM, R, MV>;
-            constexpr int NT = xr_threads<C>(MV);
+        auto go = [&](auto k) {
+            const int NT = G & 4 ? 512 : 256;
             hipLaunchKernelGGL(k, dim3(resident_grid(k, grid, NT, lds)), dim3(NT), lds, s, cs, off, idx, nc);
             return hipGetLastError();
         };
-        switch (M) {
-#define DFP_XR_CASE(m) \
-    case m: return go(std::integral_constant<int, m>{});
-            DFP_XR_LINES(DFP_XR_CASE)
-#undef DFP_XR_CASE
+        switch (G) {
+            case 1: return go(kb_irfft_xr<C, ACCUM, R, 1>);
+            case 2: return go(kb_irfft_xr<C, ACCUM, R, 2>);
+            case 3: return go(kb_irfft_xr<C, ACCUM, R, 3>);
+            case 5: return go(kb_irfft_xr<C, ACCUM, R, 5>);
+        }
+        if constexpr (sizeof(C) == sizeof(float2)) {  // FP64: 512 threads for 256 points only
+            if (G == 6) return go(kb_irfft_xr<C, ACCUM, R, 6>);
+            if (G == 7) return go(kb_irfft_xr<C, ACCUM, R, 7>);
         }
     }
     return hipErrorInvalidValue;

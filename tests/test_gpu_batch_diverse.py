@@ -1,6 +1,6 @@
 """Batches of many different sizes in one call: every stage then has many
-launches (x kernels by z split and line length, z kernels by row length), and
-the call takes them all.  Each case equals its own plan's bits."""
+launches (x kernels by z split and group of line lengths, z kernels by row
+length), and the call takes them all.  Each case equals its own plan's bits."""
 from __future__ import annotations
 
 import pytest
