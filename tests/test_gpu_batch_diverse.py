@@ -55,7 +55,7 @@ def test_diverse_batch_equals_single_plans(n, precision, sweeps, solve_only, gra
         U, V, W, P, rhs = two
         cases.append(Case(plans[1], U, V, W, rhs, P, DT, C3, save_p=True))
     batch = Batch(max_cases=n, graphs=graphs)
-    for _ in range(2):  # with graphs: captured, then replayed
+    for _ in range(3):  # with graphs: run, captured, replayed
         for c, f in zip(cases, start):
             for to, at in zip((c.U, c.V, c.W, c.P, c.rhs), f):
                 to.copy_(at)
@@ -64,6 +64,42 @@ def test_diverse_batch_equals_single_plans(n, precision, sweeps, solve_only, gra
         for size, c, s in zip(_sizes(n), cases, singles):
             for lab, a, b in zip(("U", "V", "W", "P", "phi"), (c.U, c.V, c.W, c.P, c.rhs), s):
                 assert torch.equal(a, b), (size, lab)
+    batch.close()
+    for c in cases:
+        c.plan.close()
+
+
+def test_graph_of_a_batch_is_captured_when_its_stage_list_comes_again():
+    """Sets of sizes in turn, each run directly, then captured, then replayed, other sets between: every call equals
+    the single plans' bits."""
+    import torch
+
+    from dfp.batch import Batch, Case
+
+    print("graphs over alternating sets of sizes", flush=True)
+    cases, start, want = [], [], []
+    for i, (nxp, nym, nzp, R) in enumerate(_sizes(12)):
+        g = make_grid(nxp, nym, nzp, 1.5)
+        f = [torch.from_numpy(a.T.copy()).cuda() for a in fields(g, i + 1, 0.1)]
+        start.append([a.clone() for a in f])
+        one = [a.clone() for a in f]
+        plan = dfp.Plan(g, tuning=(R, 0, 0, 0))
+        plan.project(*one[:3], one[4], one[3], DT, C3, save_p=True)
+        want.append(one)
+        cases.append(Case(plan, *f[:3], f[4], f[3], DT, C3, save_p=True))
+    batch = Batch(max_cases=12, graphs=True)
+    for call in range(8):
+        part = range(12)[call % 2::2] if call != 5 else range(12)
+        for i in part:
+            c = cases[i]
+            for to, at in zip((c.U, c.V, c.W, c.P, c.rhs), start[i]):
+                to.copy_(at)
+        torch.cuda.synchronize()
+        batch.project([cases[i] for i in part])
+        for i in part:
+            c = cases[i]
+            for lab, a, b in zip(("U", "V", "W", "P", "phi"), (c.U, c.V, c.W, c.P, c.rhs), want[i]):
+                assert torch.equal(a, b), (call, i, lab)
     batch.close()
     for c in cases:
         c.plan.close()
