@@ -514,7 +514,8 @@ int dfp_plan_create(const dfp_grid* g, int precision, int device, dfp_plan** out
 int dfp_plan_tuning(const dfp_plan* p, dfp_tuning* t) {
     if (!p || !t) return DFP_E_ARG;
     t->z_split = p->zr;
-    t->x_columns = p->tk_x;
+    // each x kernel's own choice, and narrower tiles on small grids, are what 0 chooses
+    t->x_columns = p->tuned_columns ? p->tk_x : 0;
     // the register-plane kernel is what 0, 0 choose
     t->z_rows = p->zp_nb ? 0 : p->g_zs;
     t->z_fused = p->zp_nb ? 0 : (p->zfused ? 2 : 1);

@@ -137,8 +137,9 @@ class Plan:
 
     @property
     def tuning(self) -> tuple:
-        """(z_split, x_columns, z_rows, z_fused) the plan runs with (z_fused 2: one
-        fused z kernel, 1: the split pair)."""
+        """(z_split, x_columns, z_rows, z_fused) that make this plan (x_columns 0: each x
+        kernel's own; z_fused 2: one fused z kernel, 1: the split pair, 0: sub-planes in
+        registers)."""
         t = DfpTuning()
         check(lib().dfp_plan_tuning(self._h, ctypes.byref(t)), "dfp_plan_tuning", self._h)
         return (t.z_split, t.x_columns, t.z_rows, t.z_fused)

@@ -100,7 +100,7 @@ int dfp_plan_destroy(dfp_plan *plan);
  *              then transform rows of nzp/R <= 256 points, one mode per lane)
  *   x_columns  z columns per x-kernel workgroup (divides nzp/R); given, it
  *              sets both x kernels, else each picks its own (dfp_plan_tuning
- *              reports the forward kernel's)
+ *              then reports 0)
  *   z_rows     y rows per group of the split z kernels (z_fused = 1)
  *   z_fused    1: split pair of z kernels (FFT + elimination, back
  *              substitution + inverse FFT, spectrum read and written twice);
