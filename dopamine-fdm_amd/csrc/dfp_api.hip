@@ -578,7 +578,12 @@ int dfp_plan_create_tuned(const dfp_grid* g, int precision, int device, const df
     p->fx = sh.fx;
     p->fz = sh.fz;
     p->tk_x = sh.T;
-    p->tk_xi = sh.Ti;
+    // the inflow/outflow x has no lines in registers
+    auto reg = [&](int T, XKind k) {
+        return g->x_bc_type == 1 ? T : x_reg_columns(sh.fx.n, sh.R, g->nzp / sh.R, T, k, precision == DFP_FP32_REFINE);
+    };
+    p->tk_xi = reg(sh.Ti, XKind::inverse);
+    p->tk_xs = reg(sh.T, XKind::rhs);
     p->tuned_columns = tune && tune->x_columns > 0;
     p->g_zs = sh.G;
     p->zfused = sh.fused;

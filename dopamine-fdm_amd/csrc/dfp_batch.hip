@@ -386,12 +386,13 @@ int dfp_batch_project(dfp_batch* b, int n, dfp_plan* const* plans, double* const
         XPar<double2> q = make_xpar<double2>(p);
         if (solve) q.a.rhs = rhs_p[i];
         else { q.a.U = U[i]; q.a.V = V[i]; q.a.W = W[i]; }
+        if (solve) xpar_columns(q, p, XKind::rhs);
         q.rhs = rhs_p[i];
         q.save_p = (fl & DFP_SAVE_P) ? 1 : 0;
         q.P = q.save_p ? P[i] : nullptr;
         q.dtc = q.save_p ? dt[i] * c[i] : 1.0;
         x64[a] = q;
-        xpar_columns(q, p, 1);
+        xpar_columns(q, p, XKind::inverse);
         x64i[a] = q;
         z64[a] = make_zpar<double2>(p, 0, 1);
         w64x[a] = (size_t)x64[a].nbx * p->geo.nym;
@@ -417,7 +418,7 @@ int dfp_batch_project(dfp_batch* b, int n, dfp_plan* const* plans, double* const
         q.part0 = p->d_part0;
         x32[a] = q;
         x32i[a] = q;
-        xpar_columns(x32i[a], p, 1);
+        xpar_columns(x32i[a], p, XKind::inverse);
         XPar<float2> r = q;  // sweeps: residual forward, accumulating inverse
         r.a = XArgs{};
         r.a.rhs = rhs_p[i];
@@ -428,7 +429,7 @@ int dfp_batch_project(dfp_batch* b, int n, dfp_plan* const* plans, double* const
         r.a.idz2 = 1.0 / (p->dz * p->dz);
         x32s[a] = r;
         x32si[a] = r;
-        xpar_columns(x32si[a], p, 1);
+        xpar_columns(x32si[a], p, XKind::inverse);
         z32[a] = make_zpar<float2>(p, 1, 1);
         m32[a] = make_mpar(p);
         w32x[a] = (size_t)q.nbx * p->geo.nym;
@@ -481,7 +482,7 @@ int dfp_batch_project(dfp_batch* b, int n, dfp_plan* const* plans, double* const
     // the x launches of a set of records, one per radix present; the z launches
     // for its fused and split members
     auto x_launches = [&](Launch::Kind k, int f32, int mode, size_t tab, const std::vector<int>& recs,
-                          const std::vector<int>& Rs, const std::vector<size_t>& w, int inv) {
+                          const std::vector<int>& Rs, const std::vector<size_t>& w, XKind kind) {
         // and, of the register kernels, per group of line lengths.  A launch per length made so many small ones
         // that sets of a dozen lengths lost what the kernels gain: 96 tiny FP32 cases 589 -> 520 us a graph
         // replay (547 with every line staged), 16 FP64 solves 241 -> 219, 48 cases 669 -> 600 (FP32 1085 -> 967).
@@ -489,9 +490,9 @@ int dfp_batch_project(dfp_batch* b, int n, dfp_plan* const* plans, double* const
         std::vector<size_t> need(recs.size());
         for (size_t i = 0; i < recs.size(); ++i) {
             const dfp_plan* p = plans[f32 ? i32[recs[i]] : i64[recs[i]]];
-            const size_t reg = x_reg_lds(p, inv, mode, f32);
-            group[i] = reg ? x_reg_group(p, inv, f32) : 0;
-            need[i] = reg ? reg : x_lds_bytes(p, inv, f32);
+            const size_t reg = x_reg_lds(p, kind, f32);
+            group[i] = reg ? x_reg_group(p, kind, f32) : 0;
+            need[i] = reg ? reg : x_lds_bytes(p, kind, f32);
         }
         for (int R : kRadixList)
             for (int G = 0; G < kXrGroups; ++G) {
@@ -503,7 +504,7 @@ int dfp_batch_project(dfp_batch* b, int n, dfp_plan* const* plans, double* const
                     const dfp_plan* p = plans[f32 ? i32[recs[i]] : i64[recs[i]]];
                     sel.push_back(recs[i]);
                     lds = std::max(lds, need[i]);
-                    wide = wide || (!inv && xfwd_wide(p->fx, R, p->tk_x));
+                    wide = wide || (k == Launch::XF && xfwd_wide(p->fx, R, p->tk_x));
                 }
                 if (!sel.empty()) add(k, f32, (wide ? mode | 8 : mode) | G << 4, R, tab, make_list(sel, w), lds);
             }
@@ -535,25 +536,25 @@ int dfp_batch_project(dfp_batch* b, int n, dfp_plan* const* plans, double* const
     auto first = [](int k) { std::vector<int> v(k); for (int a = 0; a < k; ++a) v[a] = a; return v; };
     if (n64) {
         const std::vector<int> all = first(n64);
-        x_launches(Launch::XF, 0, solve ? 1 : 0, L.x64, all, R64, w64x, 0);
+        x_launches(Launch::XF, 0, solve ? 1 : 0, L.x64, all, R64, w64x, solve ? XKind::rhs : XKind::forward);
         z_launches(0, L.z64, all, F64, w64z);
-        x_launches(Launch::XI, 0, 0, L.x64i, all, R64, w64xi, 1);
+        x_launches(Launch::XI, 0, 0, L.x64i, all, R64, w64xi, XKind::inverse);
     }
     if (n32) {
         const std::vector<int> all = first(n32);
         const std::vector<size_t> one(n32, 1);
-        x_launches(Launch::XF, 1, solve ? 1 : 0, L.x32, all, R32, w32x, 0);
+        x_launches(Launch::XF, 1, solve ? 1 : 0, L.x32, all, R32, w32x, XKind::forward);
         add(Launch::M00, 1, 0, 0, L.m32, make_list(all, one), 0);
         ++phase;
         z_launches(1, L.z32, all, F32, w32z);
-        x_launches(Launch::XI, 1, 0, L.x32i, all, R32, w32xi, 1);
+        x_launches(Launch::XI, 1, 0, L.x32i, all, R32, w32xi, XKind::inverse);
         for (int s = 0; s < max_sweeps; ++s) {
             const std::vector<int> pre = first(n_at_sweep[s]);
-            x_launches(Launch::XF, 1, 2, L.x32s, pre, R32, w32x, 0);
+            x_launches(Launch::XF, 1, 2, L.x32s, pre, R32, w32x, XKind::forward);
             add(Launch::M00, 1, 0, 0, L.m32, make_list(pre, one), 0);
             ++phase;
             z_launches(1, L.z32, pre, F32, w32z);
-            x_launches(Launch::XI, 1, 1, L.x32si, pre, R32, w32xi, 1);
+            x_launches(Launch::XI, 1, 1, L.x32si, pre, R32, w32xi, XKind::inverse);
         }
         if (ns) add(Launch::SAVE, 1, 0, 0, L.s32, make_list(save_rec, ws), 0);
         ++phase;

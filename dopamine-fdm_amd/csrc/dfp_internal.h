@@ -273,6 +273,7 @@ struct dfp_plan {
     // launch shapes
     int tk_x = 8;   // z columns per block of the forward x kernel (zr lines each)
     int tk_xi = 8;  // z columns per block of the inverse x kernel
+    int tk_xs = 8;  // z columns per block of the forward x kernel of a given right-hand side
     bool tuned_columns = false;  // the caller chose them (else small grids launch narrower tiles)
     int g_zs = 4;   // rows per group of the split z kernels, or rows per FFT call of the fused one
     int zfused = 0; // 1: one fused z kernel (whole sub-plane in LDS); 0: the split pair
@@ -396,15 +397,16 @@ hipError_t launch_synth(dfp_plan* p, double* U, double* V, double* W, uint64_t s
 // parameter records and batched (persistent) launches: cs (records), off
 // (per-listed-case work offsets, off[0] = 0, off[*nc] = total items), idx
 // (listed case -> record) and the count *nc are in device memory
-template <typename C> XPar<C> make_xpar(const dfp_plan* p, int inv = 0);
-// set the column fields (T, nbx, strip, div_t) of q for the forward (inv = 0) or inverse x kernel
-template <typename C> void xpar_columns(XPar<C>& q, const dfp_plan* p, int inv);
+enum class XKind { forward, inverse, rhs };  // rhs: the forward kernel of a given right-hand side
+template <typename C> XPar<C> make_xpar(const dfp_plan* p, XKind k = XKind::forward);
+// set the column fields (T, nbx, strip, div_t) of q
+template <typename C> void xpar_columns(XPar<C>& q, const dfp_plan* p, XKind k);
 // batch: the record of a batched launch (planes per workgroup of the register-plane kernel)
 template <typename C> ZPar<C> make_zpar(const dfp_plan* p, int zero00, int batch = 0);
 CPar make_cpar(const dfp_plan* p, double* U, double* V, double* W, const double* rhs);
 MPar make_mpar(const dfp_plan* p);
 SPar make_spar(const dfp_plan* p, const double* rhs, double* P, double dtc);
-size_t x_lds_bytes(const dfp_plan* p, int inv, int f32);
+size_t x_lds_bytes(const dfp_plan* p, XKind k, int f32);
 size_t z_lds_bytes(const dfp_plan* p, int f32, int batch = 0);
 template <typename C>
 hipError_t launch_xfwd_batch(hipStream_t s, int R, int mode, const XPar<C>* cs, const int* off, const int* idx,
@@ -412,12 +414,16 @@ hipError_t launch_xfwd_batch(hipStream_t s, int R, int mode, const XPar<C>* cs, 
 template <typename C>
 hipError_t launch_xinv_batch(hipStream_t s, int R, int accum, const XPar<C>* cs, const int* off, const int* idx,
                              const int* nc, int grid, size_t lds, int G);
-// LDS of the forward (inv = 0, of the given mode) or inverse x kernel with the
-// lines in registers (k_xfwd_reg.h, k_xinv_reg.h) for a plan, 0 if it does not
-// take the plan's lines; G of the batched launches: the group (x_reg_group) of
-// the lines of every case where those kernels run them, else 0
-size_t x_reg_lds(const dfp_plan* p, int inv, int mode, int f32);
-int x_reg_group(const dfp_plan* p, int inv, int f32);
+// LDS of the x kernel with the lines in registers (k_xfwd_reg.h, k_xinv_reg.h)
+// for a plan, 0 if it does not take the plan's lines; G of the batched
+// launches: the group (x_reg_group) of the lines of every case where those
+// kernels run them, else 0
+size_t x_reg_lds(const dfp_plan* p, XKind k, int f32);
+int x_reg_group(const dfp_plan* p, XKind k, int f32);
+// the most columns (a divisor of nz2 = nzp/R) up to T that the register kernel
+// of M-point lines takes; T if there is no such kernel.  Which kernel runs a
+// plan's lines, and with it the rounding, then does not depend on T.
+int x_reg_columns(int M, int R, int nz2, int T, XKind k, int f32);
 template <typename C>
 hipError_t launch_zsolve_batch(hipStream_t s, int variant, const ZPar<C>* cs, const int* off, const int* idx,
                                const int* nc, int grid, size_t lds, int wide);

@@ -33,10 +33,14 @@ bool xfwd_wide(const FftDesc& fx, int R, int T) {
     return (long)R * T * fx.n > (long)inplace_capacity(fx, 512, 2, true);  // 512 threads per x workgroup
 }
 
+static int plan_columns(const dfp_plan* p, XKind k) {
+    return k == XKind::inverse ? p->tk_xi : k == XKind::rhs ? p->tk_xs : p->tk_x;
+}
+
 template <typename C>
-void xpar_columns(XPar<C>& q, const dfp_plan* p, int inv) {
+void xpar_columns(XPar<C>& q, const dfp_plan* p, XKind k) {
     const Geo& g = p->geo;
-    q.T = inv ? p->tk_xi : p->tk_x;
+    q.T = plan_columns(p, k);
     q.nbx = (g.nzp / p->zr) / q.T;
     // A row of tiles moves about 24 * nxp * nzp bytes of u*, v*, w* (or phi and
     // b); from nxp = 512 up that exceeds an XCD's 4 MB L2 before the next row
@@ -47,8 +51,8 @@ void xpar_columns(XPar<C>& q, const dfp_plan* p, int inv) {
     q.strip = g.nxp >= 512 ? std::min(q.nbx, 8) : q.nbx;
     q.div_t = FastDiv(q.T);
 }
-template void xpar_columns<double2>(XPar<double2>&, const dfp_plan*, int);
-template void xpar_columns<float2>(XPar<float2>&, const dfp_plan*, int);
+template void xpar_columns<double2>(XPar<double2>&, const dfp_plan*, XKind);
+template void xpar_columns<float2>(XPar<float2>&, const dfp_plan*, XKind);
 
 // A single launch on a small grid: narrower tiles while the launch has fewer
 // than two workgroups per CU, down to four columns (64-byte FP64 spectrum
@@ -69,14 +73,14 @@ static void narrow_columns(XPar<double2>& q) {
 static void narrow_columns(XPar<float2>&) {}
 
 template <typename C>
-XPar<C> make_xpar(const dfp_plan* p, int inv) {
+XPar<C> make_xpar(const dfp_plan* p, XKind k) {
     XPar<C> q{};
     const Geo& g = p->geo;
     q.g = g;
     q.o = p->ops;
     q.fd = p->fx;
     q.R = p->zr;
-    xpar_columns(q, p, inv);
+    xpar_columns(q, p, k);
     q.npart0 = (g.nzp / p->zr) / p->tk_xi;
     q.ntw = twiddle_count(p->fx);
     q.div_nxp = FastDiv(g.nxp);
@@ -101,8 +105,8 @@ XPar<C> make_xpar(const dfp_plan* p, int inv) {
     }
     return q;
 }
-template XPar<double2> make_xpar<double2>(const dfp_plan*, int);
-template XPar<float2> make_xpar<float2>(const dfp_plan*, int);
+template XPar<double2> make_xpar<double2>(const dfp_plan*, XKind);
+template XPar<float2> make_xpar<float2>(const dfp_plan*, XKind);
 
 // dynamic LDS of an x kernel with T columns per workgroup
 static size_t x_lds_bytes_t(const dfp_plan* p, int T, int f32) {
@@ -112,17 +116,26 @@ static size_t x_lds_bytes_t(const dfp_plan* p, int T, int f32) {
         return cs * ((size_t)R * T * M + twiddle_count(p->fx) + 2 * M + (size_t)nz2 * (R - 1));
     return cs * ((size_t)R * T * (M + 1) + twiddle_count(p->fx) + M + 1 + (size_t)nz2 * (R - 1));
 }
-// of a plan's forward (inv = 0) or inverse (inv = 1) x kernel
-size_t x_lds_bytes(const dfp_plan* p, int inv, int f32) { return x_lds_bytes_t(p, inv ? p->tk_xi : p->tk_x, f32); }
+size_t x_lds_bytes(const dfp_plan* p, XKind k, int f32) { return x_lds_bytes_t(p, plan_columns(p, k), f32); }
 
-size_t x_reg_lds(const dfp_plan* p, int inv, int mode, int f32) {
-    if (!p->tw_xr || (!inv && (f32 || mode != 1))) return 0;
-    if (!inv) return xf_lds_any<double2>(p->fx.n, p->zr, p->tk_x);
-    return f32 ? xr_lds_any<float2>(p->fx.n, p->zr, p->tk_xi) : xr_lds_any<double2>(p->fx.n, p->zr, p->tk_xi);
+// LDS of the kernel with T lines of M points in registers per split, 0 if it does not take them
+static size_t reg_lds(int M, int R, int T, XKind k, int f32) {
+    if (k != XKind::inverse) return k == XKind::rhs && !f32 ? xf_lds_any<double2>(M, R, T) : 0;
+    return f32 ? xr_lds_any<float2>(M, R, T) : xr_lds_any<double2>(M, R, T);
 }
 
-int x_reg_group(const dfp_plan* p, int inv, int f32) {
-    if (!inv) return xf_group(p->fx.n);
+size_t x_reg_lds(const dfp_plan* p, XKind k, int f32) {
+    return p->tw_xr ? reg_lds(p->fx.n, p->zr, plan_columns(p, k), k, f32) : 0;
+}
+
+int x_reg_columns(int M, int R, int nz2, int T, XKind k, int f32) {
+    for (int t = T; t >= 1; --t)
+        if (nz2 % t == 0 && reg_lds(M, R, t, k, f32)) return t;
+    return T;
+}
+
+int x_reg_group(const dfp_plan* p, XKind k, int f32) {
+    if (k != XKind::inverse) return xf_group(p->fx.n);
     return f32 ? xr_group<float2>(p->fx.n) : xr_group<double2>(p->fx.n);
 }
 
@@ -198,6 +211,7 @@ static hipError_t xdct_inv_any(int R, hipStream_t s, const XPar<double2>& q, dim
 
 template <typename C>
 static hipError_t launch_xfwd(dfp_plan* p, int mode, XPar<C> q) {
+    if (mode == 1) xpar_columns(q, p, XKind::rhs);
     if (!p->tuned_columns) narrow_columns(q);
     const dim3 grid(q.nbx, q.g.nym);
     const size_t lds = x_lds_bytes_t(p, q.T, sizeof(C) == 8);
@@ -243,7 +257,7 @@ static hipError_t launch_xinv(dfp_plan* p, XPar<C> q) {
 }
 
 hipError_t launch_irfft_x(dfp_plan* p, double* rhs, double* P, double dtc, int save_p) {
-    XPar<double2> q = make_xpar<double2>(p, 1);
+    XPar<double2> q = make_xpar<double2>(p, XKind::inverse);
     q.rhs = rhs; q.P = P; q.dtc = dtc; q.save_p = save_p;
     if (p->geo.xbc == 1) {
         if (!p->tuned_columns) narrow_columns(q);
@@ -259,7 +273,7 @@ hipError_t launch_irfft_x(dfp_plan* p, double* rhs, double* P, double dtc, int s
 
 hipError_t launch_irfft_x32(dfp_plan* p, double* rhs, int accumulate, const double* pbar, double* part0, double* P,
                             double dtc, int save_p) {
-    XPar<float2> q = make_xpar<float2>(p, 1);
+    XPar<float2> q = make_xpar<float2>(p, XKind::inverse);
     q.rhs = rhs; q.pbar = pbar; q.part0 = part0;
     q.P = P; q.dtc = save_p ? dtc : 1.0; q.save_p = save_p;
     if (accumulate) return launch_xinv<float2, 1>(p, q);

@@ -99,8 +99,9 @@ int dfp_plan_destroy(dfp_plan *plan);
  *              applied by the x kernels (R must divide nzp; the z kernels
  *              then transform rows of nzp/R <= 256 points, one mode per lane)
  *   x_columns  z columns per x-kernel workgroup (divides nzp/R); given, it
- *              sets both x kernels, else each picks its own (dfp_plan_tuning
- *              then reports 0)
+ *              sets both x kernels (one that holds its lines in registers
+ *              takes the most of them that fit), else each picks its own
+ *              (dfp_plan_tuning then reports 0)
  *   z_rows     y rows per group of the split z kernels (z_fused = 1)
  *   z_fused    1: split pair of z kernels (FFT + elimination, back
  *              substitution + inverse FFT, spectrum read and written twice);
@@ -109,9 +110,10 @@ int dfp_plan_destroy(dfp_plan *plan);
  *              0 with z_rows = 0: a sub-plane held in registers where it
  *              fits (read and written once; dfp_plan_tuning then reports
  *              z_rows = z_fused = 0), else 1
- * Results do not depend on x_columns or, at z_fused = 1, on z_rows; z_split
- * changes the FFT's factorisation and z_fused the association of the y solve
- * (chunked across lanes at 0 and 2), both at round-off level.  DFP_E_ARG for values out of
+ * FP64 results do not depend on x_columns (the FP32 form's row sums take the
+ * order of the columns, at round-off level) or, at z_fused = 1, on z_rows;
+ * z_split changes the FFT's factorisation and z_fused the association of the y
+ * solve (chunked across lanes at 0 and 2), both at round-off level.  DFP_E_ARG for values out of
  * range, DFP_E_UNSUPPORTED for shapes that do not fit the device's LDS. */
 typedef struct dfp_tuning {
     int32_t z_split, x_columns, z_rows, z_fused;
