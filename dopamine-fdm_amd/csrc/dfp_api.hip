@@ -257,10 +257,11 @@ int choose_shape(const dfp_grid* g, int f32, size_t lds_limit, const dfp_tuning*
             if (q.G >= 1) split.push_back(q);
         }
     }
-    // periodic y, planes in registers: the smallest split from 4 on (the x
-    // kernels' spectrum segments shorten with R), else the largest below.
-    // 256x257x256: 682 us in LDS (R = 16), 558-567 in registers (R = 8);
-    // 64x65x64: 56 -> 43 us (R = 4), 128x129x96: 94 -> 76 (R = 4; 73 at 8).
+    // periodic y, planes in registers: the smallest split from 4 on, since the x
+    // kernels' spectrum segments shorten with R, else the largest below.  Within
+    // 4 % of the best split at the sizes measured: 256x257x256 558-567 us at
+    // R = 8, the first that fits (682 in LDS at R = 16); 64x65x64 43 at 4 (56 in
+    // LDS); 128x129x96 76 at 4, 73 at 8 (94 in LDS).
     if (!planes.empty()) {
         for (const Shape& q : planes)
             if (q.R >= 4) { out = q; return DFP_OK; }

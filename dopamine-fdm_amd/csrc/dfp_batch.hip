@@ -1,23 +1,26 @@
 // Batched projections: many plans (any sizes, either precision) projected
-// together with one persistent launch per stage.
+// together, each stage a few launches over all cases.
 //
 // Every stage kernel has a batched form (kb_*) whose workgroups walk the
 // concatenated work lists of all cases of the stage: the case records
 // (XPar/ZPar/CPar/MPar/SPar) and the per-case work offsets are written on the
 // host into one pinned staging buffer, copied to the device by one small
 // kernel, and read by the kernels.  The kernels' own arguments are
-// then only addresses inside that device buffer, the case counts live in it
-// too, and the grid is fixed (workgroups per CU x CUs, capped at what the
-// device holds at once of the kernel with its LDS), so a launch sequence
-// captured once in a hipGraph replays for any batch with the same stage list
+// then only addresses inside that device buffer, and the case counts live in
+// it too.  The x and stencil launches have one workgroup per tile; with graphs,
+// or after dfp_batch_set_occupancy, their grid is fixed as the z launches' is
+// (workgroups per CU x CUs, capped at what the device holds at once of the
+// kernel with its LDS), so a launch sequence captured once in a hipGraph
+// replays for any batch with the same stage list
 // and LDS sizes.  Each plan keeps its own spectrum scratch, so the cases of a
 // batch are independent; a plan may appear once per batch.
 //
 // Stage list of one call (FP64 cases a, FP32+refine cases b, the latter
 // ordered by descending sweep count so sweep s runs the first n_s of them);
 // each x stage is one launch per z-split radix present (the x kernels are
-// compiled per radix), each z stage one launch for the cases with the fused
-// z kernel and one pair for those with the split pair:
+// compiled per radix) and group of register line lengths, each z stage one
+// launch per z kernel (sub-planes in registers or streamed, by row length, or
+// held in LDS):
 //   x forward  (a: divergence, b: divergence + FP64 copy + row sums)
 //   (0,0) mode (b)
 //   z transforms and y solves (a, b)

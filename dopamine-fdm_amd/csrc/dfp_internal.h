@@ -509,12 +509,6 @@ __host__ __device__ __forceinline__ int lu_pos(int kz, int R, int nz2) {
     return lu_pos_mu(m, kz - m * R, R, nz2);
 }
 
-// MI355X dispatches workgroup w of a launch to XCD w % 8, and each XCD has its
-// own L2.  xcd_remap(w, n) renumbers the n workgroups so that each XCD gets a
-// contiguous range of logical indices: neighbouring tiles (which read the
-// same halo rows, pivot rows or cache lines) then share an L2.  A bijection
-// on [0, n) for every n; only locality, never correctness, depends on the
-// dispatch order.
 // case of work item w: the last c with off[c] <= w (off[0] = 0, off[nc] =
 // total, w < total).  Every lane of the wave must call it: 64 offsets are
 // read at once, where a bisection waits for log2(nc) loads in turn.
@@ -525,6 +519,12 @@ __device__ __forceinline__ int find_case(const int* __restrict__ off, int nc, in
     return __builtin_amdgcn_readfirstlane(c);
 }
 
+// MI355X dispatches workgroup w of a launch to XCD w % 8, and each XCD has its
+// own L2.  xcd_remap(w, n) renumbers the n workgroups so that each XCD gets a
+// contiguous range of logical indices: neighbouring tiles (which read the
+// same halo rows, pivot rows or cache lines) then share an L2.  A bijection
+// on [0, n) for every n; only locality, never correctness, depends on the
+// dispatch order.
 constexpr int kXcds = 8;
 __device__ __forceinline__ int xcd_remap(int w, int n) {
     const int q = n / kXcds, r = n - q * kXcds;

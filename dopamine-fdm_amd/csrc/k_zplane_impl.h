@@ -197,7 +197,9 @@ __device__ __forceinline__ ZRec<C> zrec_uniform(const ZPar<C>& z) {
 // one.  An item's rows load into the registers that the item before frees,
 // behind that item's inverse transform and stores.  NCHY: the chunks of a
 // periodic y (rows interleaved over them, periodic_ysolve, zy its tables; row
-// nym-1 receives row 0's values), or 0 for the wall solve.
+// nym-1, the duplicate of row 0, is neither read nor written: it keeps what the
+// forward x kernel left there, and the inverse one takes row 0 in its place),
+// or 0 for the wall solve.
 template <typename C, int N1, int N2, int BR, int NB, int NCHY, typename Rec, typename Same>
 __device__ __forceinline__ void zplane_run(int w0, int total, Rec rec, Same same, const ZyPar<C>* zy,
                                            unsigned char* smem_raw) {

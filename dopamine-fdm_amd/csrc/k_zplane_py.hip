@@ -3,7 +3,7 @@
 // and passes through LDS for the exchanges of the z rows and twice for the y
 // columns (half width), where the LDS-resident kernel (k_zfused.hip) takes
 // every stage of every transform through LDS.  256x257x256: 171 us there (16
-// modes a row), 103-106 here (32 modes a row, which shortens the x kernels).
+// modes a row), 96 here (32 modes a row, which shortens the x kernels).
 // Bound by one workgroup a CU (two waves a SIMD) running its phases in turn.
 #include <algorithm>
 

@@ -1,7 +1,7 @@
 """Batched projections over libdfp's batch executor (``dfp_batch_*``).
 
 A ``Batch`` runs the projections of many plans - uneven grid sizes, FP64 and
-FP32+refine mixed - with one persistent launch per stage (no counterpart in
+FP32+refine mixed - with a few launches per stage (no counterpart in
 the reference, which projects one grid per run).  Fields must be resident on
 the device (``DeviceArray`` or CUDA tensors in the reference's Fortran
 layout); results equal ``Plan.project`` on each case bit for bit.
@@ -49,7 +49,8 @@ class Batch:
             raise DfpError(rc, where, detail)
 
     def set_occupancy(self, x_per_cu: int, z_per_cu: int, stencil_per_cu: int):
-        """Workgroups per CU of the persistent x, z and stencil launches."""
+        """Workgroups per CU of the x, z and stencil launches, which are persistent from
+        then on (else, outside graphs, the x and stencil launches run one workgroup per tile)."""
         self._check(lib().dfp_batch_set_occupancy(self._h, int(x_per_cu), int(z_per_cu), int(stencil_per_cu)),
                     "dfp_batch_set_occupancy")
 
@@ -65,7 +66,7 @@ class Batch:
         self._check(lib().dfp_batch_set_stream(self._h, stream_handle), "dfp_batch_set_stream")
 
     def project(self, cases: list[Case], asynchronous: bool = False, solve_only: bool = False):
-        """Project every case (one persistent launch per stage).  With
+        """Project every case (a few launches per stage).  With
         solve_only, each case's rhs holds the right-hand side and receives phi
         (and P with save_p), as Plan.solve; U, V, W are not read (may be None)."""
         n = len(cases)

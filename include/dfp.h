@@ -263,7 +263,9 @@ typedef struct dfp_batch dfp_batch;
 int dfp_batch_create(int device, int max_cases, dfp_batch **out);
 int dfp_batch_destroy(dfp_batch *batch);
 int dfp_batch_set_stream(dfp_batch *batch, void *hip_stream);
-/* workgroups per CU of the persistent x, z and stencil launches (autotuned) */
+/* workgroups per CU of the x, z and stencil launches (autotuned).  Without this
+ * call the x and stencil launches run one workgroup per tile outside graphs;
+ * once made, they are persistent in every later call of the batch */
 int dfp_batch_set_occupancy(dfp_batch *batch, int x_per_cu, int z_per_cu, int stencil_per_cu);
 /* replay the launch sequence from hipGraphs keyed by its stage list: a list's
  * first call runs it, the second captures it, later ones replay it */
