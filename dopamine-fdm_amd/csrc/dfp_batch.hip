@@ -221,12 +221,14 @@ __global__ void __launch_bounds__(256) k_stage_tables(const uint4* __restrict__ 
     for (uint32_t e = blockIdx.x * 256 + threadIdx.x; e < len; e += gridDim.x * 256) dst[at + e] = src[at + e];
 }
 
-// LDS of a batched launch rounded up to a power of two of at least 4 KiB
-// (few distinct graphs), unless that would leave no room for the kernels'
-// static LDS under the device limit
-size_t lds_bucket(size_t v, size_t limit) {
-    size_t a = 4096;
-    while (a < v) a *= 2;
+// LDS of a batched launch: rounded up to a power of two of at least 4 KiB with
+// graphs (few distinct ones), else to 1 KiB (few distinct occupancy queries),
+// unless that would leave no room for the kernels' static LDS under the device
+// limit
+size_t lds_bucket(size_t v, size_t limit, bool graphs) {
+    size_t a = align_up(v, 1024);
+    if (graphs)
+        for (a = 4096; a < v;) a *= 2;
     return a + 512 <= limit ? a : v;
 }
 
@@ -479,8 +481,7 @@ int dfp_batch_project(dfp_batch* b, int n, dfp_plan* const* plans, double* const
     int phase = 0;
     auto add = [&](Launch::Kind k, int f32, int mode, int R, size_t tab, int list, size_t lds) {
         const int items = pool[(size_t)list * list_stride + counts[list]];
-        ls.push_back(Launch{k, f32, mode, R, tab, list, items, b->use_graphs ? lds_bucket(lds, lds_limit) : align_up(lds, 1024),
-                            phase});
+        ls.push_back(Launch{k, f32, mode, R, tab, list, items, lds_bucket(lds, lds_limit, b->use_graphs), phase});
     };
     // the x launches of a set of records, one per radix present; the z launches
     // for its fused and split members
