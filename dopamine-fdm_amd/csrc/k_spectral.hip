@@ -54,17 +54,19 @@ void xpar_columns(XPar<C>& q, const dfp_plan* p, XKind k) {
 template void xpar_columns<double2>(XPar<double2>&, const dfp_plan*, XKind);
 template void xpar_columns<float2>(XPar<float2>&, const dfp_plan*, XKind);
 
-// A single launch on a small grid: narrower tiles while the launch has fewer
-// than two workgroups per CU, down to four columns (64-byte FP64 spectrum
-// segments).  64x64x64 (16 columns in 64 workgroups -> 4 in
-// 256): forward 10.2 -> 7.6 us, inverse 10.6 -> 7.5.  The FP32
+// A single launch on a small grid: narrower tiles, down to four columns
+// (64-byte FP64 spectrum segments), as long as the launch stays within one
+// workgroup per CU.  64x64x64 (16 columns in 64 workgroups -> 4 in 256):
+// forward 10.2 -> 7.6 us, inverse 10.6 -> 7.5.  Beyond that the short tiles
+// cost more than the CUs they fill give: 32x200x64 with 16 columns in 200
+// workgroups 9.7 us forward, with 4 in 800 13.4.  The FP32
 // form keeps its tiles, whose sums per workgroup set the order of its row
 // sums, and batched launches theirs, since the other cases fill the GPU.
 static void narrow_columns(XPar<double2>& q) {
     const int nz2 = q.g.nzp / q.R;
     int T = q.T;
-    for (int t = T - 1; t >= 4 && (long)(nz2 / T) * q.g.nym < 512; --t)
-        if (nz2 % t == 0) T = t;
+    for (int t = T - 1; t >= 4; --t)
+        if (nz2 % t == 0 && (long)(nz2 / t) * q.g.nym <= 256) T = t;
     q.T = T;
     q.nbx = nz2 / T;
     q.strip = q.g.nxp >= 512 ? std::min(q.nbx, 8) : q.nbx;  // as xpar_columns
