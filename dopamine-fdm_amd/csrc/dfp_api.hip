@@ -517,9 +517,11 @@ int dfp_plan_tuning(const dfp_plan* p, dfp_tuning* t) {
     t->z_split = p->zr;
     // each x kernel's own choice, and narrower tiles on small grids, are what 0 chooses
     t->x_columns = p->tuned_columns ? p->tk_x : 0;
-    // the register-plane kernel is what 0, 0 choose
-    t->z_rows = p->zp_nb ? 0 : p->g_zs;
-    t->z_fused = p->zp_nb ? 0 : (p->zfused ? 2 : 1);
+    // rows per group are the streaming kernel's; the register-plane kernel and
+    // the z walls' kernels are what 0, 0 choose
+    const bool chosen = p->zp_nb || p->geo.zbc == 1;
+    t->z_rows = chosen || p->zfused ? 0 : p->g_zs;
+    t->z_fused = chosen ? 0 : (p->zfused ? 2 : 1);
     return DFP_OK;
 }
 

@@ -102,7 +102,8 @@ int dfp_plan_destroy(dfp_plan *plan);
  *              sets both x kernels (one that holds its lines in registers
  *              takes the most of them that fit), else each picks its own
  *              (dfp_plan_tuning then reports 0)
- *   z_rows     y rows per group of the split z kernels (z_fused = 1)
+ *   z_rows     y rows per group of the split z kernels (z_fused = 1;
+ *              dfp_plan_tuning reports 0 for the others)
  *   z_fused    1: split pair of z kernels (FFT + elimination, back
  *              substitution + inverse FFT, spectrum read and written twice);
  *              2: one fused kernel holding a whole (kx, z-split) sub-plane

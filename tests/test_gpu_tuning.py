@@ -37,6 +37,35 @@ def test_reported_shapes_make_the_same_plan(size, precision):
     again.close()
 
 
+@pytest.mark.parametrize("grid", [dfp.periodic_y_grid(32, 33, 32), dfp.periodic_y_grid(32, 25, 18),
+                                  dfp.duct_grid(32, 12, 20, 1.2, 0.8), dfp.zwall_periodic_y_grid(32, 13, 20, 0.8),
+                                  dfp.channel_grid(32, 12, 24, 1.2, x_bc_type=1)],
+                         ids=["planes", "lds", "duct", "zwall", "inflow"])
+def test_reported_shapes_of_every_branch_make_the_same_plan(grid):
+    print(f"{grid.nxp}x{grid.nym}x{grid.nzp}", flush=True)
+    host = fields(grid, 3, 0.1)
+    plan = dfp.Plan(grid)
+    again = dfp.Plan(grid, tuning=plan.tuning)
+    assert again.tuning == plan.tuning
+    for a, b in zip(_project(plan, host), _project(again, host)):
+        assert np.array_equal(a, b)
+    plan.close()
+    again.close()
+
+
+@pytest.mark.parametrize("precision", [dfp.DFP_FP64, dfp.DFP_FP32_REFINE], ids=["fp64", "fp32"])
+def test_reported_lds_shape_makes_the_same_plan(precision):
+    g = make_grid(32, 20, 64, 1.5)
+    plan = dfp.Plan(g, precision=precision, tuning=(4, 0, 0, 2))
+    again = dfp.Plan(g, precision=precision, tuning=plan.tuning)
+    assert again.tuning == plan.tuning and plan.tuning[3] == 2
+    host = fields(g, 3, 0.1)
+    for a, b in zip(_project(plan, host), _project(again, host)):
+        assert np.array_equal(a, b)
+    plan.close()
+    again.close()
+
+
 def test_chosen_columns_are_reported():
     g = make_grid(64, 40, 64, 1.5)
     for T in (1, 4, 16):
