@@ -263,10 +263,17 @@ int choose_shape(const dfp_grid* g, int f32, size_t lds_limit, const dfp_tuning*
     // R = 8, the first that fits (682 in LDS at R = 16); 64x65x64 43 at 4 (56 in
     // LDS); 128x129x96 76 at 4, 73 at 8 (94 in LDS).
     if (!planes.empty()) {
+        const Shape* best = &planes.back();
         for (const Shape& q : planes)
-            if (q.R >= 4) { out = q; return DFP_OK; }
-        out = planes.back();
-        return DFP_OK;
+            if (q.R >= 4) { best = &q; break; }
+        // Tall planes of short rows take longer than the LDS kernel's of a
+        // larger split, so with few of them (fewer than CUs by far) that one
+        // is left: 16x257x8 24.8 us a solve in registers (9 planes), 20.7 in
+        // LDS; 8x129x12 21.2 and 20.1 (5 planes).  From 10 planes of 128 rows
+        // and 40 of 256, and with 32 modes a row or more, registers win.
+        const int rows = g->nym - 1, few = rows >= 256 ? 40 : rows >= 128 ? 10 : 0;
+        const bool lds = want_R == 0 && !fused.empty() && best->fz.n < 32 && (g->nxp / 2 + 1) * best->R < few;
+        if (!lds) { out = *best; return DFP_OK; }
     }
     // default: the split pair with the classic split (R = 4 when it leaves at
     // least 8 points per row, else 2, else 3, else none); the fused form when
