@@ -602,8 +602,13 @@ int dfp_plan_create_tuned(const dfp_grid* g, int precision, int device, const df
     p->zp_nb = sh.py_nb;
     p->zp_nch = sh.py_nch;
     if (!sh.fused) z_two_pass(sh.fz.n, p->zn1, p->zn2);
-    // whole sub-planes in registers where they fit, unless the streaming kernel was asked for
-    if (!sh.fused && g->z_bc_type == 0 && !(tune && (tune->z_rows || tune->z_fused)) &&
+    // whole sub-planes in registers where they fit, unless the streaming kernel
+    // was asked for.  A register pass takes eight rows, so a few planes of very
+    // few short rows are left to the streaming kernel (16x5x32 7.6 us, 8.6 in
+    // registers; 16x16x32 8.9 and 8.8; 16x5x128 9.2 and 7.9; 256x5x32 9.1 and 8.7).
+    const bool few = !(tune && tune->z_split) && sh.fz.n < 32 && sh.fz.n * g->nym < 100 &&
+                     (long)sh.fz.n * sh.R * (g->x_bc_type == 1 ? g->nxp : g->nxp / 2 + 1) < 2200;
+    if (!sh.fused && !few && g->z_bc_type == 0 && !(tune && (tune->z_rows || tune->z_fused)) &&
         !zplane_shape(sh.fz.n, g->nym, precision == DFP_FP32_REFINE, p->lds_limit, p->zp_nb, p->zp_nch, p->zp_n1,
                       p->zp_n2, p->zp_br))
         p->zp_nb = 0;

@@ -110,7 +110,8 @@ int dfp_plan_destroy(dfp_plan *plan);
  *              of nym x nzp/R modes in LDS (read and written once);
  *              0 with z_rows = 0: a sub-plane held in registers where it
  *              fits (read and written once; dfp_plan_tuning then reports
- *              z_rows = z_fused = 0), else 1
+ *              z_rows = z_fused = 0; with z_split = 0 the library leaves small
+ *              sets of sub-planes to the other kernels), else 1
  * FP64 results do not depend on x_columns (the FP32 form's row sums take the
  * order of the columns, at round-off level) or, at z_fused = 1, on z_rows;
  * z_split changes the FFT's factorisation and z_fused the association of the y

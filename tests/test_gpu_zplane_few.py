@@ -1,6 +1,7 @@
-"""The library's choice of the z kernel for a periodic y where there are few
-sub-planes: tall planes of short rows keep the LDS-resident kernel below 10
-planes of 128 rows and 40 of 256, registers take the rest; a z split asked for
+"""The library's choice of the z kernel where there are few sub-planes.
+Periodic y: tall planes of short rows keep the LDS-resident kernel below 10
+planes of 128 rows and 40 of 256.  Walls: a few planes of very few short rows
+keep the streaming kernel.  Registers take the rest, and a z split asked for
 takes registers wherever they fit.  Each side of the line against the C
 oracle, and the shape reported makes the same plan."""
 from __future__ import annotations
@@ -9,7 +10,7 @@ import numpy as np
 import pytest
 
 import dfp
-from _cases import fields, oracle_project, rel_linf
+from _cases import fields, make_grid, oracle_project, rel_linf
 
 pytestmark = pytest.mark.gpu
 
@@ -40,3 +41,21 @@ def test_few_planes_of_a_periodic_y(nxp, nyp, nzp, planes):
         assert rel_linf(a, b) <= 1e-12, lab
     again, e = _project(g, shape, host)
     assert again == shape and all(np.array_equal(a, b) for a, b in zip(d, e))
+
+
+@pytest.mark.parametrize("nxp,nym,nzp,planes", [(16, 12, 32, False), (16, 13, 32, True), (32, 6, 64, False),
+                                                (32, 7, 64, True), (64, 6, 64, False), (72, 6, 64, True),
+                                                (16, 1, 128, True), (48, 1, 16, False)])
+def test_few_planes_of_few_rows_between_walls(nxp, nym, nzp, planes):
+    print(f"channel {nxp}x{nym}x{nzp}", flush=True)
+    g = make_grid(nxp, nym, nzp, 1.5)
+    host = fields(g, nym + nzp, 0.1)
+    o = [a.copy(order="F") for a in host]
+    oracle_project(g, *o, DT, C3, save_p=True)
+    shape, d = _project(g, None, host)
+    assert shape[3] == (0 if planes else 1)
+    for lab, a, b in zip(("U", "V", "W", "P", "phi"), d, o):
+        assert rel_linf(a, b) <= 1e-12, lab
+    again, e = _project(g, shape, host)
+    assert again == shape and all(np.array_equal(a, b) for a, b in zip(d, e))
+    assert _project(g, (shape[0], 0, 0, 0), host)[0][3] == 0
