@@ -36,7 +36,6 @@
 #include <cstring>
 #include <map>
 #include <new>
-#include <set>
 #include <tuple>
 
 #include <mutex>
@@ -141,7 +140,6 @@ struct dfp_batch {
     bool copy_pending = false;
     bool use_graphs = false;
     std::map<std::vector<long>, hipGraphExec_t> graphs;
-    std::set<std::vector<long>> seen;  // keys run once, not captured yet (at most kMaxSeen)
     // launches of one phase (independent case lists) run side by side on the
     // caller's stream and these, forked and joined with events
     std::vector<hipStream_t> aux;
@@ -157,7 +155,6 @@ struct dfp_batch {
 // channels, FP64 / FP32+refine: none 895 / 1268 us, one 836 / 1165, two
 // 859 / 1158, three 872 / 1217; the largest launches first instead of in turn: 868 / 1229).
 constexpr int kMaxParallel = 3;
-constexpr size_t kMaxSeen = 4096;
 constexpr int kAuxStreams = 1;
 
 namespace {
@@ -676,9 +673,11 @@ int dfp_batch_project(dfp_batch* b, int n, dfp_plan* const* plans, double* const
         return hipSuccess;
     };
 
-    // key: the launch list as the kernels see it (kind, precision, mode, radix, records, list, LDS)
-    std::vector<long> key;
-    if (b->use_graphs)
+    if (!b->use_graphs) {
+        BCHK(b, run_all(b->stream));
+    } else {
+        // key: the launch list as the kernels see it (kind, precision, mode, radix, records, list, LDS)
+        std::vector<long> key;
         for (const Launch& l : ls) {
             key.push_back(l.kind);
             key.push_back(l.f32 * 256 + l.mode);
@@ -688,18 +687,6 @@ int dfp_batch_project(dfp_batch* b, int n, dfp_plan* const* plans, double* const
             key.push_back((long)l.lds);
             key.push_back(l.phase);
         }
-    // A key is captured when it comes a second time: with many sizes most sets
-    // come once, and a capture costs more than the replays of a few calls give
-    // back (random sets of 4 to 16 of 48 sizes, FP64, us a call: new sets 501
-    // captured, 204 run; known ones 179 replayed).
-    const bool replay = b->use_graphs && (b->graphs.count(key) || b->seen.count(key));
-    if (!replay) {
-        BCHK(b, run_all(b->stream));
-        if (b->use_graphs) {
-            if (b->seen.size() >= kMaxSeen) b->seen.clear();
-            b->seen.insert(key);
-        }
-    } else {
         auto it = b->graphs.find(key);
         if (it == b->graphs.end()) {
             hipStream_t cap_stream;
@@ -719,7 +706,6 @@ int dfp_batch_project(dfp_batch* b, int n, dfp_plan* const* plans, double* const
             (void)hipStreamDestroy(cap_stream);
             if (e != hipSuccess) return bfail(b, DFP_E_HIP, "graph capture: %s", hipGetErrorString(e));
             it = b->graphs.emplace(key, exec).first;
-            b->seen.erase(key);
         }
         BCHK(b, hipGraphLaunch(it->second, b->stream));
     }

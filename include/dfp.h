@@ -269,8 +269,7 @@ int dfp_batch_set_stream(dfp_batch *batch, void *hip_stream);
  * call the x and stencil launches run one workgroup per tile outside graphs;
  * once made, they are persistent in every later call of the batch */
 int dfp_batch_set_occupancy(dfp_batch *batch, int x_per_cu, int z_per_cu, int stencil_per_cu);
-/* replay the launch sequence from hipGraphs keyed by its stage list: a list's
- * first call runs it, the second captures it, later ones replay it */
+/* replay the launch sequence from hipGraphs keyed by its stage list */
 int dfp_batch_use_graphs(dfp_batch *batch, int enable);
 /* independent launches of one stage (different z splits or z kernels) run
  * side by side on up to 1 + aux_streams streams (0..3, default 3; the library

@@ -68,16 +68,16 @@ def test_diverse_batch_equals_single_plans(n, precision, sweeps, solve_only, gra
     print(f"{n} cases, precision {precision}, {sweeps} sweeps, solve only {solve_only}, graphs {graphs}", flush=True)
     cases, start, want = _cases(n, precision, sweeps, solve_only)
     batch = Batch(max_cases=n, graphs=graphs)
-    for _ in range(4 if graphs else 1):  # with graphs: run, captured, replayed twice
+    for _ in range(3 if graphs else 1):  # with graphs: captured, then replayed
         _run(batch, range(n), cases, start, want, solve_only)
     batch.close()
     for c in cases:
         c.plan.close()
 
 
-def test_graph_of_a_batch_is_captured_when_its_stage_list_comes_again():
-    """Sets of sizes in turn, each run directly, then captured, then replayed, another set between: every call equals
-    the single plans' bits."""
+def test_graphs_of_alternating_sets_of_sizes():
+    """Sets of sizes in turn, each captured, then replayed, another set between: every call equals the single plans'
+    bits."""
     print("graphs over alternating sets of sizes", flush=True)
     cases, start, want = _cases(12)
     batch = Batch(max_cases=12, graphs=True)
