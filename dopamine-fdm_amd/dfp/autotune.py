@@ -3,7 +3,8 @@ the batched launches, cached in a JSON table.
 
 For one grid it times, with HIP events on resident fields, every valid
 (z_split, x_columns, z_rows, z_fused) of ``dfp_plan_create_tuned`` in a
-bounded candidate set and keeps the fastest; for a batch it times the persistent
+bounded candidate set, the library's own shape among them, and keeps the
+fastest; for a batch it times the persistent
 launches at a few workgroups-per-CU settings under each shape family.  The table maps
 "nxp x nym x nzp:fp64|fp32" to the chosen shape and its time:
 
@@ -111,6 +112,9 @@ def time_plan(plan: Plan, fields, reps: int = 10, warmup: int = 3) -> float:
     return 1e3 * e0.elapsed_ms(e1) / reps
 
 
+KEEP = 0.98  # a shape replaces the library's own where it takes less than this share of its time
+
+
 def tune_plan(g: ChannelGrid, precision: int = DFP_FP64, reps: int = 10, device: int = 0, seed: int = 7,
               sigma: float = 0.1, log=None) -> dict:
     """Time the candidate shapes of one grid; returns {"tuning", "us", "default_us", "tried"}."""
@@ -126,11 +130,14 @@ def tune_plan(g: ChannelGrid, precision: int = DFP_FP64, reps: int = 10, device:
         return (*fields, rhs)
 
     default_us = time_plan(base, fresh(), reps)
-    best = (default_us, base.tuning)
-    base.close()
+    own_shape = base.tuning
+    best = (default_us, own_shape)
     tried = 0
     seen = set()
-    for R, T, G, F in candidates(g):
+    # the sub-planes in registers (where they fit; else these are the split pair again) and each split's own columns
+    cands = candidates(g)
+    own = [(R, T, 0, 0) for R in sorted({c[0] for c in cands}) for T in [0] + sorted({c[1] for c in cands if c[0] == R})]
+    for R, T, G, F in own + cands:
         try:
             if G == -1:
                 probe = Plan(g, device=device, precision=precision, tuning=(R, T, 0, F))
@@ -154,6 +161,14 @@ def tune_plan(g: ChannelGrid, precision: int = DFP_FP64, reps: int = 10, device:
         if us < best[0]:
             best = (us, shape)
         p.close()
+    if best[1] != own_shape:
+        # the fastest of so many by more than runs of one shape differ: both again, in turn
+        p = Plan(g, device=device, precision=precision, tuning=best[1])
+        turns = [(time_plan(base, fresh(), reps), time_plan(p, fresh(), reps)) for _ in range(4)]
+        p.close()
+        default_us, us = (min(t) for t in zip(*turns))
+        best = (us, best[1]) if us < KEEP * default_us else (default_us, own_shape)
+    base.close()
     return {"tuning": list(best[1]), "us": round(best[0], 2), "default_us": round(default_us, 2), "tried": tried}
 
 
